@@ -133,11 +133,12 @@ template <int COLL, int S>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void adjoint_fast(AdjointBuffers b,
                                                                                            StepParams p) {
     const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
-    if ((b.static_flags[tile] | b.dyn_prev[tile] | b.dyn_cur[tile]) != 0) return;
+    if ((b.dyn_prev[tile] | b.dyn_cur[tile]) != 0) return;
     int x0, y0, z;
     tile_origin(p.g, tile, x0, y0, z);
     const int x = x0 + (int)(threadIdx.x & (TILE_X - 1));
     const int y = y0 + (int)(threadIdx.x / TILE_X);
+    if (x >= p.g.nx || y >= p.g.ny) return;   // lanes of a partial tile beyond the grid
     const uint32_t row = (uint32_t)y + (uint32_t)p.g.ny * (uint32_t)z;
     const Sources s = sources(p, x, y, z);
     // the sponge blend f_out = post + (f_far - post) s scales the adjoint by 1 - s

@@ -97,7 +97,6 @@ struct bf_context {
     uint8_t* mask[3] = {nullptr, nullptr, nullptr};
     float4* wall[2] = {nullptr, nullptr};
     uint8_t* dyn[3] = {nullptr, nullptr, nullptr};
-    uint8_t* static_flags = nullptr;
     uint8_t* tflags[4] = {nullptr, nullptr, nullptr, nullptr};   // tiles keyed at step s -> tflags[s % 4]
     uint8_t* no_tiles = nullptr;          // all-zero tile flags
     uint32_t* general_list[2] = {nullptr, nullptr};
@@ -362,22 +361,6 @@ StepParams make_step_params(const bf_context* c) {
     p.force_scale = c->cfg.force_to_physical;
     for (int q = 0; q < 19; ++q) p.far_eq[q] = equilibrium<float>(q, p.far_rho, p.far_u[0], p.far_u[1], p.far_u[2]);
     return p;
-}
-
-// Tiles that always take the general path: partial tiles at the +x / +y
-// edges (the fast kernel streams whole tiles; the sponge band streams there
-// too).
-std::vector<uint8_t> static_tile_flags(const bf_config& cfg, const Grid& g) {
-    (void)cfg;
-    std::vector<uint8_t> flags(g.tiles, 0);
-    for (int z = 0; z < g.nz; ++z)
-        for (int ty = 0; ty < g.tiles_y; ++ty)
-            for (int tx = 0; tx < g.tiles_x; ++tx) {
-                const int x0 = tx * TILE_X, y0 = ty * TILE_Y;
-                const bool general = x0 + TILE_X > g.nx || y0 + TILE_Y > g.ny;
-                flags[((size_t)z * g.tiles_y + ty) * g.tiles_x + tx] = general ? 1 : 0;
-            }
-    return flags;
 }
 
 // Geometry views of step s.
@@ -749,7 +732,7 @@ bf_status enqueue_tile_list(bf_context* c, int64_t s) {
     const StepGeometry sg = geometry_of(c, s);
     hipError_t e = launch_fill_u32(&c->counters[par2(s)], 0u, 1u, c->sb);
     if (e == hipSuccess)
-        e = launch_build_general_list(c->static_flags, sg.dyn_prev, sg.dyn_cur, c->g.tiles, c->general_list[par2(s)],
+        e = launch_build_general_list(sg.dyn_prev, sg.dyn_cur, c->g.tiles, c->general_list[par2(s)],
                                       &c->counters[par2(s)], c->sb);
     if (e != hipSuccess) return hip_fail(c, e, "tile list launch");
     return BF_OK;
@@ -765,7 +748,6 @@ FluidBuffers fluid_buffers(const bf_context* c, int64_t s) {
     b.wall = sg.wall;
     b.dyn_cur = sg.dyn_cur;
     b.dyn_prev = sg.dyn_prev;
-    b.static_flags = c->static_flags;
     b.general_list = c->general_list[par2(s)];
     b.general_count = &c->counters[par2(s)];
     b.partials = c->partials + 8ull * c->g.tiles * (uint64_t)par2(s);
@@ -988,7 +970,6 @@ bf_status bf_create(const bf_config* cfg, bf_context** out) {
     for (int i = 0; i < 3; ++i) c->mask[i] = (uint8_t*)A.take(e, n);
     for (int i = 0; i < 2; ++i) c->wall[i] = (float4*)A.take(e, 16 * n);
     for (int i = 0; i < 3; ++i) c->dyn[i] = (uint8_t*)A.take(e, g.tiles);
-    c->static_flags = (uint8_t*)A.take(e, g.tiles);
     for (int i = 0; i < 4; ++i) c->tflags[i] = (uint8_t*)A.take(e, g.tiles);
     c->no_tiles = (uint8_t*)A.take(e, g.tiles);
     for (int i = 0; i < 2; ++i) c->general_list[i] = (uint32_t*)A.take(e, 4ull * g.tiles);
@@ -1014,9 +995,7 @@ bf_status bf_create(const bf_config* cfg, bf_context** out) {
         bf_destroy(c);
         return BF_ERROR_ALLOCATION_FAILED;
     }
-    std::vector<uint8_t> sf = static_tile_flags(*cfg, g);
     hipStream_t s = c->sb;
-    e = hipMemcpyAsync(c->static_flags, sf.data(), sf.size(), hipMemcpyHostToDevice, s);
     for (int i = 0; i < 3 && e == hipSuccess; ++i) e = launch_fill_u8(c->mask[i], 0, g.n, s);
     for (int i = 0; i < 2 && e == hipSuccess; ++i) e = launch_fill_wall(c->wall[i], g.n, s);
     for (int i = 0; i < 3 && e == hipSuccess; ++i) e = launch_fill_u8(c->dyn[i], 0, g.tiles, s);
@@ -2517,7 +2496,7 @@ bf_status segment_geometry(bf_context* c, int64_t s0, uint32_t steps, uint32_t i
     for (int64_t s = sa_ + 1; s <= sb_ && e == hipSuccess; ++s) {
         const uint32_t k = (uint32_t)(s - sa_);
         const SlotGeometry gp = slot_geometry(c, k - 1, set), gc = slot_geometry(c, k, set);
-        e = launch_build_general_list(c->static_flags, gp.dyn, gc.dyn, c->g.tiles,
+        e = launch_build_general_list(gp.dyn, gc.dyn, c->g.tiles,
                                       a.slot_list[set] + (uint64_t)k * c->g.tiles, a.slot_count[set] + k, c->sa);
     }
     if (e == hipSuccess) e = hipEventRecord(a.ev_geo[set], c->sa);
@@ -2652,7 +2631,6 @@ bf_status bf_adjoint_gradient(bf_context* c, uint32_t steps, const double* load_
             fb.solid_prev = gp.mask;
             fb.solid_cur = gc.mask;
             fb.wall = gc.wall;
-            fb.static_flags = c->static_flags;
             fb.dyn_prev = gp.dyn;
             fb.dyn_cur = gc.dyn;
             fb.general_list = a.slot_list[set] + (uint64_t)(s - sa_) * c->g.tiles;
@@ -2713,7 +2691,6 @@ bf_status bf_adjoint_gradient(bf_context* c, uint32_t steps, const double* load_
             ab.solid_prev = gp.mask;
             ab.solid_cur = gc.mask;
             ab.wall = gc.wall;
-            ab.static_flags = c->static_flags;
             ab.dyn_prev = gp.dyn;
             ab.dyn_cur = gc.dyn;
             ab.general_list = a.slot_list[set] + (uint64_t)k * c->g.tiles;

@@ -551,7 +551,6 @@ __device__ __forceinline__ void capture(float* __restrict__ density, float4* __r
 template <int ARITH, int COLL, int S>
 __global__ __launch_bounds__(256) void fluid_fast(const typename Store<S>::T* __restrict__ fin,
                                                   typename Store<S>::T* __restrict__ fout,
-                                                  const uint8_t* __restrict__ static_flags,
                                                   const uint8_t* __restrict__ dyn_prev,
                                                   const uint8_t* __restrict__ dyn_cur,
                                                   float* __restrict__ density, float4* __restrict__ velocity,
@@ -562,15 +561,19 @@ __global__ __launch_bounds__(256) void fluid_fast(const typename Store<S>::T* __
     // loaded together with the populations and tested only before the
     // stores: a test up front would put a dependent memory round trip ahead
     // of every workgroup's population loads.
-    const bool general_tile = (static_flags[tile] | dyn_prev[tile] | dyn_cur[tile]) != 0;
+    const bool general_tile = (dyn_prev[tile] | dyn_cur[tile]) != 0;
     int x0, y0, z;
     tile_origin(p.g, tile, x0, y0, z);
     const int nx = p.g.nx, ny = p.g.ny, nz = p.g.nz;
-    // Lanes of a partial tile beyond the grid load from the last column / row
-    // (their tile is a general tile: nothing they load is used), so no load
-    // leaves the lattice; in whole tiles the clamp changes nothing.
-    const int x = min(x0 + (int)(threadIdx.x & (TILE_X - 1)), nx - 1);
-    const int y = min(y0 + (int)(threadIdx.x / TILE_X), ny - 1);
+    // Lanes of a partial tile beyond the grid load from the last column / row,
+    // so no load leaves the lattice, and store nothing; in whole tiles the
+    // clamp changes nothing.  Partial tiles used to take the general path:
+    // a grid of odd sides then spent most of its step there (203x117x91 BF16,
+    // 3,407 of 10,920 tiles: 99 of 163 us per step).
+    const int xl = x0 + (int)(threadIdx.x & (TILE_X - 1)), yl = y0 + (int)(threadIdx.x / TILE_X);
+    const bool in_grid = xl < nx && yl < ny;
+    const int x = min(xl, nx - 1);
+    const int y = min(yl, ny - 1);
 
     bool xm_far = false, xp_far = false, ym_far = false, yp_far = false, zm_far = false, zp_far = false;
     // source coordinates for c = +1 (s = v - 1) and c = -1 (s = v + 1)
@@ -625,21 +628,23 @@ __global__ __launch_bounds__(256) void fluid_fast(const typename Store<S>::T* __
     // toward the far-field equilibrium after the collision); a uniform branch,
     // so that without a sponge the store path carries no blend
     float crho, cmx, cmy, cmz;
-    if (p.sponge_strength > 0.0f)
-        write_post<S>(fout, x, row_self, post, sponge_factor(p, x, y, z), p, crho, cmx, cmy, cmz);
-    else
-        write_post<S>(fout, x, row_self, post, 0.0f, p, crho, cmx, cmy, cmz);
-    guard_finite(p, crho);
-    if (p.capture_fields) capture(density, velocity, gid, crho, cmx, cmy, cmz);
+    if (in_grid) {
+        if (p.sponge_strength > 0.0f)
+            write_post<S>(fout, x, row_self, post, sponge_factor(p, x, y, z), p, crho, cmx, cmy, cmz);
+        else
+            write_post<S>(fout, x, row_self, post, 0.0f, p, crho, cmx, cmy, cmz);
+        guard_finite(p, crho);
+        if (p.capture_fields) capture(density, velocity, gid, crho, cmx, cmy, cmz);
+    }
     if constexpr (COLL != COLL_TRT) {
         // Limiter activations of fast cells: an exact count and the maximum
         // restriction (order-independent integer and max atomics; restr >= 0
-        // orders like its bit pattern).  Fast tiles are whole, so every lane
-        // of the wavefront is active here.
+        // orders like its bit pattern).  Every lane of the wavefront takes
+        // part in the shuffles; those beyond the grid count nothing.
         if (p.accumulate_loads) {
-            const unsigned long long hit = __ballot(act != 0.0f);
+            const unsigned long long hit = __ballot(in_grid && act != 0.0f);
             if (hit != 0) {
-                float r = restr;
+                float r = in_grid ? restr : 0.0f;
 #pragma unroll
                 for (int off = 32; off > 0; off >>= 1) r = fmaxf(r, __shfl_xor(r, off, 64));
                 if ((threadIdx.x & 63) == 0) {
@@ -667,8 +672,8 @@ __global__ __launch_bounds__(256) void fluid_fast(const typename Store<S>::T* __
 // is exactly fluid_fast's, so a cell gets bit-identical results from either
 // kernel.  Needs nx a multiple of 128 (whole tile pairs, rows starting at
 // even elements; the launcher keeps fluid_fast otherwise); lanes of a tile
-// on the general path load but do not store, and the rows of a partial tile
-// beyond ny load from the last row.
+// on the general path load but do not store, nor do the rows of a partial
+// tile beyond ny, which load from the last row.
 // ---------------------------------------------------------------------------
 template <int S>
 struct PairStore;
@@ -704,7 +709,6 @@ struct PairStore<STORE_BF16_OFFSET> {
 template <int ARITH, int COLL, int S>
 __global__ __launch_bounds__(256) void fluid_fast_pair(const typename Store<S>::T* __restrict__ fin_t,
                                                        typename Store<S>::T* __restrict__ fout_t,
-                                                       const uint8_t* __restrict__ static_flags,
                                                        const uint8_t* __restrict__ dyn_prev,
                                                        const uint8_t* __restrict__ dyn_cur,
                                                        float* __restrict__ density, float4* __restrict__ velocity,
@@ -721,15 +725,14 @@ __global__ __launch_bounds__(256) void fluid_fast_pair(const typename Store<S>::
     const uint32_t r = pair - (uint32_t)z * per_plane;
     const uint32_t ty = r / pairs_x, px = r - ty * pairs_x;
     const uint32_t tile_a = ((uint32_t)z * (uint32_t)p.g.tiles_y + ty) * (uint32_t)p.g.tiles_x + 2u * px;
-    // the six flag bytes load with the populations and are tested after them
-    uint32_t flags_a = (uint32_t)static_flags[tile_a], flags_a1 = (uint32_t)dyn_prev[tile_a],
-             flags_a2 = (uint32_t)dyn_cur[tile_a];
-    uint32_t flags_b = (uint32_t)static_flags[tile_a + 1], flags_b1 = (uint32_t)dyn_prev[tile_a + 1],
-             flags_b2 = (uint32_t)dyn_cur[tile_a + 1];
+    // the four flag bytes load with the populations and are tested after them
+    uint32_t flags_a1 = (uint32_t)dyn_prev[tile_a], flags_a2 = (uint32_t)dyn_cur[tile_a];
+    uint32_t flags_b1 = (uint32_t)dyn_prev[tile_a + 1], flags_b2 = (uint32_t)dyn_cur[tile_a + 1];
     const int lane = (int)(threadIdx.x & 63u);
     const int wave = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int X0 = (int)px * 2 * TILE_X;
     const int xa = X0 + 2 * lane;
+    const bool in_grid = (int)ty * TILE_Y + wave < ny;
     const int y = min((int)ty * TILE_Y + wave, ny - 1);
 
     // wave-uniform sources along y and z; the halo elements along x
@@ -765,9 +768,9 @@ __global__ __launch_bounds__(256) void fluid_fast_pair(const typename Store<S>::
     // on it, and tests the flags before the population loads).
     asm volatile("" : BF_ASM19(v), "+s"(halo[1]), "+s"(halo[2]), "+s"(halo[7]), "+s"(halo[8]), "+s"(halo[9]),
                  "+s"(halo[10]), "+s"(halo[11]), "+s"(halo[12]), "+s"(halo[13]), "+s"(halo[14]));
-    asm volatile("" : "+v"(flags_a), "+v"(flags_a1), "+v"(flags_a2), "+v"(flags_b), "+v"(flags_b1), "+v"(flags_b2));
-    const bool general_a = (flags_a | flags_a1 | flags_a2) != 0;
-    const bool general_b = (flags_b | flags_b1 | flags_b2) != 0;
+    asm volatile("" : "+v"(flags_a1), "+v"(flags_a2), "+v"(flags_b1), "+v"(flags_b2));
+    const bool general_a = (flags_a1 | flags_a2) != 0;
+    const bool general_b = (flags_b1 | flags_b2) != 0;
     if (general_a && general_b) return;
     // the halo half within its word (population rows start at even elements)
     for_q(AllQ{}, [&](auto qc) {
@@ -791,7 +794,7 @@ __global__ __launch_bounds__(256) void fluid_fast_pair(const typename Store<S>::
             v[q] = (v[q] >> 16) | (second << 16);
         }
     });
-    const bool store = lane < 32 ? !general_a : !general_b;
+    const bool store = in_grid && (lane < 32 ? !general_a : !general_b);
     const bool sponge_on = p.sponge_strength > 0.0f;
     float act_n = 0.0f, restr_max = 0.0f;
     uint32_t out[19];
@@ -1326,13 +1329,13 @@ static hipError_t launch_fast_t(const FluidBuffers& b, const StepParams& p, hipS
         // two cells per lane over tile pairs (whole pairs along x)
         if (p.g.nx % (2 * TILE_X) == 0 && p.pair_cells) {
             hipLaunchKernelGGL((fluid_fast_pair<ARITH, COLL, S>), dim3(p.g.tiles / 2), dim3(256), 0, s,
-                               (const T*)b.fin, (T*)b.fout, b.static_flags, b.dyn_prev, b.dyn_cur, b.density,
-                               b.velocity, b.activation, p);
+                               (const T*)b.fin, (T*)b.fout, b.dyn_prev, b.dyn_cur, b.density, b.velocity,
+                               b.activation, p);
             return hipGetLastError();
         }
     }
     hipLaunchKernelGGL((fluid_fast<ARITH, COLL, S>), dim3(p.g.tiles), dim3(256), 0, s, (const T*)b.fin,
-                       (T*)b.fout, b.static_flags, b.dyn_prev, b.dyn_cur, b.density, b.velocity, b.activation, p);
+                       (T*)b.fout, b.dyn_prev, b.dyn_cur, b.density, b.velocity, b.activation, p);
     return hipGetLastError();
 }
 

@@ -8,14 +8,12 @@
 namespace bf {
 
 // Work list of the tiles that take the general path this step: flagged by
-// the static mask (partial or sponge tiles) or by solid cells of the
-// previous / current geometry.  Appends are aggregated per wavefront.
-__global__ __launch_bounds__(256) void build_general_list(const uint8_t* __restrict__ static_flags,
-                                                          const uint8_t* __restrict__ dyn_prev,
+// solid cells of the previous / current geometry.  Appends are aggregated per wavefront.
+__global__ __launch_bounds__(256) void build_general_list(const uint8_t* __restrict__ dyn_prev,
                                                           const uint8_t* __restrict__ dyn_cur, uint32_t tiles,
                                                           uint32_t* __restrict__ list, uint32_t* __restrict__ count) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool flagged = t < tiles && (static_flags[t] | dyn_prev[t] | dyn_cur[t]) != 0;
+    const bool flagged = t < tiles && (dyn_prev[t] | dyn_cur[t]) != 0;
     const unsigned long long b = __ballot(flagged);
     if (b == 0) return;
     const uint32_t lane = threadIdx.x & 63;
@@ -31,7 +29,6 @@ __global__ __launch_bounds__(256) void build_general_list(const uint8_t* __restr
 // Fixed-order sum of the per-tile partials of the tiles the general kernel
 // processed (flags identify them; other tiles contribute exactly zero).
 __global__ __launch_bounds__(256) void reduce_loads_tiles(const double* __restrict__ partials,
-                                                          const uint8_t* __restrict__ static_flags,
                                                           const uint8_t* __restrict__ dyn_prev,
                                                           const uint8_t* __restrict__ dyn_cur, uint32_t tiles,
                                                           double* __restrict__ block_out) {
@@ -40,7 +37,7 @@ __global__ __launch_bounds__(256) void reduce_loads_tiles(const double* __restri
     const uint32_t base = (blockIdx.x * blockDim.x + threadIdx.x) * PER_THREAD;
     for (uint32_t k = 0; k < PER_THREAD; ++k) {
         const uint32_t t = base + k;
-        if (t < tiles && (static_flags[t] | dyn_prev[t] | dyn_cur[t]) != 0) {
+        if (t < tiles && (dyn_prev[t] | dyn_cur[t]) != 0) {
 #pragma unroll
             for (int i = 0; i < 7; ++i) v[i] += partials[(size_t)t * 8 + i];
             v[7] = fmax(v[7], partials[(size_t)t * 8 + 7]);
@@ -292,8 +289,8 @@ hipError_t launch_poke_population(int storage, void* f, const Grid& g, unsigned 
 hipError_t launch_load_reduction(const FluidBuffers& b, const StepParams& p, uint32_t history_slot, hipStream_t s) {
     if (!p.accumulate_loads) return hipSuccess;
     const uint32_t blocks = (p.g.tiles + 1023) / 1024;
-    hipLaunchKernelGGL(reduce_loads_tiles, dim3(blocks), dim3(256), 0, s, b.partials, b.static_flags, b.dyn_prev,
-                       b.dyn_cur, p.g.tiles, b.block_out);
+    hipLaunchKernelGGL(reduce_loads_tiles, dim3(blocks), dim3(256), 0, s, b.partials, b.dyn_prev, b.dyn_cur,
+                       p.g.tiles, b.block_out);
     hipLaunchKernelGGL(reduce_loads_final, dim3(1), dim3(256), 0, s, b.block_out, blocks, b.activation, b.last_load,
                        b.history, history_slot);
     return hipGetLastError();
@@ -317,10 +314,10 @@ hipError_t launch_fluid_general(int arith, int storage, int coll, const FluidBuf
     return launch_fluid_general_fused(storage, coll, b, p, general_blocks, s);
 }
 
-hipError_t launch_build_general_list(const uint8_t* static_flags, const uint8_t* dyn_prev, const uint8_t* dyn_cur,
-                                     uint32_t tiles, uint32_t* list, uint32_t* count, hipStream_t s) {
-    hipLaunchKernelGGL(build_general_list, dim3((tiles + 255) / 256), dim3(256), 0, s, static_flags, dyn_prev,
-                       dyn_cur, tiles, list, count);
+hipError_t launch_build_general_list(const uint8_t* dyn_prev, const uint8_t* dyn_cur, uint32_t tiles, uint32_t* list,
+                                     uint32_t* count, hipStream_t s) {
+    hipLaunchKernelGGL(build_general_list, dim3((tiles + 255) / 256), dim3(256), 0, s, dyn_prev, dyn_cur,
+                       tiles, list, count);
     return hipGetLastError();
 }
 

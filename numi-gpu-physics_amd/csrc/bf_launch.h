@@ -15,7 +15,6 @@ struct FluidBuffers {
     const uint8_t* solid_prev;
     const uint8_t* solid_cur;
     const float4* wall;
-    const uint8_t* static_flags;
     const uint8_t* dyn_prev;
     const uint8_t* dyn_cur;
     uint32_t* general_list;
@@ -238,7 +237,6 @@ struct AdjointBuffers {
     const uint8_t* solid_prev;
     const uint8_t* solid_cur;
     const float4* wall;
-    const uint8_t* static_flags;
     const uint8_t* dyn_prev;
     const uint8_t* dyn_cur;
     const uint32_t* general_list;
@@ -325,8 +323,8 @@ hipError_t launch_fluid_fast_strict(int coll, const FluidBuffers& b, const StepP
 hipError_t launch_fluid_general_strict(int coll, const FluidBuffers& b, const StepParams& p, int general_blocks,
                                        hipStream_t s);
 hipError_t launch_load_reduction(const FluidBuffers& b, const StepParams& p, uint32_t history_slot, hipStream_t s);
-hipError_t launch_build_general_list(const uint8_t* static_flags, const uint8_t* dyn_prev, const uint8_t* dyn_cur,
-                                     uint32_t tiles, uint32_t* list, uint32_t* count, hipStream_t s);
+hipError_t launch_build_general_list(const uint8_t* dyn_prev, const uint8_t* dyn_cur, uint32_t tiles, uint32_t* list,
+                                     uint32_t* count, hipStream_t s);
 hipError_t launch_init_equilibrium(int storage, void* f, const uint8_t* solid, const float4* wall,
                                    const float* far_u, const Grid& g, hipStream_t s);
 hipError_t launch_init_shear_wave(int storage, void* f, float amplitude, const Grid& g, hipStream_t s);
