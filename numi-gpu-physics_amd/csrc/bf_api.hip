@@ -347,7 +347,6 @@ StepParams make_step_params(const bf_context* c) {
     p.load_component = (int)c->cfg.load_component;
     p.selected_part = (int)c->cfg.selected_part;
     p.accumulate_loads = c->cfg.accumulate_loads ? 1 : 0;
-    p.capture_fields = 0;
     p.omega_plus = c->cfg.omega_plus;
     p.omega_minus = c->cfg.omega_minus;
     p.sponge_strength = c->cfg.sponge_strength;
@@ -754,8 +753,6 @@ FluidBuffers fluid_buffers(const bf_context* c, int64_t s) {
     b.block_out = c->block_out;
     b.last_load = c->last_load;
     b.history = c->history;
-    b.density = c->density;
-    b.velocity = c->velocity;
     b.activation = &c->counters[4 + 2 * par2(s)];
     b.body = c->body;
     return b;
@@ -2636,8 +2633,6 @@ bf_status bf_adjoint_gradient(bf_context* c, uint32_t steps, const double* load_
             fb.general_list = a.slot_list[set] + (uint64_t)(s - sa_) * c->g.tiles;
             fb.general_count = a.slot_count[set] + (s - sa_);
             fb.partials = c->partials;
-            fb.density = c->density;
-            fb.velocity = c->velocity;
             fb.activation = &c->counters[8];
             fb.body = c->body;
             StepParams ps = pf;

@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace bf {
 
 // D3Q19 velocity set, ordering 0; +-x; +-y; +-z; (+-1,+-1,0); (+-1,0,+-1);
@@ -78,7 +80,6 @@ struct StepParams {
     int load_component;
     int selected_part;
     int accumulate_loads;
-    int capture_fields;
     int fast_priority;         // s_setprio level of the fast kernel's wavefronts (0..3)
     int pair_cells;            // 2-byte storage: fast tiles two cells per lane (fluid_fast_pair)
     int general_priority;      // and of the general kernel's
@@ -159,12 +160,29 @@ __host__ __device__ __forceinline__ size_t pop_index(const Grid& g, int q, int x
     return ((size_t)row * 19u + (size_t)q) * (size_t)g.nx + (size_t)x;
 }
 
+// First element of direction q of `row`: row_ptr + x is element pop_index(q, x, row).
+template <int S, typename T>
+__device__ __forceinline__ T* row_ptr(T* __restrict__ f, const Grid& g, int q, uint32_t row) {
+    return f + pop_index<S>(g, q, 0, row);
+}
+// Element x >= 0 of a row, as row base + 32-bit byte offset: with a
+// wave-uniform base the access takes the base from scalar registers.
+template <typename T>
+__device__ __forceinline__ T* row_at(T* __restrict__ row, int x) {
+    using C = std::conditional_t<std::is_const<T>::value, const char, char>;
+    return reinterpret_cast<T*>(reinterpret_cast<C*>(row) + (uint32_t)x * (uint32_t)sizeof(T));
+}
+
 template <>
 struct Store<STORE_FP32> {
     using T = float;
     __device__ static inline float load(const T* __restrict__ p, size_t i, int) { return p[i]; }
+    __device__ static inline float load(const T* __restrict__ row, int x, int) { return *row_at(row, x); }
     __device__ static inline void store(T* __restrict__ p, size_t i, int, float v) {
         __builtin_nontemporal_store(v, p + i);
+    }
+    __device__ static inline void store(T* __restrict__ row, int x, int, float v) {
+        __builtin_nontemporal_store(v, row_at(row, x));
     }
 };
 
@@ -174,8 +192,14 @@ struct Store<STORE_FP16_OFFSET> {
     __device__ static inline float load(const T* __restrict__ p, size_t i, int q) {
         return (float)p[i] + weight<float>(q);
     }
+    __device__ static inline float load(const T* __restrict__ row, int x, int q) {
+        return (float)*row_at(row, x) + weight<float>(q);
+    }
     __device__ static inline void store(T* __restrict__ p, size_t i, int q, float v) {
         __builtin_nontemporal_store((T)(v - weight<float>(q)), p + i);
+    }
+    __device__ static inline void store(T* __restrict__ row, int x, int q, float v) {
+        __builtin_nontemporal_store((T)(v - weight<float>(q)), row_at(row, x));
     }
 };
 
@@ -188,8 +212,14 @@ struct Store<STORE_BF16_OFFSET> {
     __device__ static inline float load(const T* __restrict__ p, size_t i, int q) {
         return to_float(p[i]) + weight<float>(q);
     }
+    __device__ static inline float load(const T* __restrict__ row, int x, int q) {
+        return to_float(*row_at(row, x)) + weight<float>(q);
+    }
     __device__ static inline void store(T* __restrict__ p, size_t i, int q, float v) {
         __builtin_nontemporal_store(from_float(v - weight<float>(q)), p + i);
+    }
+    __device__ static inline void store(T* __restrict__ row, int x, int q, float v) {
+        __builtin_nontemporal_store(from_float(v - weight<float>(q)), row_at(row, x));
     }
 };
 

@@ -94,6 +94,13 @@ __device__ __forceinline__ void moments(const float (&f)[19], float& rho, float&
     });
 }
 
+// A value above every positivity floor of a cell (with a margin of three for
+// rounding): floor_q = max(1e-12, 1e-6 max(feq_q, 0)), and every
+// feq_q <= rho (1/3 + 0.3 u^2).
+__device__ __forceinline__ float limiter_bound(float rho, float u2_15) {
+    return fmaf(1.0e-6f * rho, 1.0f + u2_15, 2.0e-12f);
+}
+
 template <int COLL>
 __device__ __forceinline__ void collide(const float (&f)[19], float rho, float ux, float uy, float uz,
                                         float op, float om, float (&post)[19], float& act, float& restr) {
@@ -106,6 +113,13 @@ __device__ __forceinline__ void collide(const float (&f)[19], float rho, float u
     });
     act = 0.0f;
     restr = 0.0f;
+    // Positivity limiters: the per-direction form (a floor of 1e-12 or 1e-6
+    // of the equilibrium, a comparison and, where it acts, a division for each
+    // direction) runs only in cells whose smallest candidate lies below a
+    // bound no floor exceeds: feq <= rho (1/3 + 0.3 u^2) in every direction.
+    // Elsewhere it cannot act, so the results are the same bit for bit; the
+    // gate costs half an instruction per direction instead of five.
+    const float limit_below = limiter_bound(rho, u2_15);
     if constexpr (COLL == COLL_TRT) {
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
@@ -117,46 +131,53 @@ __device__ __forceinline__ void collide(const float (&f)[19], float rho, float u
             post[q] = f[q] - op * (fp - ep) - om * (fm - em);
         });
     } else if constexpr (COLL == COLL_TRT_SYMMETRIC_LIMITER) {
-        float sinc[19], ainc[19];
-        float sscale = 1.0f;
-        for_q(AllQ{}, [&](auto qc) {
+        // symmetric and antisymmetric increment of direction q (formed again
+        // where the limiter acts, rather than kept: 38 registers)
+        auto increments = [&](auto qc, float& si, float& ai) {
             constexpr int q = decltype(qc)::value;
             constexpr int o = opp(q);
             float fp = 0.5f * (f[q] + f[o]);
             float fm = 0.5f * (f[q] - f[o]);
             float ep = 0.5f * (feq[q] + feq[o]);
             float em = 0.5f * (feq[q] - feq[o]);
-            float si = -op * (fp - ep);
-            float ai = -om * (fm - em);
-            sinc[q] = si;
-            ainc[q] = ai;
-            if (si < 0.0f) {
-                float base = f[q] + ai;
-                float floorv = fmaxf(1.0e-12f, 1.0e-6f * fmaxf(feq[q], 0.0f));
-                if (base + si < floorv) {
-                    float cand = (base - floorv) / fmaxf(-si, 1.0e-30f);
-                    cand = fminf(fmaxf(cand, 0.0f), 1.0f);
-                    sscale = fminf(sscale, cand);
-                }
-            }
-        });
-        if (sscale < 1.0f) {
-            act = 1.0f;
-            restr = 1.0f - sscale;
-        }
+            si = -op * (fp - ep);
+            ai = -om * (fm - em);
+            post[q] = f[q] - op * (fp - ep) - om * (fm - em);
+        };
+        float sscale = 1.0f;
+        float lowest = INFINITY;
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            constexpr int o = opp(q);
-            if (sscale < 1.0f) {
-                post[q] = f[q] + sscale * sinc[q] + ainc[q];
-            } else {
-                float fp = 0.5f * (f[q] + f[o]);
-                float fm = 0.5f * (f[q] - f[o]);
-                float ep = 0.5f * (feq[q] + feq[o]);
-                float em = 0.5f * (feq[q] - feq[o]);
-                post[q] = f[q] - op * (fp - ep) - om * (fm - em);
-            }
+            float si, ai;
+            increments(qc, si, ai);
+            lowest = fminf(lowest, f[q] + ai + si);
         });
+        if (lowest < limit_below) {
+            for_q(AllQ{}, [&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                float si, ai;
+                increments(qc, si, ai);
+                if (si < 0.0f) {
+                    float base = f[q] + ai;
+                    float floorv = fmaxf(1.0e-12f, 1.0e-6f * fmaxf(feq[q], 0.0f));
+                    if (base + si < floorv) {
+                        float cand = (base - floorv) / fmaxf(-si, 1.0e-30f);
+                        cand = fminf(fmaxf(cand, 0.0f), 1.0f);
+                        sscale = fminf(sscale, cand);
+                    }
+                }
+            });
+            if (sscale < 1.0f) {
+                act = 1.0f;
+                restr = 1.0f - sscale;
+                for_q(AllQ{}, [&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    float si, ai;
+                    increments(qc, si, ai);
+                    post[q] = f[q] + sscale * si + ai;
+                });
+            }
+        }
     } else {
         // Regularized / RR3 (BirdFlow.metal:2917-3062).  Terms whose factor is
         // a zero component of c_q are dropped at compile time: each is an
@@ -189,6 +210,7 @@ __device__ __forceinline__ void collide(const float (&f)[19], float rho, float u
         float aYzz = uy * dg2 + 2.0f * uz * od2;
         float unb[19];
         float scale = 1.0f;
+        float lowest = INFINITY;
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
             constexpr int X = cx(q), Y = cy(q), Z = cz(q);
@@ -214,22 +236,38 @@ __device__ __forceinline__ void collide(const float (&f)[19], float rho, float u
                 if constexpr (Y != 0) add((Y > 0 ? hzz : -hzz) * aYzz);
                 reg = reg + w * 13.5f * third;
             }
-            const float cand = feq[q] + (1.0f - op) * reg;
-            unb[q] = cand;
-            const float floorv = fmaxf(1.0e-12f, 1.0e-6f * fmaxf(feq[q], 0.0f));
-            if (cand < floorv) {
-                float adm = (feq[q] - floorv) / fmaxf(feq[q] - cand, 1.0e-30f);
-                adm = fminf(fmaxf(adm, 0.0f), 1.0f);
-                scale = fminf(scale, adm);
+            unb[q] = feq[q] + (1.0f - op) * reg;
+            lowest = fminf(lowest, unb[q]);
+        });
+        if (lowest < limit_below) {
+            for_q(AllQ{}, [&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                const float floorv = fmaxf(1.0e-12f, 1.0e-6f * fmaxf(feq[q], 0.0f));
+                if (unb[q] < floorv) {
+                    float adm = (feq[q] - floorv) / fmaxf(feq[q] - unb[q], 1.0e-30f);
+                    adm = fminf(fmaxf(adm, 0.0f), 1.0f);
+                    scale = fminf(scale, adm);
+                }
+            });
+            if (scale < 1.0f) {
+                act = 1.0f;
+                restr = 1.0f - scale;
             }
+        }
+        // feq + scale (unb - feq); a scale of 1 multiplies nothing
+        for_q(AllQ{}, [&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            unb[q] = unb[q] - feq[q];
         });
         if (scale < 1.0f) {
-            act = 1.0f;
-            restr = 1.0f - scale;
+            for_q(AllQ{}, [&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                unb[q] = scale * unb[q];
+            });
         }
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            post[q] = feq[q] + scale * (unb[q] - feq[q]);
+            post[q] = feq[q] + unb[q];
         });
     }
 }
@@ -242,8 +280,7 @@ __device__ __forceinline__ void collide(const float (&f)[19], float rho, float u
 // Hermite terms) through f_q - f_{q+1}, so each operator of collide<COLL>
 // yields an even part P and an odd part Q per pair with post_q = P + Q and
 // post_{q+1} = P - Q.  Products are fused into FMAs.  The positivity limiters
-// run their per-direction form only in cells where some post-collision
-// population falls below 1e-12 + 1e-6 |feq|; elsewhere they cannot act.
+// are gated as in collide<COLL>.
 // ---------------------------------------------------------------------------
 using AllPairs = QSeq<0, 1, 2, 3, 4, 5, 6, 7, 8>;   // pair k: q = 2k + 1 and q + 1
 
@@ -294,13 +331,14 @@ __device__ __forceinline__ void collide_fused(const float (&f)[19], float op, fl
             post[q + 1] = fmaf(om, ha[k], fmaf(-op, hs[k], f[q + 1]));
         });
         if constexpr (COLL == COLL_TRT_SYMMETRIC_LIMITER) {
-            float lo = fmaf(-1.0e-6f, fabsf(feq0), post[0]);
+            // f + ai + si as the limiter forms it, gated as in collide<COLL>
+            float lo = fmaf(-op, f[0] - feq0, f[0]);
             for_q(AllPairs{}, [&](auto kc) {
                 constexpr int k = decltype(kc)::value, q = 2 * k + 1;
-                lo = fminf(lo, fminf(fmaf(-1.0e-6f, fabsf(A[k] + B[k]), post[q]),
-                                     fmaf(-1.0e-6f, fabsf(A[k] - B[k]), post[q + 1])));
+                const float si = -op * hs[k], ai = -om * ha[k];
+                lo = fminf(lo, fminf(f[q] + ai + si, f[q + 1] - ai + si));
             });
-            if (lo < 2.0e-12f) {
+            if (lo < limiter_bound(rho, 1.0f - base)) {
                 // scale the symmetric increment so that no population falls
                 // below its floor (BirdFlow.metal:3100-3140)
                 float sscale = 1.0f;
@@ -415,13 +453,12 @@ __device__ __forceinline__ void collide_fused(const float (&f)[19], float op, fl
             post[q] = P + Q;
             post[q + 1] = P - Q;
         });
-        float lo = fmaf(-1.0e-6f, fabsf(feq0), post[0]);
+        float lo = post[0];
         for_q(AllPairs{}, [&](auto kc) {
             constexpr int k = decltype(kc)::value, q = 2 * k + 1;
-            lo = fminf(lo, fminf(fmaf(-1.0e-6f, fabsf(A[k] + B[k]), post[q]),
-                                 fmaf(-1.0e-6f, fabsf(A[k] - B[k]), post[q + 1])));
+            lo = fminf(lo, fminf(post[q], post[q + 1]));
         });
-        if (lo < 2.0e-12f) {
+        if (lo < limiter_bound(rho, 1.0f - base)) {
             // positivity limiter: blend toward equilibrium just enough
             float scale = 1.0f;
             auto limit = [&](float feq, float cand) {
@@ -515,34 +552,20 @@ __device__ __forceinline__ bool orphan(const Sources& s) {
            (cz(q) > 0 && s.zp_far) || (cz(q) < 0 && s.zm_far);
 }
 
+// Stores the post-collision populations of cell (x, row), blended toward the
+// far-field equilibrium where sponge > 0; returns their sum.
 template <int S>
-__device__ __forceinline__ void write_post(typename Store<S>::T* __restrict__ fout, int x, uint32_t row,
-                                           const float (&post)[19], float sponge, const StepParams& p,
-                                           float& crho, float& cmx, float& cmy, float& cmz) {
-    crho = 0.0f;
-    cmx = 0.0f;
-    cmy = 0.0f;
-    cmz = 0.0f;
+__device__ __forceinline__ float write_post(typename Store<S>::T* __restrict__ fout, int x, uint32_t row,
+                                            const float (&post)[19], float sponge, const StepParams& p) {
+    float density = 0.0f;
     for_q(AllQ{}, [&](auto qc) {
         constexpr int q = decltype(qc)::value;
         float v = post[q];
         if (sponge > 0.0f) v = v + (p.far_eq[q] - v) * sponge;
-        Store<S>::store(fout, pop_index<S>(p.g, q, x, row), q, v);
-        crho = crho + v;
-        if constexpr (cx(q) > 0) cmx = cmx + v;
-        if constexpr (cx(q) < 0) cmx = cmx - v;
-        if constexpr (cy(q) > 0) cmy = cmy + v;
-        if constexpr (cy(q) < 0) cmy = cmy - v;
-        if constexpr (cz(q) > 0) cmz = cmz + v;
-        if constexpr (cz(q) < 0) cmz = cmz - v;
+        Store<S>::store(row_ptr<S>(fout, p.g, q, row), x, q, v);
+        density = density + v;
     });
-}
-
-__device__ __forceinline__ void capture(float* __restrict__ density, float4* __restrict__ velocity, uint32_t gid,
-                                        float crho, float cmx, float cmy, float cmz) {
-    crho = fmaxf(crho, 1.0e-8f);
-    density[gid] = crho;
-    velocity[gid] = make_float4(cmx / crho, cmy / crho, cmz / crho, 0.0f);
+    return density;
 }
 
 // ---------------------------------------------------------------------------
@@ -553,7 +576,6 @@ __global__ __launch_bounds__(256) void fluid_fast(const typename Store<S>::T* __
                                                   typename Store<S>::T* __restrict__ fout,
                                                   const uint8_t* __restrict__ dyn_prev,
                                                   const uint8_t* __restrict__ dyn_cur,
-                                                  float* __restrict__ density, float4* __restrict__ velocity,
                                                   uint32_t* __restrict__ activation, StepParams p) {
     set_priority(p.fast_priority);
     const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
@@ -570,15 +592,24 @@ __global__ __launch_bounds__(256) void fluid_fast(const typename Store<S>::T* __
     // clamp changes nothing.  Partial tiles used to take the general path:
     // a grid of odd sides then spent most of its step there (203x117x91 BF16,
     // 3,407 of 10,920 tiles: 99 of 163 us per step).
-    const int xl = x0 + (int)(threadIdx.x & (TILE_X - 1)), yl = y0 + (int)(threadIdx.x / TILE_X);
+    //
+    // A wavefront is one row of the tile: y, the nine source rows and
+    // everything derived from them are wave-uniform, so the row addresses and
+    // the y / z face tests run on the scalar unit and a load is one
+    // instruction (row base in scalar registers + a 32-bit lane offset).
+    const int wave = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int xl = x0 + (int)(threadIdx.x & (TILE_X - 1)), yl = y0 + wave;
     const bool in_grid = xl < nx && yl < ny;
     const int x = min(xl, nx - 1);
     const int y = min(yl, ny - 1);
 
     bool xm_far = false, xp_far = false, ym_far = false, yp_far = false, zm_far = false, zp_far = false;
-    // source coordinates for c = +1 (s = v - 1) and c = -1 (s = v + 1)
-    const int xs_p = shift_axis(x, 1, nx, p.bc[0][0], p.bc[0][1], xm_far);
-    const int xs_m = shift_axis(x, -1, nx, p.bc[0][0], p.bc[0][1], xp_far);
+    // source coordinates for c = +1 (s = v - 1) and c = -1 (s = v + 1); a
+    // source beyond a far-field face loads an in-domain cell and discards it
+    int xs_p = shift_axis(x, 1, nx, p.bc[0][0], p.bc[0][1], xm_far);
+    int xs_m = shift_axis(x, -1, nx, p.bc[0][0], p.bc[0][1], xp_far);
+    if (xm_far) xs_p = x;
+    if (xp_far) xs_m = x;
     const int ys_p = shift_axis(y, 1, ny, p.bc[1][0], p.bc[1][1], ym_far);
     const int ys_m = shift_axis(y, -1, ny, p.bc[1][0], p.bc[1][1], yp_far);
     const int zs_p = shift_axis(z, 1, nz, p.bc[2][0], p.bc[2][1], zm_far);
@@ -586,19 +617,15 @@ __global__ __launch_bounds__(256) void fluid_fast(const typename Store<S>::T* __
 
     const uint32_t row_self = (uint32_t)y + (uint32_t)ny * (uint32_t)z;
     float f[19];
-    bool far_q[19];
     for_q(AllQ{}, [&](auto qc) {
         constexpr int q = decltype(qc)::value;
         const int xs = cx(q) > 0 ? xs_p : (cx(q) < 0 ? xs_m : x);
         const int ys = cy(q) > 0 ? ys_p : (cy(q) < 0 ? ys_m : y);
         const int zs = cz(q) > 0 ? zs_p : (cz(q) < 0 ? zs_m : z);
-        const bool far = (cx(q) > 0 && xm_far) || (cx(q) < 0 && xp_far) || (cy(q) > 0 && ym_far)
-            || (cy(q) < 0 && yp_far) || (cz(q) > 0 && zm_far) || (cz(q) < 0 && zp_far);
-        const uint32_t row_src = (uint32_t)ys + (uint32_t)ny * (uint32_t)zs;
-        // unconditional load: a far-field source reads an in-domain cell and
-        // discards it
-        f[q] = Store<S>::load(fin, far ? pop_index<S>(p.g, q, x, row_self) : pop_index<S>(p.g, q, xs, row_src), q);
-        far_q[q] = far;
+        const bool far = (cy(q) > 0 && ym_far) || (cy(q) < 0 && yp_far) || (cz(q) > 0 && zm_far) ||
+                         (cz(q) < 0 && zp_far);
+        const uint32_t row_src = far ? row_self : (uint32_t)ys + (uint32_t)ny * (uint32_t)zs;
+        f[q] = Store<S>::load(row_ptr<S>(fin, p.g, q, row_src), xs, q);
     });
     // One empty asm over all 19 loaded values: every load is issued, without
     // a branch, before any of them is consumed (otherwise the far-field
@@ -607,10 +634,16 @@ __global__ __launch_bounds__(256) void fluid_fast(const typename Store<S>::T* __
     // none sinks below the tile test.
     asm volatile("" : BF_ASM19(f));
     if (general_tile) return;
-    for_q(AllQ{}, [&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        if (far_q[q]) f[q] = p.far_eq[q];
-    });
+    // far-field sources: only the wavefronts at a far-field face take the
+    // selects (a uniform branch)
+    if (ym_far || yp_far || zm_far || zp_far || __any(xm_far || xp_far)) {
+        for_q(AllQ{}, [&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            const bool far = (cx(q) > 0 && xm_far) || (cx(q) < 0 && xp_far) || (cy(q) > 0 && ym_far) ||
+                             (cy(q) < 0 && yp_far) || (cz(q) > 0 && zm_far) || (cz(q) < 0 && zp_far);
+            if (far) f[q] = p.far_eq[q];
+        });
+    }
 
     float post[19];
     float act, restr;
@@ -623,18 +656,14 @@ __global__ __launch_bounds__(256) void fluid_fast(const typename Store<S>::T* __
         const float ux = mx / rho, uy = my / rho, uz = mz / rho;
         collide<COLL>(f, rho, ux, uy, uz, p.omega_plus, p.omega_minus, post, act, restr);
     }
-    const uint32_t gid = (uint32_t)x + (uint32_t)nx * row_self;
     // wall-free sponge tiles stream here too (the sponge is a per-cell blend
     // toward the far-field equilibrium after the collision); a uniform branch,
     // so that without a sponge the store path carries no blend
-    float crho, cmx, cmy, cmz;
     if (in_grid) {
         if (p.sponge_strength > 0.0f)
-            write_post<S>(fout, x, row_self, post, sponge_factor(p, x, y, z), p, crho, cmx, cmy, cmz);
+            guard_finite(p, write_post<S>(fout, x, row_self, post, sponge_factor(p, x, y, z), p));
         else
-            write_post<S>(fout, x, row_self, post, 0.0f, p, crho, cmx, cmy, cmz);
-        guard_finite(p, crho);
-        if (p.capture_fields) capture(density, velocity, gid, crho, cmx, cmy, cmz);
+            guard_finite(p, write_post<S>(fout, x, row_self, post, 0.0f, p));
     }
     if constexpr (COLL != COLL_TRT) {
         // Limiter activations of fast cells: an exact count and the maximum
@@ -680,11 +709,18 @@ struct PairStore;
 
 template <>
 struct PairStore<STORE_FP16_OFFSET> {
+    // h * 1 + w with h converted exactly: one mixed-precision FMA instead of a
+    // conversion and an addition (the same single rounding)
     __device__ static inline float lo(uint32_t u, int q) {
-        return (float)__builtin_bit_cast(_Float16, (uint16_t)(u & 0xffffu)) + weight<float>(q);
+        float r;
+        asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(u), "s"(weight<float>(q)));
+        return r;
     }
     __device__ static inline float hi(uint32_t u, int q) {
-        return (float)__builtin_bit_cast(_Float16, (uint16_t)(u >> 16)) + weight<float>(q);
+        float r;
+        asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+            : "=v"(r) : "v"(u), "s"(weight<float>(q)));
+        return r;
     }
     __device__ static inline uint32_t pack(float a, float b, int q) {
         typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -711,7 +747,6 @@ __global__ __launch_bounds__(256) void fluid_fast_pair(const typename Store<S>::
                                                        typename Store<S>::T* __restrict__ fout_t,
                                                        const uint8_t* __restrict__ dyn_prev,
                                                        const uint8_t* __restrict__ dyn_cur,
-                                                       float* __restrict__ density, float4* __restrict__ velocity,
                                                        uint32_t* __restrict__ activation, StepParams p) {
     static_assert(S == STORE_FP16_OFFSET || S == STORE_BF16_OFFSET, "two-byte storage only");
     set_priority(p.fast_priority);
@@ -772,33 +807,29 @@ __global__ __launch_bounds__(256) void fluid_fast_pair(const typename Store<S>::
     const bool general_a = (flags_a1 | flags_a2) != 0;
     const bool general_b = (flags_b1 | flags_b2) != 0;
     if (general_a && general_b) return;
-    // the halo half within its word (population rows start at even elements)
-    for_q(AllQ{}, [&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        if constexpr (cx(q) != 0) {
-            const int xh = cx(q) > 0 ? xh_lo : xh_hi;
-            halo[q] = (xh & 1) ? (halo[q] >> 16) : (halo[q] & 0xffffu);
-        }
-    });
-
-    // shift the x-neighbour halves into place
+    // Shift the x-neighbour halves into place: the neighbour lane's word by a
+    // DPP wavefront shift, whose end lane keeps the halo word instead (its
+    // element moved, on the scalar unit, to the half the next instruction
+    // reads; population rows start at even elements), then one funnel shift
+    // per direction takes the neighbour's half and this lane's other one.
     for_q(AllQ{}, [&](auto qc) {
         constexpr int q = decltype(qc)::value;
         if constexpr (cx(q) > 0) {
-            const uint32_t below = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[q], 0x138, 0xf, 0xf, false);
-            const uint32_t first = lane == 0 ? halo[q] : (below >> 16);
-            v[q] = first | (v[q] << 16);
+            const uint32_t end = (xh_lo & 1) ? halo[q] : (halo[q] << 16);
+            const uint32_t below = (uint32_t)__builtin_amdgcn_update_dpp((int)end, (int)v[q], 0x138, 0xf, 0xf, false);
+            v[q] = __builtin_amdgcn_alignbit(v[q], below, 16);
         } else if constexpr (cx(q) < 0) {
-            const uint32_t above = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[q], 0x130, 0xf, 0xf, false);
-            const uint32_t second = lane == 63 ? halo[q] : (above & 0xffffu);
-            v[q] = (v[q] >> 16) | (second << 16);
+            const uint32_t end = (xh_hi & 1) ? (halo[q] >> 16) : halo[q];
+            const uint32_t above = (uint32_t)__builtin_amdgcn_update_dpp((int)end, (int)v[q], 0x130, 0xf, 0xf, false);
+            v[q] = __builtin_amdgcn_alignbit(above, v[q], 16);
         }
     });
     const bool store = in_grid && (lane < 32 ? !general_a : !general_b);
     const bool sponge_on = p.sponge_strength > 0.0f;
+    const bool any_far = ym_far || yp_far || zm_far || zp_far || xlo_far || xhi_far;
     float act_n = 0.0f, restr_max = 0.0f;
     uint32_t out[19];
-    float crho[2], cmx[2], cmy[2], cmz[2];
+    float crho[2];
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
         const int x = xa + c;
@@ -806,11 +837,18 @@ __global__ __launch_bounds__(256) void fluid_fast_pair(const typename Store<S>::
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
             f[q] = c == 0 ? PairStore<S>::lo(v[q], q) : PairStore<S>::hi(v[q], q);
-            bool far = far_yz[q];
-            if constexpr (cx(q) > 0) far = far || (xlo_far && c == 0 && lane == 0);
-            if constexpr (cx(q) < 0) far = far || (xhi_far && c == 1 && lane == 63);
-            if (far) f[q] = p.far_eq[q];
         });
+        // far-field sources: only the wavefronts at a far-field face take the
+        // selects (a uniform branch)
+        if (any_far) {
+            for_q(AllQ{}, [&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                bool far = far_yz[q];
+                if constexpr (cx(q) > 0) far = far || (xlo_far && c == 0 && lane == 0);
+                if constexpr (cx(q) < 0) far = far || (xhi_far && c == 1 && lane == 63);
+                if (far) f[q] = p.far_eq[q];
+            });
+        }
         float post[19];
         float act, restr;
         if constexpr (ARITH == ARITH_FUSED) {
@@ -823,24 +861,19 @@ __global__ __launch_bounds__(256) void fluid_fast_pair(const typename Store<S>::
         }
         act_n += act;
         restr_max = fmaxf(restr_max, restr);
-        const float sponge = sponge_on ? sponge_factor(p, x, y, z) : 0.0f;
+        if (sponge_on) {
+            const float sponge = sponge_factor(p, x, y, z);
+            for_q(AllQ{}, [&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                if (sponge > 0.0f) post[q] = post[q] + (p.far_eq[q] - post[q]) * sponge;
+            });
+        }
         crho[c] = 0.0f;
-        cmx[c] = 0.0f;
-        cmy[c] = 0.0f;
-        cmz[c] = 0.0f;
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            float val = post[q];
-            if (sponge > 0.0f) val = val + (p.far_eq[q] - val) * sponge;
-            if (c == 0) out[q] = __float_as_uint(val);
-            else out[q] = PairStore<S>::pack(__uint_as_float(out[q]), val, q);
-            crho[c] = crho[c] + val;
-            if constexpr (cx(q) > 0) cmx[c] = cmx[c] + val;
-            if constexpr (cx(q) < 0) cmx[c] = cmx[c] - val;
-            if constexpr (cy(q) > 0) cmy[c] = cmy[c] + val;
-            if constexpr (cy(q) < 0) cmy[c] = cmy[c] - val;
-            if constexpr (cz(q) > 0) cmz[c] = cmz[c] + val;
-            if constexpr (cz(q) < 0) cmz[c] = cmz[c] - val;
+            if (c == 0) out[q] = __float_as_uint(post[q]);
+            else out[q] = PairStore<S>::pack(__uint_as_float(out[q]), post[q], q);
+            crho[c] = crho[c] + post[q];
         });
     }
     if (store) {
@@ -849,11 +882,6 @@ __global__ __launch_bounds__(256) void fluid_fast_pair(const typename Store<S>::
             __builtin_nontemporal_store(out[q], fout + (pop_index<S>(p.g, q, xa, row_self) >> 1));
         });
         guard_finite(p, crho[0] + crho[1]);
-        if (p.capture_fields) {
-            const uint32_t gid = (uint32_t)xa + (uint32_t)nx * row_self;
-            capture(density, velocity, gid, crho[0], cmx[0], cmy[0], cmz[0]);
-            capture(density, velocity, gid + 1, crho[1], cmx[1], cmy[1], cmz[1]);
-        }
     }
     if constexpr (COLL != COLL_TRT) {
         // limiter activations of the stored cells: an exact count and the
@@ -903,8 +931,7 @@ struct CellLoad {
 template <int ARITH, int COLL, int S>
 __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restrict__ fin, typename Store<S>::T* __restrict__ fout,
                              const uint8_t* __restrict__ solid_prev, const uint8_t* __restrict__ solid_cur,
-                             const float4* __restrict__ wall, float* __restrict__ density,
-                             float4* __restrict__ velocity, const StepParams& p, int x, int y, int z,
+                             const float4* __restrict__ wall, const StepParams& p, int x, int y, int z,
                              float bx, float by, float bz, CellLoad& L) {
     const Grid& g = p.g;
     const uint32_t row = (uint32_t)y + (uint32_t)g.ny * (uint32_t)z;
@@ -925,7 +952,7 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
         const float4 wv = wall[gid];
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            Store<S>::store(fout, pop_index<S>(g, q, x, row), q, equilibrium<float>(q, 1.0f, wv.x, wv.y, wv.z));
+            Store<S>::store(row_ptr<S>(fout, g, q, row), x, q, equilibrium<float>(q, 1.0f, wv.x, wv.y, wv.z));
         });
         if (p.accumulate_loads && !was_solid && include_topology) {
             float prho = 0.0f, pmx = 0.0f, pmy = 0.0f, pmz = 0.0f;
@@ -944,10 +971,6 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
             L.fy = cvy * fscale;
             L.fz = cvz * fscale;
             cross3(ax, ay, az, L.fx, L.fy, L.fz, L.tx, L.ty, L.tz);
-        }
-        if (p.capture_fields) {
-            density[gid] = 1.0f;
-            velocity[gid] = make_float4(wv.x, wv.y, wv.z, 0.0f);
         }
         return;
     }
@@ -1239,10 +1262,7 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
         const float ux = mx / rho, uy = my / rho, uz = mz / rho;
         collide<COLL>(f, rho, ux, uy, uz, p.omega_plus, p.omega_minus, post, act, restr);
     }
-    float crho, cmx, cmy, cmz;
-    write_post<S>(fout, x, row, post, sponge, p, crho, cmx, cmy, cmz);
-    guard_finite(p, crho);
-    if (p.capture_fields) capture(density, velocity, gid, crho, cmx, cmy, cmz);
+    guard_finite(p, write_post<S>(fout, x, row, post, sponge, p));
     if (p.accumulate_loads) {
         L.fx = flx * fscale;
         L.fy = fly * fscale;
@@ -1294,7 +1314,6 @@ __global__ __launch_bounds__(256) void fluid_general(const typename Store<S>::T*
                                                      const uint32_t* __restrict__ general_list,
                                                      const uint32_t* __restrict__ general_count,
                                                      double* __restrict__ partials,
-                                                     float* __restrict__ density, float4* __restrict__ velocity,
                                                      const double* __restrict__ body, StepParams p) {
     set_priority(p.general_priority);
     const uint32_t count = *general_count;
@@ -1305,11 +1324,10 @@ __global__ __launch_bounds__(256) void fluid_general(const typename Store<S>::T*
         int x0, y0, z;
         tile_origin(p.g, tile, x0, y0, z);
         const int x = x0 + (int)(threadIdx.x & (TILE_X - 1));
-        const int y = y0 + (int)(threadIdx.x / TILE_X);
+        const int y = y0 + (int)__builtin_amdgcn_readfirstlane(threadIdx.x / TILE_X);
         CellLoad L{0, 0, 0, 0, 0, 0, 0, 0};
         if (x < p.g.nx && y < p.g.ny)
-            general_cell<ARITH, COLL, S>(fin, fout, solid_prev, solid_cur, wall, density, velocity, p, x, y, z, bx, by,
-                                             bz, L);
+            general_cell<ARITH, COLL, S>(fin, fout, solid_prev, solid_cur, wall, p, x, y, z, bx, by, bz, L);
         if (p.accumulate_loads) {
             double v[8] = {(double)L.fx, (double)L.fy, (double)L.fz, (double)L.tx,
                            (double)L.ty, (double)L.tz, (double)L.act, (double)L.restr};
@@ -1329,13 +1347,12 @@ static hipError_t launch_fast_t(const FluidBuffers& b, const StepParams& p, hipS
         // two cells per lane over tile pairs (whole pairs along x)
         if (p.g.nx % (2 * TILE_X) == 0 && p.pair_cells) {
             hipLaunchKernelGGL((fluid_fast_pair<ARITH, COLL, S>), dim3(p.g.tiles / 2), dim3(256), 0, s,
-                               (const T*)b.fin, (T*)b.fout, b.dyn_prev, b.dyn_cur, b.density, b.velocity,
-                               b.activation, p);
+                               (const T*)b.fin, (T*)b.fout, b.dyn_prev, b.dyn_cur, b.activation, p);
             return hipGetLastError();
         }
     }
     hipLaunchKernelGGL((fluid_fast<ARITH, COLL, S>), dim3(p.g.tiles), dim3(256), 0, s, (const T*)b.fin,
-                       (T*)b.fout, b.dyn_prev, b.dyn_cur, b.density, b.velocity, b.activation, p);
+                       (T*)b.fout, b.dyn_prev, b.dyn_cur, b.activation, p);
     return hipGetLastError();
 }
 
@@ -1344,7 +1361,7 @@ static hipError_t launch_general_t(const FluidBuffers& b, const StepParams& p, i
     using T = typename Store<S>::T;
     hipLaunchKernelGGL((fluid_general<ARITH, COLL, S>), dim3(general_blocks), dim3(256), 0, s, (const T*)b.fin,
                        (T*)b.fout, b.solid_prev, b.solid_cur, b.wall, b.general_list, b.general_count,
-                       b.partials, b.density, b.velocity, b.body, p);
+                       b.partials, b.body, p);
     return hipGetLastError();
 }
 

@@ -23,8 +23,6 @@ struct FluidBuffers {
     double* block_out;
     double* last_load;
     double* history;
-    float* density;
-    float4* velocity;
     uint32_t* activation;   // [count, max restriction bits] of this step's fast tiles
     const double* body;     // body state (position first): torque reference point
 };
