@@ -110,6 +110,7 @@ struct bf_context {
     float* density = nullptr;
     float4* velocity = nullptr;
     float* staging = nullptr;             // host-layout FP32 buffer for population transfers
+    HostPipe pipe;                        // pinned slots of large host copies
     // geometry
     int source = BF_GEOMETRY_STATIC;
     bool static_prev_differs = false;
@@ -758,6 +759,18 @@ FluidBuffers fluid_buffers(const bf_context* c, int64_t s) {
     return b;
 }
 
+// The last `want` records (`width` doubles each) of a step-indexed history
+// ring, oldest first; at most two copies, of those records alone.
+hipError_t read_ring(bf_context* c, double* out, const double* ring, uint64_t width, uint64_t want) {
+    if (want == 0) return hipSuccess;
+    const uint64_t first = ((uint64_t)c->step - want + 1) % HISTORY_CAPACITY;
+    const uint64_t head = std::min<uint64_t>(want, HISTORY_CAPACITY - first);
+    double* r = const_cast<double*>(ring);
+    const HostCopy copies[2] = {{out, r + width * first, 8 * width * head},
+                                {out + width * head, r, 8 * width * (want - head)}};
+    return copy_to_host(c->pipe, c->device, copies, want > head ? 2 : 1, c->sb);
+}
+
 bf_status check_host_array(bf_context* c, const void* p, const char* name) {
     if (!p) return fail(c, BF_ERROR_INVALID_ARGUMENT, std::string(name) + " is NULL");
     return BF_OK;
@@ -1042,6 +1055,7 @@ void bf_destroy(bf_context* c) {
         if (c->adj.ev_tan[i]) (void)hipEventDestroy(c->adj.ev_tan[i]);
         if (c->adj.ev_used[i]) (void)hipEventDestroy(c->adj.ev_used[i]);
     }
+    c->pipe.release();
     c->mesh_alloc.release();
     c->static_alloc.release();
     c->ledger_alloc.release();
@@ -1170,7 +1184,7 @@ bf_status bf_write_populations(bf_context* c, const float* host, uint64_t count)
     // through the staging buffer: the device layout differs from the host's
     // direction-major one for every storage
     if (bf_status st = ensure_staging(c)) return st;
-    hipError_t e = hipMemcpyAsync(c->staging, host, count * 4, hipMemcpyHostToDevice, c->sb);
+    hipError_t e = copy_to_device(c->pipe, c->device, c->staging, host, count * 4, c->sb);
     if (e == hipSuccess)
         e = launch_convert_populations((int)c->cfg.storage, true, c->staging, c->f[c->cur], count, c->g, c->sb);
     if (e == hipSuccess) e = hipStreamSynchronize(c->sb);
@@ -1184,8 +1198,7 @@ bf_status bf_read_populations(bf_context* c, float* host, uint64_t count) {
     if (count != 19ull * c->g.n) return fail(c, BF_ERROR_INVALID_ARGUMENT, "population count must be 19 * N");
     if (bf_status st = ensure_staging(c)) return st;
     hipError_t e = launch_convert_populations((int)c->cfg.storage, false, c->f[c->cur], c->staging, count, c->g, c->sb);
-    if (e == hipSuccess) e = hipMemcpyAsync(host, c->staging, count * 4, hipMemcpyDeviceToHost, c->sb);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->sb);
+    if (e == hipSuccess) e = copy_to_host(c->pipe, c->device, host, c->staging, count * 4, c->sb);
     if (e != hipSuccess) return hip_fail(c, e, "read populations");
     return BF_OK;
 }
@@ -1202,7 +1215,7 @@ bf_status bf_write_population_storage(bf_context* c, const void* host, uint64_t 
     if (bytes != stored_bytes(c))
         return fail(c, BF_ERROR_INVALID_ARGUMENT, "population storage size must be 19 * N * element size");
     if (bf_status st = ensure_staging(c)) return st;
-    hipError_t e = hipMemcpyAsync(c->staging, host, bytes, hipMemcpyHostToDevice, c->sb);
+    hipError_t e = copy_to_device(c->pipe, c->device, c->staging, host, bytes, c->sb);
     if (e == hipSuccess)
         e = launch_permute_populations((int)c->cfg.storage, true, c->staging, c->f[c->cur], 19ull * c->g.n, c->g,
                                        c->sb);
@@ -1219,8 +1232,7 @@ bf_status bf_read_population_storage(bf_context* c, void* host, uint64_t bytes) 
     if (bf_status st = ensure_staging(c)) return st;
     hipError_t e = launch_permute_populations((int)c->cfg.storage, false, c->f[c->cur], c->staging, 19ull * c->g.n,
                                               c->g, c->sb);
-    if (e == hipSuccess) e = hipMemcpyAsync(host, c->staging, bytes, hipMemcpyDeviceToHost, c->sb);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->sb);
+    if (e == hipSuccess) e = copy_to_host(c->pipe, c->device, host, c->staging, bytes, c->sb);
     if (e != hipSuccess) return hip_fail(c, e, "read population storage");
     return BF_OK;
 }
@@ -1231,9 +1243,8 @@ bf_status bf_read_fields(bf_context* c, float* density, float* velocity3) {
         return BF_ERROR_INVALID_ARGUMENT;
     float* dv = (float*)c->velocity;   // 16 B per cell; holds 3 floats per cell here
     hipError_t e = launch_extract_fields((int)c->cfg.storage, c->f[c->cur], c->density, dv, c->g, c->sb);
-    if (e == hipSuccess) e = hipMemcpyAsync(density, c->density, 4ull * c->g.n, hipMemcpyDeviceToHost, c->sb);
-    if (e == hipSuccess) e = hipMemcpyAsync(velocity3, dv, 12ull * c->g.n, hipMemcpyDeviceToHost, c->sb);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->sb);
+    const HostCopy copies[2] = {{density, c->density, 4ull * c->g.n}, {velocity3, dv, 12ull * c->g.n}};
+    if (e == hipSuccess) e = copy_to_host(c->pipe, c->device, copies, 2, c->sb);
     if (e != hipSuccess) return hip_fail(c, e, "read fields");
     return BF_OK;
 }
@@ -1246,9 +1257,9 @@ bf_status bf_set_geometry(bf_context* c, const uint8_t* mask_prev, const uint8_t
     c->source = BF_GEOMETRY_STATIC;
     c->static_prev_differs = mask_prev && std::memcmp(mask_prev, mask_cur, n) != 0;
     hipStream_t s = c->sb;
-    hipError_t e = hipMemcpyAsync(c->mask[0], mask_cur, n, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess && c->static_prev_differs) e = hipMemcpyAsync(c->mask[1], mask_prev, n, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(c->wall[0], wall4, 16 * n, hipMemcpyHostToDevice, s);
+    hipError_t e = copy_to_device(c->pipe, c->device, c->mask[0], mask_cur, n, s);
+    if (e == hipSuccess && c->static_prev_differs) e = copy_to_device(c->pipe, c->device, c->mask[1], mask_prev, n, s);
+    if (e == hipSuccess) e = copy_to_device(c->pipe, c->device, c->wall[0], wall4, 16 * n, s);
     int periodic[3];
     for (int a = 0; a < 3; ++a) periodic[a] = periodic_axis(c->cfg, a) ? 1 : 0;
     if (e == hipSuccess) e = launch_mark_tiles(c->mask[0], c->dyn[0], c->g, periodic, true, s);
@@ -1263,10 +1274,11 @@ bf_status bf_read_geometry(bf_context* c, uint8_t* mask, float* wall4) {
     BF_ENTER(c);
     const StepGeometry sg = geometry_of(c, c->step);
     const size_t n = c->g.n;
-    hipError_t e = hipSuccess;
-    if (mask) e = hipMemcpyAsync(mask, sg.mask_cur, n, hipMemcpyDeviceToHost, c->sb);
-    if (e == hipSuccess && wall4) e = hipMemcpyAsync(wall4, sg.wall, 16 * n, hipMemcpyDeviceToHost, c->sb);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->sb);
+    HostCopy copies[2];
+    int count = 0;
+    if (mask) copies[count++] = {mask, const_cast<uint8_t*>(sg.mask_cur), n};
+    if (wall4) copies[count++] = {wall4, const_cast<float4*>(sg.wall), 16 * n};
+    hipError_t e = count ? copy_to_host(c->pipe, c->device, copies, count, c->sb) : hipSuccess;
     if (e != hipSuccess) return hip_fail(c, e, "read geometry");
     return BF_OK;
 }
@@ -2090,7 +2102,7 @@ bf_status bf_synchronize(bf_context* c) {
         // a non-finite population is reported once, with the first step
         // that stored one
         unsigned long long h[2];
-        e = hipMemcpy(h, c->health, sizeof h, hipMemcpyDeviceToHost);
+        e = copy_to_host(c->pipe, c->device, h, c->health, sizeof h, c->sb);
         if (e != hipSuccess) return hip_fail(c, e, "read fluid health");
         if (h[0] != 0ull) {
             c->health_reported = true;
@@ -2183,7 +2195,7 @@ bf_status bf_body_get(bf_context* c, bf_body_state* state) {
     BF_ENTER(c);
     if (!state) return BF_ERROR_INVALID_ARGUMENT;
     double v[16];
-    hipError_t e = hipMemcpy(v, c->body, sizeof v, hipMemcpyDeviceToHost);
+    hipError_t e = copy_to_host(c->pipe, c->device, v, c->body, sizeof v, c->sb);
     if (e != hipSuccess) return hip_fail(c, e, "body read");
     for (int i = 0; i < 3; ++i) {
         state->position[i] = v[i];
@@ -2199,12 +2211,11 @@ bf_status bf_read_body_history(bf_context* c, bf_body_state* out, uint32_t max_r
     if (!out || !records) return BF_ERROR_INVALID_ARGUMENT;
     const uint64_t avail = std::min<uint64_t>(c->body_history_count, HISTORY_CAPACITY);
     const uint64_t want = std::min<uint64_t>(avail, max_records);
-    std::vector<double> all(16ull * HISTORY_CAPACITY);
-    hipError_t e = hipMemcpy(all.data(), c->body_history, 128ull * HISTORY_CAPACITY, hipMemcpyDeviceToHost);
+    std::vector<double> all(16ull * want);
+    hipError_t e = read_ring(c, all.data(), c->body_history, 16, want);
     if (e != hipSuccess) return hip_fail(c, e, "read body history");
     for (uint64_t i = 0; i < want; ++i) {
-        const uint64_t step = (uint64_t)c->step - want + 1 + i;
-        const double* v = all.data() + 16 * (step % HISTORY_CAPACITY);
+        const double* v = all.data() + 16 * i;
         for (int k = 0; k < 3; ++k) {
             out[i].position[k] = v[k];
             out[i].linear_velocity[k] = v[7 + k];
@@ -2772,8 +2783,7 @@ bf_status bf_adjoint_read_sensitivity(bf_context* c, float* out, uint64_t count)
     if (bf_status st = ensure_staging(c)) return st;
     hipError_t e = launch_convert_populations(STORE_FP32, false, c->adj.lam[c->adj.lam_cur], c->staging, count, c->g,
                                               c->sb);
-    if (e == hipSuccess) e = hipMemcpyAsync(out, c->staging, 4 * count, hipMemcpyDeviceToHost, c->sb);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->sb);
+    if (e == hipSuccess) e = copy_to_host(c->pipe, c->device, out, c->staging, 4 * count, c->sb);
     if (e != hipSuccess) return hip_fail(c, e, "read sensitivity");
     return BF_OK;
 }
@@ -2781,8 +2791,7 @@ bf_status bf_adjoint_read_sensitivity(bf_context* c, float* out, uint64_t count)
 bf_status bf_read_loads(bf_context* c, double out[8]) {
     BF_ENTER(c);
     if (!out) return BF_ERROR_INVALID_ARGUMENT;
-    hipError_t e = hipMemcpyAsync(out, c->last_load, 64, hipMemcpyDeviceToHost, c->sb);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->sb);
+    hipError_t e = copy_to_host(c->pipe, c->device, out, c->last_load, 64, c->sb);
     if (e != hipSuccess) return hip_fail(c, e, "read loads");
     return BF_OK;
 }
@@ -2792,14 +2801,8 @@ bf_status bf_read_load_history(bf_context* c, double* out, uint32_t max_records,
     if (!out || !records) return BF_ERROR_INVALID_ARGUMENT;
     const uint64_t avail = std::min<uint64_t>(c->history_count, HISTORY_CAPACITY);
     const uint64_t want = std::min<uint64_t>(avail, max_records);
-    std::vector<double> all(8ull * HISTORY_CAPACITY);
-    hipError_t e = hipMemcpyAsync(all.data(), c->history, 64ull * HISTORY_CAPACITY, hipMemcpyDeviceToHost, c->sb);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->sb);
+    hipError_t e = read_ring(c, out, c->history, 8, want);
     if (e != hipSuccess) return hip_fail(c, e, "read load history");
-    for (uint64_t i = 0; i < want; ++i) {
-        const uint64_t step = (uint64_t)c->step - want + 1 + i;
-        std::memcpy(out + 8 * i, all.data() + 8 * (step % HISTORY_CAPACITY), 64);
-    }
     *records = (uint32_t)want;
     return BF_OK;
 }

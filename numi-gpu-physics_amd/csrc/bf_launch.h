@@ -9,6 +9,25 @@
 
 namespace bf {
 
+// Pinned slots of a context's host copies (bf_transfer.hip).  The copies
+// follow the work already on stream s and return when the data has arrived.
+struct HostPipe {
+    static constexpr int SLOTS = 8;
+    void* slot[SLOTS] = {};
+    hipEvent_t done[SLOTS] = {};
+    int slots = 0;                      // made so far
+    bool exhausted = false;             // no more pinned memory
+    void release();
+};
+struct HostCopy {
+    void* host;
+    void* dev;
+    size_t bytes;
+};
+hipError_t copy_to_host(HostPipe& p, int device, const HostCopy* copies, int n, hipStream_t s);
+hipError_t copy_to_host(HostPipe& p, int device, void* host, const void* dev, size_t bytes, hipStream_t s);
+hipError_t copy_to_device(HostPipe& p, int device, void* dev, const void* host, size_t bytes, hipStream_t s);
+
 struct FluidBuffers {
     const void* fin;
     void* fout;
