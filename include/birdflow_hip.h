@@ -407,12 +407,13 @@ bf_status bf_read_load_history(bf_context* ctx, double* out, uint32_t max_record
 bf_status bf_link_census(bf_context* ctx, uint64_t counts[21]);
 
 /* ---- measurement ---- */
-/* enabled = 1: every step records HIP events around the fast-fluid launch on
- * its stream; 2: also around the general-fluid launch and the next step's
- * geometry (each event pair adds latency to the step); 0: off. */
+/* enabled = 1: every step records HIP events around its fluid launch on its
+ * stream; 2: the wall tiles and the wall-free tiles go in launches of their own
+ * with events around each, and around the next step's geometry (each event
+ * pair and launch adds latency to the step); 0: off. */
 bf_status bf_set_profiling(bf_context* ctx, int enabled);
-/* {geometry ms, fast fluid ms, general fluid ms (0 unless level 2), steps
- * profiled, tiles on the general path in the last step, total tiles (64 x 4
+/* {geometry ms, fluid ms (level 2: its wall-free tiles), wall-tile ms (0
+ * unless level 2), steps profiled, tiles on the general path in the last step, total tiles (64 x 4
  * cells)} summed over the steps profiled since the last reset; resets the
  * counters. */
 bf_status bf_read_profile(bf_context* ctx, double out[6]);

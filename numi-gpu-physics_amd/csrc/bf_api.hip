@@ -6,17 +6,17 @@
 // mask, fluid step current -> next lattice with the previous / current
 // masks, load reduction, swap.
 //
-// Two HIP streams form a software pipeline, per step s:
-//   stream A  fluid_fast(s)                              (HBM-bound, wall-free tiles)
-//   stream B  geometry(s+1) + tile list(s+1)  [overlaps fast(s)],
-//             then fluid_general(s)                       [after fast(s)]
-//             and the load reduction of step s            [overlaps fast(s+1)]
-// fast(s) waits for event R[(s-1)&1] (general(s-1) done, which follows
-// geometry(s) on B); general(s) waits for F[s&1] (fast(s) done).  Geometry of
-// step s+1 only writes buffers that steps s-1 and s-2 last read: masks and
-// solid-proximity tile flags rotate over 3 buffers, the wall field and the
-// general-tile list over 2, the touched-tile flags over 4.  Every entry point
-// other than bf_step drains both streams first.
+// With moving geometry two HIP streams form a software pipeline, per step s:
+//   stream A  fluid_step(s): wall tiles and wall-free tiles in one launch
+//   stream B  geometry(s+1) + tile list(s+1)  [overlaps fluid_step(s)],
+//             then the load reduction of step s    [overlaps fluid_step(s+1)]
+// fluid_step(s) waits for L[s] (its tile list, stream B); the reduction of
+// step s for F[s] (fluid_step(s) done).  Geometry of step s+1 only writes
+// buffers that steps s-1 and s-2 last read: masks and solid-proximity tile
+// flags rotate over 3 buffers, the wall field and the wall-tile list over 2,
+// the touched-tile flags and the load partials over 4.  With static geometry
+// the list is built once and everything runs on stream A, the reductions in
+// batches.  Every entry point other than bf_step drains both streams first.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -83,11 +83,11 @@ inline int par2(int64_t s) { return (int)(s & 1); }
 struct bf_context {
     bf_config cfg{};
     Grid g{};
-    hipStream_t sa = nullptr;             // fast fluid
-    hipStream_t sb = nullptr;             // general fluid, reductions, geometry, everything else
+    hipStream_t sa = nullptr;             // fluid
+    hipStream_t sb = nullptr;             // reductions, geometry, everything else
     hipEvent_t ev_fast[2] = {nullptr, nullptr};
     hipEvent_t ev_ready[2] = {nullptr, nullptr};
-    hipEvent_t ev_general[2] = {nullptr, nullptr};   // general(s) done (stream A)
+    hipEvent_t ev_general[2] = {nullptr, nullptr};   // wall tiles of step s done (stream A), coupled free flight
     int device = 0;
     DeviceAlloc alloc;
     DeviceAlloc mesh_alloc;
@@ -101,7 +101,15 @@ struct bf_context {
     uint8_t* no_tiles = nullptr;          // all-zero tile flags
     uint32_t* general_list[2] = {nullptr, nullptr};
     uint32_t* geo_list = nullptr;
-    uint32_t* counters = nullptr;         // [0],[1] general-list counts by step parity, [2] geometry tile list
+    // [0],[1] wall-tile list counts by list slot, [2] geometry tile list,
+    // [8],[9] limiter activations of recomputed steps, [16 + 2 k] those of load
+    // slot k
+    uint32_t* counters = nullptr;
+    // static geometry: the wall-tile list in slot 1 holds the current mask's
+    // tiles (slot 0 the first step's, when its previous mask differs)
+    bool static_list_ready = false;
+    uint32_t static_tiles = 0;            // and how many they are
+    int last_list = 0;                    // list slot of the last step
     double* partials = nullptr;
     double* block_out = nullptr;
     double* last_load = nullptr;
@@ -279,7 +287,8 @@ struct bf_context {
     int profiling_level = 0;              // 1: fast kernel only; 2: also general and geometry
     std::vector<hipEvent_t> events;
     uint32_t profiled = 0;
-    int general_blocks = 1024;
+    uint32_t wall_blocks = 512;           // workgroups of a step that walk the wall-tile list
+    int general_blocks = 1024;            // of the adjoint's wall-tile passes
     // replayed part masks (finite-difference checks with the link set fixed)
     DeviceAlloc frozen_alloc;
     uint8_t* frozen = nullptr;
@@ -291,7 +300,6 @@ struct bf_context {
     uint32_t raster_batch = 0;            // triangles per raster wave; 0: from the mesh size
     int fast_priority = 0, general_priority = 0;   // s_setprio of the fluid kernels' wavefronts
     bool pair_cells = true;                        // 2-byte storage: fast tiles two cells per lane
-    bool geometry_after_general = true;            // stream B starts the next geometry after general(s)
     uint32_t raster_batch_cap = 32;                // largest automatic raster batch
     uint32_t compute_units = 1;
     uint32_t tile_pass_blocks = 512;
@@ -727,18 +735,38 @@ bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
     return BF_OK;
 }
 
-// List of the tiles that take the general path in step s (stream B).
-bf_status enqueue_tile_list(bf_context* c, int64_t s) {
+// List of the tiles that take the general path in step s, into list slot
+// `slot`, on stream st.
+bf_status enqueue_tile_list(bf_context* c, int64_t s, int slot, hipStream_t st) {
     const StepGeometry sg = geometry_of(c, s);
-    hipError_t e = launch_fill_u32(&c->counters[par2(s)], 0u, 1u, c->sb);
+    hipError_t e = launch_fill_u32(&c->counters[slot], 0u, 1u, st);
     if (e == hipSuccess)
-        e = launch_build_general_list(sg.dyn_prev, sg.dyn_cur, c->g.tiles, c->general_list[par2(s)],
-                                      &c->counters[par2(s)], c->sb);
+        e = launch_build_general_list(sg.dyn_prev, sg.dyn_cur, c->g.tiles, c->general_list[slot], &c->counters[slot],
+                                      st);
     if (e != hipSuccess) return hip_fail(c, e, "tile list launch");
     return BF_OK;
 }
 
-FluidBuffers fluid_buffers(const bf_context* c, int64_t s) {
+// Workgroups for at most `tiles` wall tiles: a multiple of 8, so that the
+// blocks after them keep their place in the XCD order.
+uint32_t wall_blocks_for(const bf_context* c, uint32_t tiles) {
+    return tiles == 0 ? 0u : std::min(c->wall_blocks, (tiles + 7u) & ~7u);
+}
+
+LoadBuffers load_buffers(const bf_context* c, const FluidBuffers& fb) {
+    LoadBuffers b{};
+    b.partials = c->partials;
+    b.dyn_prev = fb.dyn_prev;
+    b.dyn_cur = fb.dyn_cur;
+    b.block_out = c->block_out;
+    b.activation = &c->counters[16];
+    b.last_load = c->last_load;
+    b.history = c->history;
+    b.history_capacity = HISTORY_CAPACITY;
+    return b;
+}
+
+FluidBuffers fluid_buffers(const bf_context* c, int64_t s, int list_slot) {
     const StepGeometry sg = geometry_of(c, s);
     FluidBuffers b{};
     b.fin = c->f[c->cur];
@@ -748,13 +776,11 @@ FluidBuffers fluid_buffers(const bf_context* c, int64_t s) {
     b.wall = sg.wall;
     b.dyn_cur = sg.dyn_cur;
     b.dyn_prev = sg.dyn_prev;
-    b.general_list = c->general_list[par2(s)];
-    b.general_count = &c->counters[par2(s)];
-    b.partials = c->partials + 8ull * c->g.tiles * (uint64_t)par2(s);
-    b.block_out = c->block_out;
-    b.last_load = c->last_load;
-    b.history = c->history;
-    b.activation = &c->counters[4 + 2 * par2(s)];
+    const uint64_t load_slot = (uint64_t)s % LOAD_SLOTS;
+    b.general_list = c->general_list[list_slot];
+    b.general_count = &c->counters[list_slot];
+    b.partials = c->partials + 8ull * c->g.tiles * load_slot;
+    b.activation = &c->counters[16 + 2 * load_slot];
     b.body = c->body;
     return b;
 }
@@ -911,18 +937,14 @@ bf_status bf_create(const bf_config* cfg, bf_context** out) {
     c->tile_pass_blocks = (uint32_t)std::max(1, prop.multiProcessorCount);
     // tuning overrides (workgroup counts)
     if (const char* v = std::getenv("BIRDFLOW_RASTER_BLOCKS")) c->raster_blocks = (uint32_t)std::max(1, std::atoi(v));
-    // Scheduling of the next step's geometry against the fluid kernels (sweeps
-    // on the 512x256x256 bird, 40k triangles):
-    //  * FP32: the fast kernel runs at issue priority 2 over the raster, which
-    //    starts after the general kernel and still finishes within the fast
-    //    kernel (1.03 -> 1.01 ms per step);
-    //  * FP16 / BF16: the fast kernel is too short for a deprioritized raster;
-    //    the raster starts at once, beside the general kernel (priority 3),
-    //    in batches of 16 triangles (0.664 -> 0.640 ms per step).
+    // Issue priority of the wall-free tiles' wavefronts: none.  Raised over the
+    // next step's geometry it gained 0.5 % on the 512x256x256 bird (FP32,
+    // 984 -> 982 us) and starved that geometry where it is the longer of the
+    // two (160x160x128 wing 137 -> 176 us per step, 384x192x192 bird with exact
+    // roots 561 -> 608).
     const bool fp32 = cfg->storage == BF_STORAGE_FP32;
-    c->fast_priority = fp32 ? 2 : 0;
+    c->fast_priority = 0;
     c->general_priority = 3;
-    c->geometry_after_general = fp32;
     c->raster_batch_cap = fp32 ? 32u : 16u;
     if (const char* v = std::getenv("BIRDFLOW_FAST_PRIORITY")) c->fast_priority = std::min(3, std::max(0, std::atoi(v)));
     // FP16 / BF16: fast tiles two cells per lane (0 selects one cell per lane)
@@ -932,7 +954,7 @@ bf_status bf_create(const bf_config* cfg, bf_context** out) {
     if (const char* v = std::getenv("BIRDFLOW_RAY_STATIC")) c->ray_static_enabled = std::atoi(v) != 0;
     if (const char* v = std::getenv("BIRDFLOW_GENERAL_PRIORITY"))
         c->general_priority = std::min(3, std::max(0, std::atoi(v)));
-    if (const char* v = std::getenv("BIRDFLOW_GEOMETRY_AFTER_GENERAL")) c->geometry_after_general = std::atoi(v) != 0;
+    if (const char* v = std::getenv("BIRDFLOW_WALL_BLOCKS")) c->wall_blocks = (uint32_t)std::max(8, std::atoi(v) & ~7);
     if (const char* v = std::getenv("BIRDFLOW_RASTER_BATCH"))
         c->raster_batch = (uint32_t)std::min(64, std::max(1, std::atoi(v)));
     if (const char* v = std::getenv("BIRDFLOW_RAY_BLOCKS_PER_CU"))
@@ -945,7 +967,7 @@ bf_status bf_create(const bf_config* cfg, bf_context** out) {
     // Working-set plan (MetalBackend.validateAllocationPlan, :77-106).
     const uint64_t n = g.n;
     const uint64_t pop_bytes = 19ull * n * c->pop_elem;
-    const uint64_t plan = 2 * pop_bytes + 3 * n + 32 * n + 3ull * g.tiles + 4ull * g.tiles + 128ull * g.tiles +
+    const uint64_t plan = 2 * pop_bytes + 3 * n + 32 * n + 3ull * g.tiles + 4ull * g.tiles + 64ull * LOAD_SLOTS * g.tiles +
                           64ull * HISTORY_CAPACITY + 128ull * HISTORY_CAPACITY + 4 * n + 16 * n;
     size_t free_b = 0, total_b = 0;
     (void)hipMemGetInfo(&free_b, &total_b);
@@ -989,9 +1011,9 @@ bf_status bf_create(const bf_config* cfg, bf_context** out) {
     c->health = (unsigned long long*)A.take(e, 2 * sizeof(unsigned long long));
     c->popmin = (PopulationMinimum*)A.take(e, (POPULATION_MINIMUM_BLOCKS + 1) * sizeof(PopulationMinimum));
     c->wing_reaction = (float*)A.take(e, 32 * sizeof(float));
-    c->counters = (uint32_t*)A.take(e, 64);
-    c->partials = (double*)A.take(e, 128ull * g.tiles);   // two steps' per-tile load partials
-    c->block_out = (double*)A.take(e, 64ull * ((g.tiles + 1023) / 1024 + 1));
+    c->counters = (uint32_t*)A.take(e, 128);
+    c->partials = (double*)A.take(e, 64ull * LOAD_SLOTS * g.tiles);   // per-tile load partials by load slot
+    c->block_out = (double*)A.take(e, 64ull * LOAD_SLOTS * ((g.tiles + 1023) / 1024));
     c->last_load = (double*)A.take(e, 64);
     c->history = (double*)A.take(e, 64ull * HISTORY_CAPACITY);
     c->census = (unsigned long long*)A.take(e, 8 * 24);
@@ -1011,9 +1033,9 @@ bf_status bf_create(const bf_config* cfg, bf_context** out) {
     for (int i = 0; i < 3 && e == hipSuccess; ++i) e = launch_fill_u8(c->dyn[i], 0, g.tiles, s);
     for (int i = 0; i < 4 && e == hipSuccess; ++i) e = launch_fill_u8(c->tflags[i], 0, g.tiles, s);
     if (e == hipSuccess) e = launch_fill_u8(c->no_tiles, 0, g.tiles, s);
-    if (e == hipSuccess) e = launch_fill_u32(c->counters, 0u, 16u, s);
+    if (e == hipSuccess) e = launch_fill_u32(c->counters, 0u, 32u, s);
     if (e == hipSuccess) e = launch_fill_u8((uint8_t*)c->last_load, 0, 64, s);
-    if (e == hipSuccess) e = launch_fill_u8((uint8_t*)c->partials, 0, (uint32_t)(128ull * g.tiles), s);
+    if (e == hipSuccess) e = launch_fill_u32((uint32_t*)c->partials, 0u, (uint32_t)(16ull * LOAD_SLOTS * g.tiles), s);
     if (e == hipSuccess) e = launch_fill_u8((uint8_t*)c->wing_momentum, 0, 16 * sizeof(float), s);
     if (e == hipSuccess) e = launch_fill_u8((uint8_t*)c->health, 0, 8, s);
     if (e == hipSuccess) e = launch_fill_u8((uint8_t*)c->health + 8, 0xFF, 8, s);
@@ -1264,8 +1286,14 @@ bf_status bf_set_geometry(bf_context* c, const uint8_t* mask_prev, const uint8_t
     for (int a = 0; a < 3; ++a) periodic[a] = periodic_axis(c->cfg, a) ? 1 : 0;
     if (e == hipSuccess) e = launch_mark_tiles(c->mask[0], c->dyn[0], c->g, periodic, true, s);
     if (e == hipSuccess && c->static_prev_differs) e = launch_mark_tiles(c->mask[1], c->dyn[1], c->g, periodic, true, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    // the wall-tile list of every step but a first one with another previous
+    // mask, and its length
+    if (e == hipSuccess) e = launch_fill_u32(&c->counters[1], 0u, 1u, s);
+    if (e == hipSuccess)
+        e = launch_build_general_list(c->dyn[0], c->dyn[0], c->g.tiles, c->general_list[1], &c->counters[1], s);
+    if (e == hipSuccess) e = copy_to_host(c->pipe, c->device, &c->static_tiles, &c->counters[1], 4, s);
     if (e != hipSuccess) return hip_fail(c, e, "set geometry");
+    c->static_list_ready = true;
     c->geometry_ready = c->step;
     return BF_OK;
 }
@@ -1967,6 +1995,84 @@ bf_status bf_ledger_step_sources_noalloc(bf_context* c, double sums[16], uint64_
     return ledger_step_sources_into(c, b, sums, counts);
 }
 
+// The profiling events of the next step (nullptr when it is not profiled).
+static bf_status profile_events(bf_context* c, hipEvent_t*& pe) {
+    pe = nullptr;
+    if (!c->profiling || c->profiled >= PROFILE_CAPACITY) return BF_OK;
+    while (c->events.size() < (size_t)(c->profiled + 1) * PROFILE_EVENTS) {
+        hipEvent_t ev;
+        if (hipEventCreate(&ev) != hipSuccess) return fail(c, BF_ERROR_ALLOCATION_FAILED, "profile event");
+        c->events.push_back(ev);
+    }
+    pe = &c->events[(size_t)c->profiled * PROFILE_EVENTS];
+    return BF_OK;
+}
+
+static StepParams step_params(const bf_context* c, int64_t s) {
+    StepParams p = make_step_params(c);
+    // the link table of step s; geometry(s + 1) fills the other slot meanwhile
+    p.links = (c->cfg.wall_rule == BF_WALL_INTERPOLATED_RAY ? c->ray_links : c->wing_links)[par2(s)];
+    p.health = c->health;
+    p.step_index = (unsigned long long)s;
+    return p;
+}
+
+// Steps with static geometry and a fixed body: nothing to build between the
+// steps, so one fluid launch per step on stream A, back to back, and a load
+// reduction per LOAD_SLOTS steps (64^3 periodic TRT: 46 -> 10 us per step; the
+// list rebuilt, three launches and four event records and waits per step before).
+static bf_status step_static(bf_context* c, uint32_t steps) {
+    const int storage = (int)c->cfg.storage, coll = (int)c->cfg.collision, arith = arithmetic_of(c->cfg);
+    // after what earlier calls enqueued on stream B (a snapshot of f[cur], say)
+    hipError_t e = hipEventRecord(c->ev_ready[0], c->sb);
+    if (e == hipSuccess) e = hipStreamWaitEvent(c->sa, c->ev_ready[0], 0);
+    if (e != hipSuccess) return hip_fail(c, e, "event wait");
+    uint32_t waiting = 0;                // steps whose loads wait for their reduction
+    for (uint32_t i = 0; i < steps; ++i) {
+        const int64_t s = c->step + 1;
+        const bool differs = c->static_prev_differs;   // the first step after bf_set_geometry with another mask
+        const int slot = differs ? 0 : 1;
+        if (differs || !c->static_list_ready) {
+            if (bf_status r = enqueue_tile_list(c, s, slot, c->sa)) return r;
+            if (!differs) c->static_list_ready = true;
+        }
+        hipEvent_t* pe = nullptr;
+        if (bf_status r = profile_events(c, pe)) return r;
+        const bool split = pe && c->profiling_level >= 2;
+        const FluidBuffers fb = fluid_buffers(c, s, slot);
+        const StepParams p = step_params(c, s);
+        const uint32_t wall_blocks = wall_blocks_for(c, differs ? c->g.tiles : c->static_tiles);
+        c->ledger_prev = fb.solid_prev;
+        c->last_list = slot;
+        c->static_prev_differs = false;
+        if (split) {
+            for (int k = 2; k < 5 && e == hipSuccess; ++k) e = hipEventRecord(pe[k], c->sa);   // no geometry: 2 -> 3
+            if (e == hipSuccess) e = launch_fluid_step(arith, storage, coll, fb, p, STEP_WALL_TILES, wall_blocks, c->sa);
+            if (e == hipSuccess) e = hipEventRecord(pe[5], c->sa);
+        }
+        if (pe && e == hipSuccess) e = hipEventRecord(pe[0], c->sa);
+        if (e == hipSuccess)
+            e = launch_fluid_step(arith, storage, coll, fb, p, split ? STEP_FAST_TILES : STEP_ALL, wall_blocks, c->sa);
+        if (pe && e == hipSuccess) e = hipEventRecord(pe[1], c->sa);
+        ++waiting;
+        if (e == hipSuccess && (waiting == LOAD_SLOTS || i + 1 == steps || differs)) {
+            e = launch_load_reduction(load_buffers(c, fb), p, (uint64_t)s - waiting + 1, waiting, c->sa);
+            waiting = 0;
+        }
+        if (e != hipSuccess) return hip_fail(c, e, "fluid step launch");
+        c->step = s;
+        c->cur = 1 - c->cur;
+        ++c->history_count;
+        c->geometry_ready = s + 1;
+        if (pe) ++c->profiled;
+    }
+    e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(c, e, "step");
+    c->ledger_epoch = c->f_writes;
+    c->ledger_step = c->step;
+    return BF_OK;
+}
+
 bf_status bf_step(bf_context* c, uint32_t steps) {
     if (!c) return BF_ERROR_INVALID_ARGUMENT;
     if (c->invalidated) return BF_ERROR_STATE_INVALIDATED;
@@ -1978,93 +2084,83 @@ bf_status bf_step(bf_context* c, uint32_t steps) {
         return fail(c, BF_ERROR_INVALID_ARGUMENT, "the exact-root wall rule needs an uploaded mesh");
     const int storage = (int)c->cfg.storage, coll = (int)c->cfg.collision, arith = arithmetic_of(c->cfg);
     hipError_t e = hipSuccess;
+    if (c->source == BF_GEOMETRY_STATIC && !c->free_flight) return step_static(c, steps);
+    const uint32_t wall_blocks = wall_blocks_for(c, c->g.tiles);
     // Prologue: geometry (unless already built) and tile list of the first
-    // step of this call; event R of the previous step then releases fast(s).
+    // step of this call; event L of that step then releases its fluid launch.
     {
         const int64_t s = c->step + 1;
         if (c->source != BF_GEOMETRY_STATIC && c->geometry_ready < s) {
             if (bf_status r = enqueue_geometry(c, s, false, false)) return r;
         }
-        if (bf_status r = enqueue_tile_list(c, s)) return r;
+        c->static_list_ready = false;
+        if (bf_status r = enqueue_tile_list(c, s, par2(s), c->sb)) return r;
         e = hipEventRecord(c->ev_ready[par2(s)], c->sb);
         if (e != hipSuccess) return hip_fail(c, e, "event record");
         c->geometry_ready = s;
     }
     for (uint32_t i = 0; i < steps; ++i) {
         const int64_t s = c->step + 1;
-        const bool prof = c->profiling && c->profiled < PROFILE_CAPACITY;
-        const bool prof_all = prof && c->profiling_level >= 2;
         hipEvent_t* pe = nullptr;
-        if (prof) {
-            while (c->events.size() < (size_t)(c->profiled + 1) * PROFILE_EVENTS) {
-                hipEvent_t ev;
-                if (hipEventCreate(&ev) != hipSuccess) return fail(c, BF_ERROR_ALLOCATION_FAILED, "profile event");
-                c->events.push_back(ev);
-            }
-            pe = &c->events[(size_t)c->profiled * PROFILE_EVENTS];
-        }
-        StepParams p = make_step_params(c);
-        // the link table of step s; geometry(s + 1) fills the other slot meanwhile
-        p.links = (c->cfg.wall_rule == BF_WALL_INTERPOLATED_RAY ? c->ray_links : c->wing_links)[par2(s)];
-        p.health = c->health;
-        p.step_index = (unsigned long long)s;
-        const FluidBuffers fb = fluid_buffers(c, s);
+        if (bf_status r = profile_events(c, pe)) return r;
+        const bool split = pe && c->profiling_level >= 2;
+        const FluidBuffers fb = fluid_buffers(c, s, par2(s));
+        const StepParams p = step_params(c, s);
         c->ledger_prev = fb.solid_prev;
+        c->last_list = par2(s);
         if (c->source == BF_GEOMETRY_STATIC) c->static_prev_differs = false;
-        // stream A: the wall tiles of step s, then the wall-free tiles, once
-        // the tile list of step s (event L[s], stream B) is built.  Both read
-        // f_in, which the previous step finished writing on this stream.
+        // Coupled free flight puts the reduction, body update and next
+        // geometry on the critical path.  With TRT the loads come from the
+        // wall tiles alone (the fast tiles add limiter activations only for
+        // the other collisions): the wall tiles then go first, in a launch of
+        // their own, and that chain starts when they end and overlaps the
+        // fast tiles, which read none of the buffers it writes (geometry s+1
+        // writes the dyn flags of s-2, and everything of step s-1 precedes).
+        const bool coupled = c->free_flight && ((c->move_mesh && c->source == BF_GEOMETRY_MESH) ||
+                                                c->source == BF_GEOMETRY_BIRD);
+        const bool early_loads = coupled && c->cfg.collision == BF_COLLISION_TRT;
+        // stream A: the fluid step, once the tile list of step s (event L[s],
+        // stream B) is built; it reads f_in, which the previous step finished
+        // writing on this stream
         e = hipStreamWaitEvent(c->sa, c->ev_ready[par2(s)], 0);
-        if (prof_all && e == hipSuccess) e = hipEventRecord(pe[4], c->sa);
-        if (e == hipSuccess) e = launch_fluid_general(arith, storage, coll, fb, p, c->general_blocks, c->sa);
-        if (prof_all && e == hipSuccess) e = hipEventRecord(pe[5], c->sa);
-        if (e == hipSuccess) e = hipEventRecord(c->ev_general[par2(s)], c->sa);
-        if (prof && e == hipSuccess) e = hipEventRecord(pe[0], c->sa);
-        if (e == hipSuccess) e = launch_fluid_fast(arith, storage, coll, fb, p, c->sa);
-        if (prof && e == hipSuccess) e = hipEventRecord(pe[1], c->sa);
+        if (early_loads || split) {
+            if (split && e == hipSuccess) e = hipEventRecord(pe[4], c->sa);
+            if (e == hipSuccess) e = launch_fluid_step(arith, storage, coll, fb, p, STEP_WALL_TILES, wall_blocks, c->sa);
+            if (split && e == hipSuccess) e = hipEventRecord(pe[5], c->sa);
+            if (early_loads && e == hipSuccess) e = hipEventRecord(c->ev_general[par2(s)], c->sa);
+            if (pe && e == hipSuccess) e = hipEventRecord(pe[0], c->sa);
+            if (e == hipSuccess) e = launch_fluid_step(arith, storage, coll, fb, p, STEP_FAST_TILES, 0, c->sa);
+        } else {
+            if (pe && e == hipSuccess) e = hipEventRecord(pe[0], c->sa);
+            if (e == hipSuccess) e = launch_fluid_step(arith, storage, coll, fb, p, STEP_ALL, wall_blocks, c->sa);
+        }
+        if (pe && e == hipSuccess) e = hipEventRecord(pe[1], c->sa);
         if (e == hipSuccess) e = hipEventRecord(c->ev_fast[par2(s)], c->sa);
         if (e != hipSuccess) return hip_fail(c, e, "fluid step launch");
         // stream B: geometry and tile list of step s+1 while step s streams
         // (they write only buffers that step s-1 last read; this stream
         // waited for step s-1 before its load reduction), then event L[s+1];
-        // then the load reduction of step s (partials double-buffered by
-        // step parity) and the body update.  general(s+1) reads the torque
-        // reference point from the body state, so in free flight L[s+1]
-        // follows the body update; a mesh riding on a free-flying body also
-        // needs the pose after step s, so its geometry follows it too.
-        const bool coupled = c->free_flight && ((c->move_mesh && c->source == BF_GEOMETRY_MESH) ||
-                                                c->source == BF_GEOMETRY_BIRD);
+        // then the load reduction of step s and the body update.  The wall
+        // tiles of step s+1 read the torque reference point from the body
+        // state, so in free flight L[s+1] follows the body update; a mesh
+        // riding on a free-flying body also needs the pose after step s, so
+        // its geometry follows it too.
         auto next_geometry = [&]() -> bf_status {
-            if (prof_all) e = hipEventRecord(pe[2], c->sb);
+            if (split) e = hipEventRecord(pe[2], c->sb);
             if (e == hipSuccess && c->source != BF_GEOMETRY_STATIC) {
                 if (bf_status r = enqueue_geometry(c, s + 1, false, false)) return r;
             }
-            if (bf_status r = enqueue_tile_list(c, s + 1)) return r;
-            if (prof_all) e = hipEventRecord(pe[3], c->sb);
+            if (bf_status r = enqueue_tile_list(c, s + 1, par2(s + 1), c->sb)) return r;
+            if (split) e = hipEventRecord(pe[3], c->sb);
             return e == hipSuccess ? BF_OK : hip_fail(c, e, "geometry launch");
         };
         if (!coupled) {
-            // after general(s): its latency-bound wavefronts would otherwise
-            // share the machine with the raster; the geometry then overlaps
-            // fast(s) only
-            if (c->geometry_after_general) e = hipStreamWaitEvent(c->sb, c->ev_general[par2(s)], 0);
-            if (e != hipSuccess) return hip_fail(c, e, "event wait");
             if (bf_status r = next_geometry()) return r;
         }
         if (!c->free_flight) e = hipEventRecord(c->ev_ready[par2(s + 1)], c->sb);
-        // Coupled free flight puts the reduction, body update and next
-        // geometry on the critical path.  With TRT the loads come from the
-        // wall tiles alone (the fast kernel adds limiter activations only for
-        // the other collisions), so they start when general(s) ends and
-        // overlap fast(s): fast(s) reads none of the buffers they write
-        // (geometry s+1 writes the dyn flags of s-2, which fast(s-1) read and
-        // general(s) followed), and general(s) itself follows fast(s-1).
-        // Uncoupled, the geometry of s+1 may precede general(s) on this
-        // stream, so the reduction keeps waiting for fast(s).
-        const bool early_loads = coupled && c->cfg.collision == BF_COLLISION_TRT;
         if (e == hipSuccess)
             e = hipStreamWaitEvent(c->sb, early_loads ? c->ev_general[par2(s)] : c->ev_fast[par2(s)], 0);
-        if (e == hipSuccess) e = launch_load_reduction(fb, p, (uint32_t)(s % HISTORY_CAPACITY), c->sb);
+        if (e == hipSuccess) e = launch_load_reduction(load_buffers(c, fb), p, (uint64_t)s, 1, c->sb);
         if (e == hipSuccess && c->free_flight)
             e = launch_body_step(c->body, c->last_load, c->body_history, (uint32_t)(s % HISTORY_CAPACITY),
                                  c->safety_metrics, c->safety_event, (uint64_t)s, c->body_params, c->sb,
@@ -2083,7 +2179,7 @@ bf_status bf_step(bf_context* c, uint32_t steps) {
         ++c->history_count;
         if (c->free_flight) ++c->body_history_count;
         c->geometry_ready = s + 1;
-        if (prof) ++c->profiled;
+        if (pe) ++c->profiled;
     }
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(c, e, "step");
@@ -2658,8 +2754,8 @@ bf_status bf_adjoint_gradient(bf_context* c, uint32_t steps, const double* load_
                                                           ray_params(c), c->sb);
                 ps.links = c->ray_links[s & 1];
             }
-            if (e == hipSuccess) e = launch_fluid_fast(arith, storage, coll, fb, ps, c->sb);
-            if (e == hipSuccess) e = launch_fluid_general(arith, storage, coll, fb, ps, c->general_blocks, c->sb);
+            if (e == hipSuccess)
+                e = launch_fluid_step(arith, storage, coll, fb, ps, STEP_ALL, wall_blocks_for(c, c->g.tiles), c->sb);
         }
         if (e != hipSuccess) return hip_fail(c, e, "adjoint recompute");
         for (int64_t s = sb_; s > sa_; --s) {
@@ -2854,7 +2950,7 @@ bf_status bf_read_profile(bf_context* c, double out[6]) {
     out[2] = general;
     out[3] = (double)c->profiled;
     uint32_t general_tiles = 0;
-    hipError_t e = hipMemcpy(&general_tiles, &c->counters[par2(c->step)], 4, hipMemcpyDeviceToHost);
+    hipError_t e = hipMemcpy(&general_tiles, &c->counters[c->last_list], 4, hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(c, e, "read profile");
     out[4] = (double)general_tiles;
     out[5] = (double)c->g.tiles;

@@ -3,7 +3,7 @@
 //
 // Replaces the fluid part of stepFluidTRT (Sources/BirdFlowMetal/Metal/
 // BirdFlow.metal:2507-3236).  The lattice is split into 64x4 tiles, one
-// 256-lane workgroup each:
+// 256-lane workgroup each; one launch (fluid_step) covers both kinds:
 //   * fluid_fast    — tiles with no solid cell (current or previous step) in
 //                     their 1-cell halo: pure pull stream with per-face
 //                     boundary sources, collision, sponge blend, store.
@@ -572,13 +572,13 @@ __device__ __forceinline__ float write_post(typename Store<S>::T* __restrict__ f
 // Fast tiles.
 // ---------------------------------------------------------------------------
 template <int ARITH, int COLL, int S>
-__global__ __launch_bounds__(256) void fluid_fast(const typename Store<S>::T* __restrict__ fin,
-                                                  typename Store<S>::T* __restrict__ fout,
-                                                  const uint8_t* __restrict__ dyn_prev,
-                                                  const uint8_t* __restrict__ dyn_cur,
-                                                  uint32_t* __restrict__ activation, StepParams p) {
+__device__ __forceinline__ void fluid_fast(uint32_t block, uint32_t blocks,
+                                           const typename Store<S>::T* __restrict__ fin,
+                                           typename Store<S>::T* __restrict__ fout,
+                                           const uint8_t* __restrict__ dyn_prev, const uint8_t* __restrict__ dyn_cur,
+                                           uint32_t* __restrict__ activation, const StepParams& p) {
     set_priority(p.fast_priority);
-    const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t tile = xcd_remap(block, blocks);
     // Tiles with walls belong to fluid_general.  The flags are
     // loaded together with the populations and tested only before the
     // stores: a test up front would put a dependent memory round trip ahead
@@ -743,18 +743,19 @@ struct PairStore<STORE_BF16_OFFSET> {
 };
 
 template <int ARITH, int COLL, int S>
-__global__ __launch_bounds__(256) void fluid_fast_pair(const typename Store<S>::T* __restrict__ fin_t,
-                                                       typename Store<S>::T* __restrict__ fout_t,
-                                                       const uint8_t* __restrict__ dyn_prev,
-                                                       const uint8_t* __restrict__ dyn_cur,
-                                                       uint32_t* __restrict__ activation, StepParams p) {
+__device__ __forceinline__ void fluid_fast_pair(uint32_t block, uint32_t blocks,
+                                                const typename Store<S>::T* __restrict__ fin_t,
+                                                typename Store<S>::T* __restrict__ fout_t,
+                                                const uint8_t* __restrict__ dyn_prev,
+                                                const uint8_t* __restrict__ dyn_cur,
+                                                uint32_t* __restrict__ activation, const StepParams& p) {
     static_assert(S == STORE_FP16_OFFSET || S == STORE_BF16_OFFSET, "two-byte storage only");
     set_priority(p.fast_priority);
     const uint32_t* __restrict__ fin = reinterpret_cast<const uint32_t*>(fin_t);
     uint32_t* __restrict__ fout = reinterpret_cast<uint32_t*>(fout_t);
     const int nx = p.g.nx, ny = p.g.ny, nz = p.g.nz;
     const uint32_t pairs_x = (uint32_t)p.g.tiles_x / 2u;
-    const uint32_t pair = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t pair = xcd_remap(block, blocks);
     const uint32_t per_plane = pairs_x * (uint32_t)p.g.tiles_y;
     const int z = (int)(pair / per_plane);
     const uint32_t r = pair - (uint32_t)z * per_plane;
@@ -932,16 +933,16 @@ template <int ARITH, int COLL, int S>
 __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restrict__ fin, typename Store<S>::T* __restrict__ fout,
                              const uint8_t* __restrict__ solid_prev, const uint8_t* __restrict__ solid_cur,
                              const float4* __restrict__ wall, const StepParams& p, int x, int y, int z,
-                             float bx, float by, float bz, CellLoad& L) {
+                             float bx, float by, float bz, float* __restrict__ own, CellLoad& L) {
     const Grid& g = p.g;
-    const uint32_t row = (uint32_t)y + (uint32_t)g.ny * (uint32_t)z;
-    const uint32_t gid = (uint32_t)x + (uint32_t)g.nx * row;
+    const uint32_t row = (uint32_t)y + (uint32_t)g.ny * (uint32_t)z;   // y, z: wave-uniform
+    const size_t cells = (size_t)row * (size_t)g.nx;                   // first cell of the row
     const float wx = p.origin[0] + ((float)x + 0.5f) * p.dx;
     const float wy = p.origin[1] + ((float)y + 0.5f) * p.dx;
     const float wz = p.origin[2] + ((float)z + 0.5f) * p.dx;
     const float ax = wx - bx, ay = wy - by, az = wz - bz;
-    const bool was_solid = solid_prev[gid] != 0;
-    const bool is_solid = solid_cur[gid] != 0;
+    const bool was_solid = *row_at(solid_prev + cells, x) != 0;
+    const bool is_solid = *row_at(solid_cur + cells, x) != 0;
     const int mode = p.force_mode;
     const bool include_link = p.load_component != 2;
     const bool include_topology = p.load_component != 1;
@@ -949,7 +950,7 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
     L = CellLoad{0, 0, 0, 0, 0, 0, 0, 0};
 
     if (is_solid) {
-        const float4 wv = wall[gid];
+        const float4 wv = *row_at(wall + cells, x);
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
             Store<S>::store(row_ptr<S>(fout, g, q, row), x, q, equilibrium<float>(q, 1.0f, wv.x, wv.y, wv.z));
@@ -958,7 +959,7 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
             float prho = 0.0f, pmx = 0.0f, pmy = 0.0f, pmz = 0.0f;
             for_q(AllQ{}, [&](auto qc) {
                 constexpr int q = decltype(qc)::value;
-                float v = Store<S>::load(fin, pop_index<S>(g, q, x, row), q);
+                float v = Store<S>::load(row_ptr<S>(fin, g, q, row), x, q);
                 prho = prho + v;
                 pmx = pmx + v * (float)cx(q);
                 pmy = pmy + v * (float)cy(q);
@@ -981,7 +982,7 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
     float tqx = 0.0f, tqy = 0.0f, tqz = 0.0f;
 
     if (was_solid) {
-        const float4 rv = wall[gid];
+        const float4 rv = *row_at(wall + cells, x);
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
             float v = equilibrium<float>(q, 1.0f, rv.x, rv.y, rv.z);
@@ -993,48 +994,57 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
         });
         if (p.accumulate_loads && include_topology && mode == 6) {
             float tx = -mx, ty = -my, tz = -mz;
-            // two rounds of unconditional loads (a neighbour outside the
-            // domain reads this cell and is ignored): the neighbours' part
-            // ids, then the populations of the open directions
-            auto nb_of = [&](auto qc) {
+            // rounds of unconditional loads (a neighbour outside the domain
+            // reads this cell and is ignored): the neighbours' part ids, then
+            // the populations, six directions at a time
+            // row (wave-uniform) and x of neighbour x + c_q; this cell's where
+            // that leaves the domain
+            auto nb_row = [&](auto qc) {
                 constexpr int q = decltype(qc)::value;
-                const int bx = x + cx(q), by = y + cy(q), bz = z + cz(q);
-                return inside(g, bx, by, bz) ? flat(g, bx, by, bz) : gid;
+                const int by = y + cy(q), bz = z + cz(q);
+                return by >= 0 && bz >= 0 && by < g.ny && bz < g.nz ? (uint32_t)by + (uint32_t)g.ny * (uint32_t)bz
+                                                                    : row;
             };
-            // population opp(q) of that neighbour (of this cell outside the domain)
-            auto nb_pop = [&](auto qc) {
+            auto nb_x = [&](auto qc) {
                 constexpr int q = decltype(qc)::value;
-                const int bx = x + cx(q), by = y + cy(q), bz = z + cz(q);
-                return inside(g, bx, by, bz) ? pop_index<S>(g, opp(q), bx, (uint32_t)by + (uint32_t)g.ny * (uint32_t)bz)
-                                             : pop_index<S>(g, opp(q), x, row);
+                return min(max(x + cx(q), 0), g.nx - 1);
             };
             uint32_t mk[19];
-            uint32_t inbits = 0;
+            uint32_t open = 0;
             for_q(AllQ{}, [&](auto qc) {
                 constexpr int q = decltype(qc)::value;
-                const uint32_t nb = nb_of(qc);
-                mk[q] = (uint32_t)solid_prev[nb] | (uint32_t)solid_cur[nb];
-                inbits |= (uint32_t)inside(g, x + cx(q), y + cy(q), z + cz(q)) << q;
+                const size_t nb = (size_t)nb_row(qc) * (size_t)g.nx;
+                mk[q] = (uint32_t)*row_at(solid_prev + nb, nb_x(qc)) | (uint32_t)*row_at(solid_cur + nb, nb_x(qc));
             });
             asm volatile("" : BF_ASM19(mk));
-            float own[19], far[19];
             for_q(AllQ{}, [&](auto qc) {
                 constexpr int q = decltype(qc)::value;
-                own[q] = Store<S>::load(fin, pop_index<S>(g, q, x, row), q);
-                far[q] = Store<S>::load(fin, nb_pop(qc), opp(q));
+                open |= (uint32_t)(q != 0 && mk[q] == 0 && inside(g, x + cx(q), y + cy(q), z + cz(q))) << q;
             });
-            asm volatile("" : BF_ASM19(own), BF_ASM19(far));
-            for_q(AllQ{}, [&](auto qc) {
-                constexpr int q = decltype(qc)::value;
-                if constexpr (q != 0) {
-                    if (((inbits >> q) & 1u) && mk[q] == 0) {
-                        float s = own[q] + far[q];
+            auto impulse_group = [&](auto seq, auto first_c) {
+                constexpr int q0 = decltype(first_c)::value;
+                float near[6], far[6];
+                for_q(seq, [&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    near[q - q0] = Store<S>::load(row_ptr<S>(fin, g, q, row), x, q);
+                    far[q - q0] = Store<S>::load(row_ptr<S>(fin, g, opp(q), nb_row(qc)), nb_x(qc), opp(q));
+                });
+                asm volatile("" : "+v"(near[0]), "+v"(near[1]), "+v"(near[2]), "+v"(near[3]), "+v"(near[4]),
+                             "+v"(near[5]), "+v"(far[0]), "+v"(far[1]), "+v"(far[2]), "+v"(far[3]), "+v"(far[4]),
+                             "+v"(far[5]));
+                for_q(seq, [&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    if ((open >> q) & 1u) {
+                        float s = near[q - q0] + far[q - q0];
                         tx = tx - s * (float)cx(q);
                         ty = ty - s * (float)cy(q);
                         tz = tz - s * (float)cz(q);
                     }
-                }
-            });
+                });
+            };
+            impulse_group(QSeq<1, 2, 3, 4, 5, 6>{}, std::integral_constant<int, 1>{});
+            impulse_group(QSeq<7, 8, 9, 10, 11, 12>{}, std::integral_constant<int, 7>{});
+            impulse_group(QSeq<13, 14, 15, 16, 17, 18>{}, std::integral_constant<int, 13>{});
             flx = flx + tx;
             fly = fly + ty;
             flz = flz + tz;
@@ -1047,88 +1057,81 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
     } else {
         const float mwd = p.far_rho;
         const bool interpolated_rule = p.wall_rule != WALL_HALFWAY;
-        const float4 wg = wall[gid];
-        // Loads in two passes.  First, unconditionally and without a branch
-        // between them (a far-field source, or a far side outside the
-        // domain, reads this cell and is ignored): every source's part id and
-        // population, this cell's own populations (reflected and x-side
-        // values of its links) and the part id of each link's far side.
-        // Conditional loads here would cost one memory round trip per
-        // direction.  Then, per link, the source's wall entry and the
-        // far-side population.
+        // Loads in rounds, each without a branch between its loads (a load
+        // inside a link's branch would cost a memory round trip per link
+        // direction of the wavefront).  First the part ids of the 18 sources (a
+        // far-field source reads this cell's and is ignored).  A wavefront
+        // without links, most of a wall tile, then streams as fluid_fast does.
         const Sources sq = sources(p, x, y, z);
-        // source and far-side cell of direction q (far-field / outside: this
-        // cell); recomputed where needed rather than kept in registers
-        auto src_of = [&](auto qc) {
+        // the source of direction q: its row (wave-uniform, as everything
+        // along y and z) and x; this cell's coordinate along an axis on which
+        // it lies beyond a far-field face
+        auto src_row = [&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            bool far;
-            const uint32_t src = source_of<q>(sq, g, x, y, z, far);
-            return far ? gid : src;
+            const bool fy = (cy(q) > 0 && sq.ym_far) || (cy(q) < 0 && sq.yp_far);
+            const bool fz = (cz(q) > 0 && sq.zm_far) || (cz(q) < 0 && sq.zp_far);
+            const int ys = fy || cy(q) == 0 ? y : (cy(q) > 0 ? sq.ys_p : sq.ys_m);
+            const int zs = fz || cz(q) == 0 ? z : (cz(q) > 0 ? sq.zs_p : sq.zs_m);
+            return (uint32_t)ys + (uint32_t)g.ny * (uint32_t)zs;
         };
-        auto far_side_of = [&](auto qc) {
+        const int xs_p = sq.xm_far ? x : sq.xs_p, xs_m = sq.xp_far ? x : sq.xs_m;
+        auto src_x = [&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            const int fx = x + cx(q), fy = y + cy(q), fz = z + cz(q);
-            return inside(g, fx, fy, fz) ? flat(g, fx, fy, fz) : gid;
+            return cx(q) > 0 ? xs_p : (cx(q) < 0 ? xs_m : x);
         };
-        // population opp(q) on the far side (of this cell outside the domain)
-        auto far_side_pop = [&](auto qc) {
+        uint32_t partq[19];
+        for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            const int fx = x + cx(q), fy = y + cy(q), fz = z + cz(q);
-            return inside(g, fx, fy, fz) ? pop_index<S>(g, opp(q), fx, (uint32_t)fy + (uint32_t)g.ny * (uint32_t)fz)
-                                         : pop_index<S>(g, opp(q), x, row);
-        };
-        uint32_t partq[19], fpart[19];
-        float fsrc[19], fown[19];
-        uint32_t farbits = 0, okbits = 0;
+            partq[q] = *row_at(solid_cur + (size_t)src_row(qc) * (size_t)g.nx, src_x(qc));
+        });
+        asm volatile("" : BF_ASM19(partq));
+        // links; links whose part counts toward the loads; links whose far
+        // side x + c_q is outside the domain or solid, which forces the halfway
+        // fallback.  Inside the domain the far side of q is the source of the
+        // opposite direction, so its part id and its population (pulled along
+        // that direction) are already here.
+        uint32_t farbits = 0, linkbits = 0, selbits = 0, fallbits = 0;
+        const int sel = p.selected_part;
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
             bool far;
             (void)source_of<q>(sq, g, x, y, z, far);
             farbits |= (uint32_t)far << q;
-            okbits |= (uint32_t)inside(g, x + cx(q), y + cy(q), z + cz(q)) << q;
-            const uint32_t src = src_of(qc), fid = far_side_of(qc);
-            partq[q] = solid_cur[src];
-            fpart[q] = solid_cur[fid];
-            int xs;
-            uint32_t rows;
-            bool farq;
-            source_xr<q>(sq, g, x, y, z, xs, rows, farq);
-            fsrc[q] = Store<S>::load(fin, farq ? pop_index<S>(g, q, x, row) : pop_index<S>(g, q, xs, rows), q);
-            fown[q] = Store<S>::load(fin, pop_index<S>(g, q, x, row), q);
+            linkbits |= (uint32_t)(partq[q] != 0 && !far) << q;
+            selbits |= (uint32_t)(sel == 0 || sel == (int)partq[q]) << q;
+            fallbits |= (uint32_t)(!inside(g, x + cx(q), y + cy(q), z + cz(q)) || partq[opp(q)] != 0) << q;
         });
-        asm volatile("" : BF_ASM19(fsrc), BF_ASM19(fown), BF_ASM19(partq), BF_ASM19(fpart));
-        // links; far sides that force the halfway fallback; links whose part
-        // counts toward the loads
-        uint32_t linkbits = 0, fallbits = 0, selbits = 0;
-        const int sel = p.selected_part;
+        // the pulled populations; in a wavefront with links also the cell's
+        // own ones (reflected and x-side values), kept in this lane's column of
+        // LDS rather than in 19 registers, and its wall entry
         for_q(AllQ{}, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            linkbits |= (uint32_t)(partq[q] != 0 && !((farbits >> q) & 1u)) << q;
-            fallbits |= (uint32_t)(!((okbits >> q) & 1u) || fpart[q] != 0) << q;
-            selbits |= (uint32_t)(sel == 0 || sel == (int)partq[q]) << q;
+            f[q] = Store<S>::load(row_ptr<S>(fin, g, q, src_row(qc)), src_x(qc), q);
         });
-        // Second load pass, six directions at a time: the wall entry of each link's
-        // source and the population on its far side, all loaded before any is
-        // used (a direction without a link reads this cell's entries and
-        // ignores them); then the values of the group's directions in
-        // ascending q.  A load per link inside the link branch would cost one
-        // memory round trip per link direction of the wavefront.
+        float4 wg = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (__any(linkbits != 0)) {
+            float fown[19];
+            wg = *row_at(wall + cells, x);
+            for_q(AllQ{}, [&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                fown[q] = Store<S>::load(row_ptr<S>(fin, g, q, row), x, q);
+            });
+            asm volatile("" : BF_ASM19(f), BF_ASM19(fown));
+            for (int q = 0; q < 19; ++q) own[q * TILE_CELLS] = fown[q];
+        } else {
+            asm volatile("" : BF_ASM19(f));
+        }
+        // then, six directions at a time, the wall entries of the links'
+        // sources (a direction without a link ignores what it reads), and the
+        // values of the group's directions in ascending q
         auto link_group = [&](auto seq, auto first_c, uint32_t gmask) {
             constexpr int q0 = decltype(first_c)::value;
             float4 wsg[7];
-            float fog[7];
-            for (int k = 0; k < 7; ++k) {
-                wsg[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                fog[k] = 0.0f;
-            }
+            for (int k = 0; k < 7; ++k) wsg[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (linkbits & gmask) {
                 for_q(seq, [&](auto qc) {
                     constexpr int q = decltype(qc)::value;
-                    if constexpr (q != 0) {
-                        const bool lk = (linkbits >> q) & 1u;
-                        wsg[q - q0] = wall[lk ? src_of(qc) : gid];
-                        fog[q - q0] = Store<S>::load(fin, lk ? far_side_pop(qc) : pop_index<S>(g, opp(q), x, row), opp(q));
-                    }
+                    if constexpr (q != 0) wsg[q - q0] = *row_at(wall + (size_t)src_row(qc) * (size_t)g.nx, src_x(qc));
                 });
                 asm volatile("" : "+v"(wsg[0].x), "+v"(wsg[0].y), "+v"(wsg[0].z), "+v"(wsg[0].w),
                              "+v"(wsg[1].x), "+v"(wsg[1].y), "+v"(wsg[1].z), "+v"(wsg[1].w),
@@ -1136,9 +1139,7 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
                              "+v"(wsg[3].x), "+v"(wsg[3].y), "+v"(wsg[3].z), "+v"(wsg[3].w),
                              "+v"(wsg[4].x), "+v"(wsg[4].y), "+v"(wsg[4].z), "+v"(wsg[4].w),
                              "+v"(wsg[5].x), "+v"(wsg[5].y), "+v"(wsg[5].z), "+v"(wsg[5].w),
-                             "+v"(wsg[6].x), "+v"(wsg[6].y), "+v"(wsg[6].z), "+v"(wsg[6].w),
-                             "+v"(fog[0]), "+v"(fog[1]), "+v"(fog[2]), "+v"(fog[3]), "+v"(fog[4]), "+v"(fog[5]),
-                             "+v"(fog[6]));
+                             "+v"(wsg[6].x), "+v"(wsg[6].y), "+v"(wsg[6].z), "+v"(wsg[6].w));
             }
             for_q(seq, [&](auto qc) {
             constexpr int q = decltype(qc)::value;
@@ -1148,10 +1149,12 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
                 value = p.far_eq[q];
             } else {
                 if ((linkbits >> q) & 1u) {
-                    const float reflected = fown[opp(q)];
+                    const float reflected = own[opp(q) * TILE_CELLS];
                     float lf = 0.5f;
                     const float4 ws = wsg[q - q0];
-                    const float fo_far = fog[q - q0];
+                    // (f[opp(q)] still holds the pulled value: had it been a
+                    // link's, the far side would be solid)
+                    const float fo_far = f[opp(q)];
                     float wvx = ws.x, wvy = ws.y, wvz = ws.z;
                     bool interp = interpolated_rule;
                     if (interp) {
@@ -1188,7 +1191,7 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
                             const float fo = fo_far;
                             value = 2.0f * lf * reflected + (1.0f - 2.0f * lf) * fo + corr;
                         } else {
-                            const float pin = fown[q];
+                            const float pin = own[q * TILE_CELLS];
                             value = (reflected + corr) / (2.0f * lf) + (2.0f * lf - 1.0f) * pin / (2.0f * lf);
                         }
                     }
@@ -1237,7 +1240,7 @@ __device__ __forceinline__ void general_cell(const typename Store<S>::T* __restr
                         tqz = tqz + oz;
                     }
                 } else {
-                    value = fsrc[q];
+                    value = f[q];
                 }
             }
             f[q] = value;
@@ -1306,20 +1309,21 @@ __device__ __forceinline__ void block_reduce8(double (&v)[8], double* __restrict
 }
 
 template <int ARITH, int COLL, int S>
-__global__ __launch_bounds__(256) void fluid_general(const typename Store<S>::T* __restrict__ fin,
-                                                     typename Store<S>::T* __restrict__ fout,
-                                                     const uint8_t* __restrict__ solid_prev,
-                                                     const uint8_t* __restrict__ solid_cur,
-                                                     const float4* __restrict__ wall,
-                                                     const uint32_t* __restrict__ general_list,
-                                                     const uint32_t* __restrict__ general_count,
-                                                     double* __restrict__ partials,
-                                                     const double* __restrict__ body, StepParams p) {
+__device__ __forceinline__ void fluid_general(uint32_t block, uint32_t blocks,
+                                              const typename Store<S>::T* __restrict__ fin,
+                                              typename Store<S>::T* __restrict__ fout,
+                                              const uint8_t* __restrict__ solid_prev,
+                                              const uint8_t* __restrict__ solid_cur, const float4* __restrict__ wall,
+                                              const uint32_t* __restrict__ general_list,
+                                              const uint32_t* __restrict__ general_count,
+                                              double* __restrict__ partials, const double* __restrict__ body,
+                                              const StepParams& p) {
     set_priority(p.general_priority);
     const uint32_t count = *general_count;
     // torque reference point: the body position, read once per workgroup
     const float bx = (float)body[0], by = (float)body[1], bz = (float)body[2];
-    for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
+    __shared__ float own[19 * TILE_CELLS];   // each lane's own column, no exchange
+    for (uint32_t i = block; i < count; i += blocks) {
         const uint32_t tile = general_list[i];
         int x0, y0, z;
         tile_origin(p.g, tile, x0, y0, z);
@@ -1327,7 +1331,8 @@ __global__ __launch_bounds__(256) void fluid_general(const typename Store<S>::T*
         const int y = y0 + (int)__builtin_amdgcn_readfirstlane(threadIdx.x / TILE_X);
         CellLoad L{0, 0, 0, 0, 0, 0, 0, 0};
         if (x < p.g.nx && y < p.g.ny)
-            general_cell<ARITH, COLL, S>(fin, fout, solid_prev, solid_cur, wall, p, x, y, z, bx, by, bz, L);
+            general_cell<ARITH, COLL, S>(fin, fout, solid_prev, solid_cur, wall, p, x, y, z, bx, by, bz,
+                                         own + threadIdx.x, L);
         if (p.accumulate_loads) {
             double v[8] = {(double)L.fx, (double)L.fy, (double)L.fz, (double)L.tx,
                            (double)L.ty, (double)L.tz, (double)L.act, (double)L.restr};
@@ -1337,32 +1342,68 @@ __global__ __launch_bounds__(256) void fluid_general(const typename Store<S>::T*
 }
 
 // ---------------------------------------------------------------------------
+// One launch per step: the first wall_blocks workgroups walk the wall-tile
+// list, the others stream one tile (or tile pair) each.
+//
+// The wall tiles are bound by latency (three rounds of dependent loads, a few
+// hundred workgroups), the others by HBM; as two launches in a row the wall
+// tiles left the card idle for 30 - 100 us of every step, and as concurrent
+// launches their 208-register wavefronts found no room beside the others'.
+// In one launch they start first and the streaming fills the rest.  Held to 4
+// wavefronts per SIMD (128 registers): the wall path spills 7 - 72 of them
+// and still ends long before the streaming does; the streaming alone loses 1 %
+// to its natural 7 wavefronts at 512x256x256.  5 wavefronts gain that back on
+// the largest grids (969 against 982 us per step) and lose where the wall
+// tiles are the step (80x80x48 half-way plate: 34.6 against 27.2); 6 lose
+// everywhere.  256x128x128 plate 168 -> 139 us per step, 64^3 box 46 -> 10
+// (with the launches that static geometry no longer needs).
+// ---------------------------------------------------------------------------
+template <int ARITH, int COLL, int S, bool PAIR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+void fluid_step(const typename Store<S>::T* __restrict__ fin, typename Store<S>::T* __restrict__ fout,
+                const uint8_t* __restrict__ solid_prev, const uint8_t* __restrict__ solid_cur,
+                const float4* __restrict__ wall, const uint8_t* __restrict__ dyn_prev,
+                const uint8_t* __restrict__ dyn_cur, const uint32_t* __restrict__ general_list,
+                const uint32_t* __restrict__ general_count, double* __restrict__ partials,
+                const double* __restrict__ body, uint32_t* __restrict__ activation, StepParams p,
+                uint32_t wall_blocks) {
+    if (blockIdx.x < wall_blocks) {
+        fluid_general<ARITH, COLL, S>(blockIdx.x, wall_blocks, fin, fout, solid_prev, solid_cur, wall, general_list,
+                                      general_count, partials, body, p);
+        return;
+    }
+    const uint32_t block = blockIdx.x - wall_blocks, blocks = gridDim.x - wall_blocks;
+    if constexpr (PAIR)
+        fluid_fast_pair<ARITH, COLL, S>(block, blocks, fin, fout, dyn_prev, dyn_cur, activation, p);
+    else
+        fluid_fast<ARITH, COLL, S>(block, blocks, fin, fout, dyn_prev, dyn_cur, activation, p);
+}
+
+// ---------------------------------------------------------------------------
 // Host-side launchers (called from bf_api.hip).
 // ---------------------------------------------------------------------------
 
-template <int ARITH, int COLL, int S>
-static hipError_t launch_fast_t(const FluidBuffers& b, const StepParams& p, hipStream_t s) {
+template <int ARITH, int COLL, int S, bool PAIR>
+static hipError_t launch_step_p(const FluidBuffers& b, const StepParams& p, uint32_t wall_blocks, uint32_t fast_blocks,
+                                hipStream_t s) {
     using T = typename Store<S>::T;
-    if constexpr (S != STORE_FP32) {
-        // two cells per lane over tile pairs (whole pairs along x)
-        if (p.g.nx % (2 * TILE_X) == 0 && p.pair_cells) {
-            hipLaunchKernelGGL((fluid_fast_pair<ARITH, COLL, S>), dim3(p.g.tiles / 2), dim3(256), 0, s,
-                               (const T*)b.fin, (T*)b.fout, b.dyn_prev, b.dyn_cur, b.activation, p);
-            return hipGetLastError();
-        }
-    }
-    hipLaunchKernelGGL((fluid_fast<ARITH, COLL, S>), dim3(p.g.tiles), dim3(256), 0, s, (const T*)b.fin,
-                       (T*)b.fout, b.dyn_prev, b.dyn_cur, b.activation, p);
+    if (wall_blocks + fast_blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL((fluid_step<ARITH, COLL, S, PAIR>), dim3(wall_blocks + fast_blocks), dim3(256), 0, s,
+                       (const T*)b.fin, (T*)b.fout, b.solid_prev, b.solid_cur, b.wall, b.dyn_prev, b.dyn_cur,
+                       b.general_list, b.general_count, b.partials, b.body, b.activation, p, wall_blocks);
     return hipGetLastError();
 }
 
 template <int ARITH, int COLL, int S>
-static hipError_t launch_general_t(const FluidBuffers& b, const StepParams& p, int general_blocks, hipStream_t s) {
-    using T = typename Store<S>::T;
-    hipLaunchKernelGGL((fluid_general<ARITH, COLL, S>), dim3(general_blocks), dim3(256), 0, s, (const T*)b.fin,
-                       (T*)b.fout, b.solid_prev, b.solid_cur, b.wall, b.general_list, b.general_count,
-                       b.partials, b.body, p);
-    return hipGetLastError();
+static hipError_t launch_step_t(const FluidBuffers& b, const StepParams& p, int parts, uint32_t wall_blocks,
+                                hipStream_t s) {
+    const uint32_t wb = parts & STEP_WALL_TILES ? wall_blocks : 0u;
+    if constexpr (S != STORE_FP32) {
+        // two cells per lane over tile pairs (whole pairs along x)
+        if (p.g.nx % (2 * TILE_X) == 0 && p.pair_cells)
+            return launch_step_p<ARITH, COLL, S, true>(b, p, wb, parts & STEP_FAST_TILES ? p.g.tiles / 2 : 0u, s);
+    }
+    return launch_step_p<ARITH, COLL, S, false>(b, p, wb, parts & STEP_FAST_TILES ? p.g.tiles : 0u, s);
 }
 
 }  // namespace bf

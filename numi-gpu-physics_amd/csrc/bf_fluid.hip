@@ -26,14 +26,18 @@ __global__ __launch_bounds__(256) void build_general_list(const uint8_t* __restr
 
 
 
-// Fixed-order sum of the per-tile partials of the tiles the general kernel
-// processed (flags identify them; other tiles contribute exactly zero).
+// Fixed-order sum of the per-tile partials of the tiles the general path
+// processed (flags identify them; other tiles contribute exactly zero), for a
+// batch of steps with the same flags (one grid row each).
 __global__ __launch_bounds__(256) void reduce_loads_tiles(const double* __restrict__ partials,
                                                           const uint8_t* __restrict__ dyn_prev,
                                                           const uint8_t* __restrict__ dyn_cur, uint32_t tiles,
-                                                          double* __restrict__ block_out) {
+                                                          double* __restrict__ block_out, uint32_t slot0) {
     constexpr uint32_t PER_THREAD = 4;
     double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    // row k of the grid: the k-th step of the batch, its partials in their slot
+    partials += (size_t)((slot0 + blockIdx.y) % LOAD_SLOTS) * tiles * 8;
+    block_out += (size_t)blockIdx.y * gridDim.x * 8;
     const uint32_t base = (blockIdx.x * blockDim.x + threadIdx.x) * PER_THREAD;
     for (uint32_t k = 0; k < PER_THREAD; ++k) {
         const uint32_t t = base + k;
@@ -51,8 +55,12 @@ __global__ __launch_bounds__(256) void reduce_loads_tiles(const double* __restri
 __global__ __launch_bounds__(256) void reduce_loads_final(const double* __restrict__ block_out, uint32_t blocks,
                                                           uint32_t* __restrict__ activation,
                                                           double* __restrict__ last, double* __restrict__ history,
-                                                          uint32_t history_slot) {
+                                                          uint32_t history_slot, uint32_t history_capacity,
+                                                          uint32_t slot0) {
     double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    block_out += (size_t)blockIdx.x * blocks * 8;
+    activation += 2 * ((slot0 + blockIdx.x) % LOAD_SLOTS);
+    history_slot = (history_slot + blockIdx.x) % history_capacity;
     for (uint32_t b = threadIdx.x; b < blocks; b += blockDim.x) {
 #pragma unroll
         for (int i = 0; i < 7; ++i) v[i] += block_out[(size_t)b * 8 + i];
@@ -64,7 +72,7 @@ __global__ __launch_bounds__(256) void reduce_loads_final(const double* __restri
         double t = total[threadIdx.x];
         if (threadIdx.x == 6) t += (double)activation[0];
         if (threadIdx.x == 7) t = fmax(t, (double)__uint_as_float(activation[1]));
-        last[threadIdx.x] = t;
+        if (blockIdx.x == gridDim.x - 1) last[threadIdx.x] = t;
         if (history) history[(size_t)history_slot * 8 + threadIdx.x] = t;
     }
     __syncthreads();
@@ -286,32 +294,30 @@ hipError_t launch_poke_population(int storage, void* f, const Grid& g, unsigned 
     return hipGetLastError();
 }
 
-hipError_t launch_load_reduction(const FluidBuffers& b, const StepParams& p, uint32_t history_slot, hipStream_t s) {
-    if (!p.accumulate_loads) return hipSuccess;
-    const uint32_t blocks = (p.g.tiles + 1023) / 1024;
-    hipLaunchKernelGGL(reduce_loads_tiles, dim3(blocks), dim3(256), 0, s, b.partials, b.dyn_prev, b.dyn_cur,
-                       p.g.tiles, b.block_out);
-    hipLaunchKernelGGL(reduce_loads_final, dim3(1), dim3(256), 0, s, b.block_out, blocks, b.activation, b.last_load,
-                       b.history, history_slot);
+hipError_t launch_load_reduction(const LoadBuffers& b, const StepParams& p, uint64_t step, uint32_t batch,
+                                 hipStream_t s) {
+    if (!p.accumulate_loads || batch == 0) return hipSuccess;
+    if (batch > LOAD_SLOTS) return hipErrorInvalidValue;
+    const uint32_t blocks = (p.g.tiles + 1023) / 1024, slot0 = (uint32_t)(step % LOAD_SLOTS);
+    hipLaunchKernelGGL(reduce_loads_tiles, dim3(blocks, batch), dim3(256), 0, s, b.partials, b.dyn_prev, b.dyn_cur,
+                       p.g.tiles, b.block_out, slot0);
+    hipLaunchKernelGGL(reduce_loads_final, dim3(batch), dim3(256), 0, s, b.block_out, blocks, b.activation,
+                       b.last_load, b.history, (uint32_t)(step % b.history_capacity), b.history_capacity, slot0);
     return hipGetLastError();
 }
 
-hipError_t launch_fluid_fast(int arith, int storage, int coll, const FluidBuffers& b, const StepParams& p,
-                             hipStream_t s) {
+hipError_t launch_fluid_step(int arith, int storage, int coll, const FluidBuffers& b, const StepParams& p, int parts,
+                             uint32_t wall_blocks, hipStream_t s) {
     if (arith == ARITH_STRICT) {
         if (storage != STORE_FP32) return hipErrorInvalidValue;
-        return launch_fluid_fast_strict(coll, b, p, s);
+        return launch_fluid_step_strict(coll, b, p, parts, wall_blocks, s);
     }
-    return launch_fluid_fast_fused(storage, coll, b, p, s);
-}
-
-hipError_t launch_fluid_general(int arith, int storage, int coll, const FluidBuffers& b, const StepParams& p,
-                                int general_blocks, hipStream_t s) {
-    if (arith == ARITH_STRICT) {
-        if (storage != STORE_FP32) return hipErrorInvalidValue;
-        return launch_fluid_general_strict(coll, b, p, general_blocks, s);
+    switch (storage) {
+        case STORE_FP32: return launch_fluid_step_fused(coll, b, p, parts, wall_blocks, s);
+        case STORE_FP16_OFFSET: return launch_fluid_step_fp16(coll, b, p, parts, wall_blocks, s);
+        case STORE_BF16_OFFSET: return launch_fluid_step_bf16(coll, b, p, parts, wall_blocks, s);
+        default: return hipErrorInvalidValue;
     }
-    return launch_fluid_general_fused(storage, coll, b, p, general_blocks, s);
 }
 
 hipError_t launch_build_general_list(const uint8_t* dyn_prev, const uint8_t* dyn_cur, uint32_t tiles, uint32_t* list,

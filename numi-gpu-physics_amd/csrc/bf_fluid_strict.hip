@@ -14,15 +14,9 @@ namespace bf {
         default: return hipErrorInvalidValue;                 \
     }
 
-hipError_t launch_fluid_fast_strict(int coll, const FluidBuffers& b, const StepParams& p, hipStream_t s) {
-#define CALL(C) launch_fast_t<ARITH_STRICT, C, STORE_FP32>(b, p, s)
-    BF_STRICT_DISPATCH(coll, CALL)
-#undef CALL
-}
-
-hipError_t launch_fluid_general_strict(int coll, const FluidBuffers& b, const StepParams& p, int general_blocks,
-                                       hipStream_t s) {
-#define CALL(C) launch_general_t<ARITH_STRICT, C, STORE_FP32>(b, p, general_blocks, s)
+hipError_t launch_fluid_step_strict(int coll, const FluidBuffers& b, const StepParams& p, int parts,
+                                    uint32_t wall_blocks, hipStream_t s) {
+#define CALL(C) launch_step_t<ARITH_STRICT, C, STORE_FP32>(b, p, parts, wall_blocks, s)
     BF_STRICT_DISPATCH(coll, CALL)
 #undef CALL
 }

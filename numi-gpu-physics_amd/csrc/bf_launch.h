@@ -39,11 +39,21 @@ struct FluidBuffers {
     uint32_t* general_list;
     uint32_t* general_count;
     double* partials;
-    double* block_out;
-    double* last_load;
-    double* history;
     uint32_t* activation;   // [count, max restriction bits] of this step's fast tiles
     const double* body;     // body state (position first): torque reference point
+};
+
+// A step's load partials wait in slot step % LOAD_SLOTS for their reduction.
+constexpr uint32_t LOAD_SLOTS = 4;
+struct LoadBuffers {
+    const double* partials;      // [LOAD_SLOTS][tiles][8]
+    const uint8_t* dyn_prev;
+    const uint8_t* dyn_cur;
+    double* block_out;           // [LOAD_SLOTS][blocks][8]
+    uint32_t* activation;        // [LOAD_SLOTS][2]
+    double* last_load;
+    double* history;             // [history_capacity][8]
+    uint32_t history_capacity;
 };
 
 struct MeshParams {
@@ -326,20 +336,25 @@ hipError_t launch_body_step(double* state, const double* load, double* history, 
                             double* metrics, uint32_t* event, uint64_t step, const BodyParams& bp, hipStream_t s,
                             const float* wing_reaction = nullptr);
 
-hipError_t launch_fluid_fast(int arith, int storage, int coll, const FluidBuffers& b, const StepParams& p,
-                             hipStream_t s);
-hipError_t launch_fluid_general(int arith, int storage, int coll, const FluidBuffers& b, const StepParams& p,
-                                int general_blocks, hipStream_t s);
-// Per translation unit: fused arithmetic for every storage, strict
+// The fluid step in one launch, or one of its parts alone: the wall tiles of
+// b.general_list over wall_blocks workgroups, the wall-free tiles.
+enum : int { STEP_WALL_TILES = 1, STEP_FAST_TILES = 2, STEP_ALL = 3 };
+hipError_t launch_fluid_step(int arith, int storage, int coll, const FluidBuffers& b, const StepParams& p, int parts,
+                             uint32_t wall_blocks, hipStream_t s);
+// Per translation unit: fused arithmetic by storage (FP32, FP16, BF16), strict
 // arithmetic for FP32 storage.
-hipError_t launch_fluid_fast_fused(int storage, int coll, const FluidBuffers& b, const StepParams& p,
-                                   hipStream_t s);
-hipError_t launch_fluid_general_fused(int storage, int coll, const FluidBuffers& b, const StepParams& p,
-                                      int general_blocks, hipStream_t s);
-hipError_t launch_fluid_fast_strict(int coll, const FluidBuffers& b, const StepParams& p, hipStream_t s);
-hipError_t launch_fluid_general_strict(int coll, const FluidBuffers& b, const StepParams& p, int general_blocks,
-                                       hipStream_t s);
-hipError_t launch_load_reduction(const FluidBuffers& b, const StepParams& p, uint32_t history_slot, hipStream_t s);
+hipError_t launch_fluid_step_fused(int coll, const FluidBuffers& b, const StepParams& p, int parts,
+                                   uint32_t wall_blocks, hipStream_t s);
+hipError_t launch_fluid_step_fp16(int coll, const FluidBuffers& b, const StepParams& p, int parts,
+                                  uint32_t wall_blocks, hipStream_t s);
+hipError_t launch_fluid_step_bf16(int coll, const FluidBuffers& b, const StepParams& p, int parts,
+                                  uint32_t wall_blocks, hipStream_t s);
+hipError_t launch_fluid_step_strict(int coll, const FluidBuffers& b, const StepParams& p, int parts,
+                                    uint32_t wall_blocks, hipStream_t s);
+// Loads of steps `step` .. `step` + batch - 1 (batch <= LOAD_SLOTS, the same
+// tile flags for all of them) into the history and, the last one's, last_load.
+hipError_t launch_load_reduction(const LoadBuffers& b, const StepParams& p, uint64_t step, uint32_t batch,
+                                 hipStream_t s);
 hipError_t launch_build_general_list(const uint8_t* dyn_prev, const uint8_t* dyn_cur, uint32_t tiles, uint32_t* list,
                                      uint32_t* count, hipStream_t s);
 hipError_t launch_init_equilibrium(int storage, void* f, const uint8_t* solid, const float4* wall,
