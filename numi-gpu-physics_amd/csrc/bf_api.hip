@@ -46,6 +46,10 @@ static_assert(BF_COLLISION_RR3 == COLL_RR3 && BF_WALL_INTERPOLATED_HALF == WALL_
 namespace {
 constexpr uint32_t HISTORY_CAPACITY = 1u << 16;
 constexpr uint32_t PROFILE_CAPACITY = 4096;
+// Events that order one stream after another on the same device: no timing,
+// and no system-scope fence (the host waits for streams, never for these;
+// 4 - 6 us less between the fluid launches of consecutive steps).
+constexpr unsigned STREAM_EVENT = hipEventDisableTiming | hipEventDisableSystemFence;
 constexpr int PROFILE_EVENTS = 6;   // A: fast start/end; B: geometry start/end, general start/end
 
 struct DeviceAlloc {
@@ -124,6 +128,7 @@ struct bf_context {
     bool static_prev_differs = false;
     float time_start = 0.0f;              // time of step 0
     int64_t geometry_ready = 0;           // highest step whose geometry is enqueued
+    int64_t list_step = -1;               // step whose wall-tile list follows it (moving geometry)
     // mesh
     float* m_points = nullptr;
     float* m_times = nullptr;
@@ -622,6 +627,7 @@ bf_status ensure_ray_static(bf_context* c) {
     return BF_OK;
 }
 
+// (Also clears the length of the step's wall-tile list.)
 bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
     hipError_t e = hipSuccess;
     if (c->source == BF_GEOMETRY_MESH) {
@@ -632,6 +638,7 @@ bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
         b.tiles_wall_old = fresh ? c->no_tiles : c->tflags[mod4(s - 2)];   // wall[s&1] last written at s-2
         b.list = c->geo_list;
         b.list_count = &c->counters[2];
+        b.general_count = &c->counters[par2(s)];
         b.mask = c->mask[mod3(s)];
         b.wall = c->wall[par2(s)];
         b.dyn = c->dyn[mod3(s)];
@@ -677,6 +684,7 @@ bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
         b.tiles_wall_old = fresh ? c->no_tiles : c->tflags[mod4(s - 2)];
         b.list = c->geo_list;
         b.list_count = &c->counters[2];
+        b.general_count = &c->counters[par2(s)];
         b.mask = c->mask[mod3(s)];
         b.wall = c->wall[par2(s)];
         b.dyn = c->dyn[mod3(s)];
@@ -708,6 +716,7 @@ bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
         b.tiles_wall_old = fresh ? c->no_tiles : c->tflags[mod4(s - 2)];
         b.list = c->geo_list;
         b.list_count = &c->counters[2];
+        b.general_count = &c->counters[par2(s)];
         b.mask = c->mask[mod3(s)];
         b.wall = c->wall[par2(s)];
         b.dyn = c->dyn[mod3(s)];
@@ -729,17 +738,19 @@ bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
         int periodic[3];
         for (int a = 0; a < 3; ++a) periodic[a] = periodic_axis(c->cfg, a) ? 1 : 0;
         e = launch_sphere_geometry(c->mask[mod3(s)], c->wall[par2(s)], c->dyn[mod3(s)], c->g, c->sphere_cr,
-                                   c->sphere_gv, c->sphere_wv, time_of(c, s), periodic, c->sb);
+                                   c->sphere_gv, c->sphere_wv, time_of(c, s), periodic, &c->counters[par2(s)],
+                                   c->sb);
     }
     if (e != hipSuccess) return hip_fail(c, e, "geometry launch");
     return BF_OK;
 }
 
 // List of the tiles that take the general path in step s, into list slot
-// `slot`, on stream st.
-bf_status enqueue_tile_list(bf_context* c, int64_t s, int slot, hipStream_t st) {
+// `slot`, on stream st; `cleared`: the step's geometry was enqueued just
+// before and cleared its length.
+bf_status enqueue_tile_list(bf_context* c, int64_t s, int slot, bool cleared, hipStream_t st) {
     const StepGeometry sg = geometry_of(c, s);
-    hipError_t e = launch_fill_u32(&c->counters[slot], 0u, 1u, st);
+    hipError_t e = cleared ? hipSuccess : launch_fill_u32(&c->counters[slot], 0u, 1u, st);
     if (e == hipSuccess)
         e = launch_build_general_list(sg.dyn_prev, sg.dyn_cur, c->g.tiles, c->general_list[slot], &c->counters[slot],
                                       st);
@@ -988,9 +999,9 @@ bf_status bf_create(const bf_config* cfg, bf_context** out) {
         return BF_ERROR_DEVICE_UNAVAILABLE;
     }
     for (int i = 0; i < 2; ++i) {
-        if (hipEventCreateWithFlags(&c->ev_fast[i], hipEventDisableTiming) != hipSuccess ||
-            hipEventCreateWithFlags(&c->ev_ready[i], hipEventDisableTiming) != hipSuccess ||
-            hipEventCreateWithFlags(&c->ev_general[i], hipEventDisableTiming) != hipSuccess) {
+        if (hipEventCreateWithFlags(&c->ev_fast[i], STREAM_EVENT) != hipSuccess ||
+            hipEventCreateWithFlags(&c->ev_ready[i], STREAM_EVENT) != hipSuccess ||
+            hipEventCreateWithFlags(&c->ev_general[i], STREAM_EVENT) != hipSuccess) {
             bf_destroy(c);
             return BF_ERROR_DEVICE_UNAVAILABLE;
         }
@@ -2033,7 +2044,7 @@ static bf_status step_static(bf_context* c, uint32_t steps) {
         const bool differs = c->static_prev_differs;   // the first step after bf_set_geometry with another mask
         const int slot = differs ? 0 : 1;
         if (differs || !c->static_list_ready) {
-            if (bf_status r = enqueue_tile_list(c, s, slot, c->sa)) return r;
+            if (bf_status r = enqueue_tile_list(c, s, slot, false, c->sa)) return r;
             if (!differs) c->static_list_ready = true;
         }
         hipEvent_t* pe = nullptr;
@@ -2090,14 +2101,22 @@ bf_status bf_step(bf_context* c, uint32_t steps) {
     // step of this call; event L of that step then releases its fluid launch.
     {
         const int64_t s = c->step + 1;
-        if (c->source != BF_GEOMETRY_STATIC && c->geometry_ready < s) {
+        const bool dynamic = c->source != BF_GEOMETRY_STATIC;
+        // both are there from the previous call unless something else moved
+        // the geometry or the step since
+        const bool built = dynamic && c->geometry_ready >= s && c->list_step == s;
+        const bool build = dynamic && c->geometry_ready < s;
+        if (build) {
             if (bf_status r = enqueue_geometry(c, s, false, false)) return r;
         }
         c->static_list_ready = false;
-        if (bf_status r = enqueue_tile_list(c, s, par2(s), c->sb)) return r;
+        if (!built) {
+            if (bf_status r = enqueue_tile_list(c, s, par2(s), build, c->sb)) return r;
+        }
         e = hipEventRecord(c->ev_ready[par2(s)], c->sb);
         if (e != hipSuccess) return hip_fail(c, e, "event record");
         c->geometry_ready = s;
+        c->list_step = s;
     }
     for (uint32_t i = 0; i < steps; ++i) {
         const int64_t s = c->step + 1;
@@ -2150,7 +2169,7 @@ bf_status bf_step(bf_context* c, uint32_t steps) {
             if (e == hipSuccess && c->source != BF_GEOMETRY_STATIC) {
                 if (bf_status r = enqueue_geometry(c, s + 1, false, false)) return r;
             }
-            if (bf_status r = enqueue_tile_list(c, s + 1, par2(s + 1), c->sb)) return r;
+            if (bf_status r = enqueue_tile_list(c, s + 1, par2(s + 1), c->source != BF_GEOMETRY_STATIC, c->sb)) return r;
             if (split) e = hipEventRecord(pe[3], c->sb);
             return e == hipSuccess ? BF_OK : hip_fail(c, e, "geometry launch");
         };
@@ -2179,6 +2198,7 @@ bf_status bf_step(bf_context* c, uint32_t steps) {
         ++c->history_count;
         if (c->free_flight) ++c->body_history_count;
         c->geometry_ready = s + 1;
+        c->list_step = s + 1;
         if (pe) ++c->profiled;
     }
     e = hipGetLastError();
@@ -2860,6 +2880,7 @@ bf_status bf_mesh_freeze_masks(bf_context* c, const uint8_t* masks, uint32_t cou
     if (e != hipSuccess) return hip_fail(c, e, "mask replay upload", false);
     c->frozen_count = count;
     c->frozen_first = c->step;
+    c->list_step = -1;                    // the replayed mask of the next step has other tiles
     // the current step's geometry (and its copy as the previous step's)
     e = replay_mask(c, c->step, 0, mod3(c->step));
     if (e == hipSuccess) e = replay_mask(c, c->step - 1, 0, mod3(c->step - 1));

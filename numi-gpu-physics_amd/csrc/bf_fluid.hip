@@ -27,18 +27,14 @@ __global__ __launch_bounds__(256) void build_general_list(const uint8_t* __restr
 
 
 // Fixed-order sum of the per-tile partials of the tiles the general path
-// processed (flags identify them; other tiles contribute exactly zero), for a
-// batch of steps with the same flags (one grid row each).
-__global__ __launch_bounds__(256) void reduce_loads_tiles(const double* __restrict__ partials,
-                                                          const uint8_t* __restrict__ dyn_prev,
-                                                          const uint8_t* __restrict__ dyn_cur, uint32_t tiles,
-                                                          double* __restrict__ block_out, uint32_t slot0) {
+// processed (flags identify them; other tiles contribute exactly zero) over
+// one workgroup's 1024 tiles.
+__device__ __forceinline__ void sum_tiles(const double* __restrict__ partials, const uint8_t* __restrict__ dyn_prev,
+                                          const uint8_t* __restrict__ dyn_cur, uint32_t tiles, uint32_t block,
+                                          double* __restrict__ out) {
     constexpr uint32_t PER_THREAD = 4;
     double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    // row k of the grid: the k-th step of the batch, its partials in their slot
-    partials += (size_t)((slot0 + blockIdx.y) % LOAD_SLOTS) * tiles * 8;
-    block_out += (size_t)blockIdx.y * gridDim.x * 8;
-    const uint32_t base = (blockIdx.x * blockDim.x + threadIdx.x) * PER_THREAD;
+    const uint32_t base = (block * blockDim.x + threadIdx.x) * PER_THREAD;
     for (uint32_t k = 0; k < PER_THREAD; ++k) {
         const uint32_t t = base + k;
         if (t < tiles && (dyn_prev[t] | dyn_cur[t]) != 0) {
@@ -47,11 +43,35 @@ __global__ __launch_bounds__(256) void reduce_loads_tiles(const double* __restri
             v[7] = fmax(v[7], partials[(size_t)t * 8 + 7]);
         }
     }
-    block_reduce8(v, block_out + (size_t)blockIdx.x * 8);
+    block_reduce8(v, out);
 }
 
 // Adds the fast tiles' limiter activations (an integer count and a maximum,
-// exact in any order) and clears them for the step that reuses the slot.
+// exact in any order), stores the step's loads and clears the activations
+// for the step that reuses the slot.  total: in LDS, complete.
+__device__ __forceinline__ void finish_loads(const double* total, uint32_t* __restrict__ activation,
+                                             double* __restrict__ last, double* __restrict__ history) {
+    if (threadIdx.x < 8) {
+        double t = total[threadIdx.x];
+        if (threadIdx.x == 6) t += (double)activation[0];
+        if (threadIdx.x == 7) t = fmax(t, (double)__uint_as_float(activation[1]));
+        if (last) last[threadIdx.x] = t;
+        history[threadIdx.x] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) activation[threadIdx.x] = 0u;
+}
+
+// A batch of steps with the same flags, one grid row each, its partials in
+// their slot.
+__global__ __launch_bounds__(256) void reduce_loads_tiles(const double* __restrict__ partials,
+                                                          const uint8_t* __restrict__ dyn_prev,
+                                                          const uint8_t* __restrict__ dyn_cur, uint32_t tiles,
+                                                          double* __restrict__ block_out, uint32_t slot0) {
+    sum_tiles(partials + (size_t)((slot0 + blockIdx.y) % LOAD_SLOTS) * tiles * 8, dyn_prev, dyn_cur, tiles, blockIdx.x,
+              block_out + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 8);
+}
+
 __global__ __launch_bounds__(256) void reduce_loads_final(const double* __restrict__ block_out, uint32_t blocks,
                                                           uint32_t* __restrict__ activation,
                                                           double* __restrict__ last, double* __restrict__ history,
@@ -59,8 +79,6 @@ __global__ __launch_bounds__(256) void reduce_loads_final(const double* __restri
                                                           uint32_t slot0) {
     double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     block_out += (size_t)blockIdx.x * blocks * 8;
-    activation += 2 * ((slot0 + blockIdx.x) % LOAD_SLOTS);
-    history_slot = (history_slot + blockIdx.x) % history_capacity;
     for (uint32_t b = threadIdx.x; b < blocks; b += blockDim.x) {
 #pragma unroll
         for (int i = 0; i < 7; ++i) v[i] += block_out[(size_t)b * 8 + i];
@@ -68,15 +86,8 @@ __global__ __launch_bounds__(256) void reduce_loads_final(const double* __restri
     }
     __shared__ double total[8];
     block_reduce8(v, total);
-    if (threadIdx.x < 8) {
-        double t = total[threadIdx.x];
-        if (threadIdx.x == 6) t += (double)activation[0];
-        if (threadIdx.x == 7) t = fmax(t, (double)__uint_as_float(activation[1]));
-        if (blockIdx.x == gridDim.x - 1) last[threadIdx.x] = t;
-        if (history) history[(size_t)history_slot * 8 + threadIdx.x] = t;
-    }
-    __syncthreads();
-    if (threadIdx.x < 2) activation[threadIdx.x] = 0u;
+    finish_loads(total, activation + 2 * ((slot0 + blockIdx.x) % LOAD_SLOTS), blockIdx.x == gridDim.x - 1 ? last : nullptr,
+                 history + (size_t)((history_slot + blockIdx.x) % history_capacity) * 8);
 }
 
 // ---------------------------------------------------------------------------
@@ -294,11 +305,31 @@ hipError_t launch_poke_population(int storage, void* f, const Grid& g, unsigned 
     return hipGetLastError();
 }
 
+// Both in one workgroup per step, for grids of one block of tiles.
+__global__ __launch_bounds__(256) void reduce_loads_small(const double* __restrict__ partials,
+                                                          const uint8_t* __restrict__ dyn_prev,
+                                                          const uint8_t* __restrict__ dyn_cur, uint32_t tiles,
+                                                          uint32_t* __restrict__ activation,
+                                                          double* __restrict__ last, double* __restrict__ history,
+                                                          uint32_t history_slot, uint32_t history_capacity,
+                                                          uint32_t slot0) {
+    __shared__ double total[8];
+    sum_tiles(partials + (size_t)((slot0 + blockIdx.x) % LOAD_SLOTS) * tiles * 8, dyn_prev, dyn_cur, tiles, 0u, total);
+    finish_loads(total, activation + 2 * ((slot0 + blockIdx.x) % LOAD_SLOTS), blockIdx.x == gridDim.x - 1 ? last : nullptr,
+                 history + (size_t)((history_slot + blockIdx.x) % history_capacity) * 8);
+}
+
 hipError_t launch_load_reduction(const LoadBuffers& b, const StepParams& p, uint64_t step, uint32_t batch,
                                  hipStream_t s) {
     if (!p.accumulate_loads || batch == 0) return hipSuccess;
     if (batch > LOAD_SLOTS) return hipErrorInvalidValue;
     const uint32_t blocks = (p.g.tiles + 1023) / 1024, slot0 = (uint32_t)(step % LOAD_SLOTS);
+    if (blocks == 1) {
+        hipLaunchKernelGGL(reduce_loads_small, dim3(batch), dim3(256), 0, s, b.partials, b.dyn_prev, b.dyn_cur,
+                           p.g.tiles, b.activation, b.last_load, b.history, (uint32_t)(step % b.history_capacity),
+                           b.history_capacity, slot0);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(reduce_loads_tiles, dim3(blocks, batch), dim3(256), 0, s, b.partials, b.dyn_prev, b.dyn_cur,
                        p.g.tiles, b.block_out, slot0);
     hipLaunchKernelGGL(reduce_loads_final, dim3(batch), dim3(256), 0, s, b.block_out, blocks, b.activation,

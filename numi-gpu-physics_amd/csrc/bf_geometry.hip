@@ -113,13 +113,36 @@ __device__ __forceinline__ void place_vertex(uint32_t v, const float lp[3], cons
     vel[v] = make_float4(ve[0], ve[1], ve[2], 0.0f);
 }
 
+// Flags and counts that a step's geometry starts from zero, cleared by the
+// first kernel of its chain (a launch of its own for each cost 4 - 6 us of the
+// chain, and the chain is the step where the fluid is the shorter of the two).
+struct ChainClear {
+    uint8_t* tiles_new;          // [tiles], or null
+    uint8_t* dyn;                // [tiles], or null
+    uint32_t* list_count;
+    uint32_t* general_count;
+    uint32_t tiles;
+};
+__device__ __forceinline__ void chain_clear(const ChainClear& c, uint32_t i) {
+    if (i < c.tiles) {
+        if (c.tiles_new) c.tiles_new[i] = 0;
+        if (c.dyn) c.dyn[i] = 0;
+    }
+    if (i == 0) {
+        if (c.list_count) *c.list_count = 0u;
+        if (c.general_count) *c.general_count = 0u;
+    }
+}
+__global__ void clear_tiles(ChainClear c) { chain_clear(c, blockIdx.x * blockDim.x + threadIdx.x); }
+
 // Vertex positions and lattice velocities at the query time
 // (BirdFlow.metal:1589-1622): frames interpolated, velocity from the frame
 // difference.
 __global__ void mesh_prepare(const float* __restrict__ points, const float* __restrict__ times,
                              float4* __restrict__ pos, float4* __restrict__ vel, const double* __restrict__ body,
-                             MeshParams m) {
+                             MeshParams m, ChainClear clear) {
     const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+    chain_clear(clear, v);
     if (v >= m.vertex_count) return;
     const uint32_t first = min(m.first, m.frame_count - 2u);
     const uint32_t second = first + 1u;
@@ -139,7 +162,7 @@ struct Kinematics;
 __global__ void articulated_prepare(const float* __restrict__ rest, const uint8_t* __restrict__ vertex_joint,
                                     const float* __restrict__ span_fraction, const Kinematics* __restrict__ kin,
                                     float4* __restrict__ pos, float4* __restrict__ vel,
-                                    const double* __restrict__ body, MeshParams m);
+                                    const double* __restrict__ body, MeshParams m, ChainClear clear);
 
 __global__ void fill_u8(uint8_t* __restrict__ p, uint8_t v, uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -470,6 +493,17 @@ __device__ inline void mark_tiles(const Grid& g, const int periodic[3], uint8_t*
                     + (uint32_t)txs[i]] = 1;
 }
 
+// Appends the flagged lanes' tiles to a list, one atomic per wavefront.
+__device__ __forceinline__ void list_tile(bool flagged, uint32_t t, uint32_t* __restrict__ list,
+                                          uint32_t* __restrict__ count) {
+    const unsigned long long b = __ballot(flagged);
+    if (b == 0) return;
+    uint32_t base = 0;
+    if (lane_rank(b) == 0 && flagged) base = atomicAdd(count, (uint32_t)__popcll(b));
+    base = __shfl(base, __ffsll(b) - 1, 64);
+    if (flagged) list[base + lane_rank(b)] = t;
+}
+
 // Tiles the geometry pass visits this step: keyed now, or holding mask /
 // wall entries written by the steps that last used those buffers.
 __global__ __launch_bounds__(256) void geometry_tile_list(const uint8_t* __restrict__ tiles_new,
@@ -477,13 +511,7 @@ __global__ __launch_bounds__(256) void geometry_tile_list(const uint8_t* __restr
                                                           const uint8_t* __restrict__ tiles_wall_old, uint32_t tiles,
                                                           uint32_t* __restrict__ list, uint32_t* __restrict__ count) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool flagged = t < tiles && (tiles_new[t] | tiles_mask_old[t] | tiles_wall_old[t]) != 0;
-    const unsigned long long b = __ballot(flagged);
-    if (b == 0) return;
-    uint32_t base = 0;
-    if ((threadIdx.x & 63) == 0) base = atomicAdd(count, (uint32_t)__popcll(b));
-    base = __shfl(base, 0, 64);
-    if (flagged) list[base + lane_rank(b)] = t;
+    list_tile(t < tiles && (tiles_new[t] | tiles_mask_old[t] | tiles_wall_old[t]) != 0, t, list, count);
 }
 
 // BirdFlow.metal:1697-1738 on the listed tiles.  In a tile keyed this step
@@ -639,13 +667,19 @@ __global__ void link_census(const uint8_t* __restrict__ prev, const uint8_t* __r
 // Host launchers.
 // ---------------------------------------------------------------------------
 
-hipError_t launch_mesh_prepare(const MeshBuffers& b, const MeshParams& m, hipStream_t s) {
+// The vertex pass, which also clears what `clear` names.
+static void prepare_vertices(const MeshBuffers& b, const MeshParams& m, const ChainClear& clear, hipStream_t s) {
+    const uint32_t blocks = (std::max(m.vertex_count, clear.tiles) + 255) / 256;
     if (b.kinematics)
-        hipLaunchKernelGGL(articulated_prepare, dim3((m.vertex_count + 255) / 256), dim3(256), 0, s, b.rest,
-                           b.vertex_joint, b.span_fraction, b.kinematics, b.pos, b.vel, b.body, m);
+        hipLaunchKernelGGL(articulated_prepare, dim3(blocks), dim3(256), 0, s, b.rest, b.vertex_joint, b.span_fraction,
+                           b.kinematics, b.pos, b.vel, b.body, m, clear);
     else
-        hipLaunchKernelGGL(mesh_prepare, dim3((m.vertex_count + 255) / 256), dim3(256), 0, s, b.points, b.times,
-                           b.pos, b.vel, b.body, m);
+        hipLaunchKernelGGL(mesh_prepare, dim3(blocks), dim3(256), 0, s, b.points, b.times, b.pos, b.vel, b.body, m,
+                           clear);
+}
+
+hipError_t launch_mesh_prepare(const MeshBuffers& b, const MeshParams& m, hipStream_t s) {
+    prepare_vertices(b, m, ChainClear{}, s);
     return hipGetLastError();
 }
 
@@ -820,8 +854,10 @@ __device__ inline void measured_angles(const float* __restrict__ kf, int count, 
 // (world angular velocity, geometry radius), then left and right wing
 // (root, chord, span, normal, angular velocity).
 __global__ void bird_prepare(BirdShape b, const double* __restrict__ body, const float* __restrict__ keyframes,
-                             int keyframe_count, float time, float dx, float4* __restrict__ frame) {
+                             int keyframe_count, float time, float dx, float4* __restrict__ frame,
+                             ChainClear clear) {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
+    chain_clear(clear, 0);
     const V3 pos = v3((float)body[0], (float)body[1], (float)body[2]);
     Quat q = {(float)body[3], (float)body[4], (float)body[5], (float)body[6]};
     const float n2 = q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w;
@@ -888,10 +924,15 @@ __device__ inline float tile_box_dist2(float lx, float hx, float ly, float hy, f
 // span plus sweep, half the largest chord and half the thickness), so every
 // cell that can be solid lies in one; and, with a previous geometry, the
 // tiles near last step's solid cells (evaluated even beyond the radius, as
-// the reference does).  Every tile's flag is written.
+// the reference does).  Every tile's flag is written, its solid-proximity
+// flag cleared, and the tiles the tile pass visits are listed.
 __global__ __launch_bounds__(256) void bird_mark_tiles(BirdShape b, const float4* __restrict__ frame,
                                                        const uint8_t* __restrict__ dyn_prev,
-                                                       uint8_t* __restrict__ tiles_new, BirdParams p) {
+                                                       uint8_t* __restrict__ tiles_new,
+                                                       const uint8_t* __restrict__ tiles_mask_old,
+                                                       const uint8_t* __restrict__ tiles_wall_old,
+                                                       uint8_t* __restrict__ dyn, uint32_t* __restrict__ list,
+                                                       uint32_t* __restrict__ count, BirdParams p) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= p.g.tiles) return;
     int x0, y0, z;
@@ -921,7 +962,10 @@ __global__ __launch_bounds__(256) void bird_mark_tiles(BirdShape b, const float4
         const V3 wc = vadd(row3(frame[4 + 5 * wing]), vmul(row3(frame[6 + 5 * wing]), 0.5f * b.wing_span));
         hit = hit || tile_box_dist2(lx, hx, ly, hy, zc, wc.x, wc.y, wc.z) <= rw * rw;
     }
-    tiles_new[t] = (hit || (dyn_prev && dyn_prev[t])) ? 1 : 0;
+    const bool marked = hit || (dyn_prev && dyn_prev[t]);
+    tiles_new[t] = marked ? 1 : 0;
+    dyn[t] = 0;
+    list_tile(marked || tiles_mask_old[t] != 0 || tiles_wall_old[t] != 0, t, list, count);
 }
 
 // buildBirdGeometry on the tiles marked this step: every cell gets the
@@ -1059,17 +1103,14 @@ __global__ void wing_inertial_reaction(const float4* __restrict__ frame, WingDyn
 hipError_t launch_bird_geometry(const BirdShape& shape, const BirdBuffers& b, const BirdParams& p, hipStream_t s,
                                 const WingDynamics* wing_dynamics) {
     const unsigned tile_blocks = (p.g.tiles + 255) / 256;
+    const ChainClear counts{nullptr, nullptr, b.list_count, b.general_count, 0u};
     hipLaunchKernelGGL(bird_prepare, dim3(1), dim3(64), 0, s, shape, b.body, b.keyframes, (int)b.keyframe_count,
-                       p.time, p.dx, b.frame);
+                       p.time, p.dx, b.frame, counts);
     if (wing_dynamics && b.wing_momentum && b.wing_reaction)
         hipLaunchKernelGGL(wing_inertial_reaction, dim3(1), dim3(64), 0, s, (const float4*)b.frame, *wing_dynamics,
                            b.wing_momentum, b.wing_reaction);
     hipLaunchKernelGGL(bird_mark_tiles, dim3(tile_blocks), dim3(256), 0, s, shape, (const float4*)b.frame,
-                       b.dyn_prev, b.tiles_new, p);
-    hipLaunchKernelGGL(fill_u8, dim3(tile_blocks), dim3(256), 0, s, b.dyn, (uint8_t)0, p.g.tiles);
-    hipLaunchKernelGGL(fill_u32, dim3(1), dim3(64), 0, s, b.list_count, 0u, 1u);
-    hipLaunchKernelGGL(geometry_tile_list, dim3(tile_blocks), dim3(256), 0, s, b.tiles_new, b.tiles_mask_old,
-                       b.tiles_wall_old, p.g.tiles, b.list, b.list_count);
+                       b.dyn_prev, b.tiles_new, b.tiles_mask_old, b.tiles_wall_old, b.dyn, b.list, b.list_count, p);
     hipLaunchKernelGGL(bird_tile_pass, dim3(p.tile_pass_blocks), dim3(256), 0, s, shape, (const float4*)b.frame,
                        b.list, b.list_count, (const uint8_t*)b.tiles_new, b.mask_prev, b.mask, b.wall, b.dyn, p);
     return hipGetLastError();
@@ -1207,8 +1248,9 @@ __device__ inline float wing_violation(const WingShape& w, const float4* f, floa
 
 }  // namespace
 
-__global__ void wing_prepare(WingShape w, float time, float4* __restrict__ frame) {
+__global__ void wing_prepare(WingShape w, float time, float4* __restrict__ frame, ChainClear clear) {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
+    chain_clear(clear, 0);
     const float a = time / w.cycle;
     float phase = a - truncf(a);
     phase = phase < 0.0f ? phase + 1.0f : phase;
@@ -1236,7 +1278,11 @@ __global__ void wing_prepare(WingShape w, float time, float4* __restrict__ frame
 // span + 1.5 mean chords + 2 cells), or near last step's solid cells.
 __global__ __launch_bounds__(256) void wing_mark_tiles(WingShape w, const float4* __restrict__ frame,
                                                        const uint8_t* __restrict__ dyn_prev,
-                                                       uint8_t* __restrict__ tiles_new, BirdParams p) {
+                                                       uint8_t* __restrict__ tiles_new,
+                                                       const uint8_t* __restrict__ tiles_mask_old,
+                                                       const uint8_t* __restrict__ tiles_wall_old,
+                                                       uint8_t* __restrict__ dyn, uint32_t* __restrict__ list,
+                                                       uint32_t* __restrict__ count, BirdParams p) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= p.g.tiles) return;
     int x0, y0, z;
@@ -1273,7 +1319,10 @@ __global__ __launch_bounds__(256) void wing_mark_tiles(WingShape w, const float4
         const float r = w.radius + 1.5f * c.w + 2.0f * p.dx + 2.0f * p.dx;
         hit = tile_box_dist2(lx, hx, ly, hy, zc, c.x, c.y, c.z) <= r * r;
     }
-    tiles_new[t] = (hit || (dyn_prev && dyn_prev[t])) ? 1 : 0;
+    const bool marked = hit || (dyn_prev && dyn_prev[t]);
+    tiles_new[t] = marked ? 1 : 0;
+    dyn[t] = 0;
+    list_tile(marked || tiles_mask_old[t] != 0 || tiles_wall_old[t] != 0, t, list, count);
 }
 
 // buildPrescribedFlappingWing on the marked tiles (every cell the
@@ -1360,29 +1409,59 @@ __global__ __launch_bounds__(256) void wing_links(WingShape w, const float4* __r
     __shared__ float4 fr[WING_FRAME_ROWS];
     if (threadIdx.x < WING_FRAME_ROWS) fr[threadIdx.x] = frame[threadIdx.x];
     __syncthreads();
+    // A tile's links are queued in LDS first, then spread over the lanes: the
+    // links of a tile crowd into a few cells, and a bisection (ten violation
+    // functions with a power each) in each cell's own loop over its links ran
+    // up to 18 of them in a row with most lanes idle (160x160x128, 16 cells per
+    // chord, beside the fluid: 80 us; queued 25).
+    __shared__ uint16_t queue[18 * TILE_CELLS];
+    __shared__ uint32_t queued;
     // Tiles with wing cells or their neighbours (dyn) are marked tiles, so
     // they are on the step's geometry list.
     const uint32_t n_tiles = *count;
     for (uint32_t i = blockIdx.x; i < n_tiles; i += gridDim.x) {
         const uint32_t tile = list[i];
-        if (!dyn[tile]) continue;
+        if (!dyn[tile]) continue;                    // the same for the whole workgroup
         int x0, y0, z;
         tile_origin(p.g, tile, x0, y0, z);
-        const int x = x0 + (int)(threadIdx.x & (TILE_X - 1));
-        const int y = y0 + (int)(threadIdx.x / TILE_X);
-        if (x >= p.g.nx || y >= p.g.ny) continue;
-        const uint32_t gid = (uint32_t)x + (uint32_t)p.g.nx * ((uint32_t)y + (uint32_t)p.g.ny * (uint32_t)z);
-        if (mask[gid] != 0) continue;
-        float* out = links + (size_t)tile * 19 * TILE_CELLS + threadIdx.x;
-        for (int q = 1; q < 19; ++q) {
-            // the source the fluid kernel pulls from: wrapped across a
-            // periodic face, clamped at an outlet, none beyond a far field
+        // the source the fluid kernel pulls direction q of cell (cx, cy) from:
+        // wrapped across a periodic face, clamped at an outlet, none beyond a
+        // far field
+        auto source = [&](int px, int py, int q, int& sx, int& sy, int& sz) {
+            return link_source(p.bc[0], px - cx(q), p.g.nx, sx) && link_source(p.bc[1], py - cy(q), p.g.ny, sy) &&
+                   link_source(p.bc[2], z - cz(q), p.g.nz, sz);
+        };
+        if (threadIdx.x == 0) queued = 0u;
+        __syncthreads();
+        {
+            const int x = x0 + (int)(threadIdx.x & (TILE_X - 1));
+            const int y = y0 + (int)(threadIdx.x / TILE_X);
+            const bool in_grid = x < p.g.nx && y < p.g.ny;
+            const uint32_t gid = (uint32_t)x + (uint32_t)p.g.nx * ((uint32_t)y + (uint32_t)p.g.ny * (uint32_t)z);
+            if (in_grid && mask[gid] == 0) {
+                uint32_t links_of = 0;
+#pragma unroll
+                for (int q = 1; q < 19; ++q) {
+                    int sx, sy, sz;
+                    const bool has = source(x, y, q, sx, sy, sz);
+                    const uint32_t src = has ? (uint32_t)sx + (uint32_t)p.g.nx * ((uint32_t)sy + (uint32_t)p.g.ny * (uint32_t)sz)
+                                             : gid;
+                    links_of |= (uint32_t)(has && mask[src] != 0) << q;
+                }
+                if (links_of) {
+                    uint32_t at = atomicAdd(&queued, (uint32_t)__popc(links_of));
+                    for (; links_of; links_of &= links_of - 1)
+                        queue[at++] = (uint16_t)(threadIdx.x | (uint32_t)(__ffs(links_of) - 1) << 8);
+                }
+            }
+        }
+        __syncthreads();
+        float* out = links + (size_t)tile * 19 * TILE_CELLS;
+        for (uint32_t k = threadIdx.x; k < queued; k += blockDim.x) {
+            const int lane = queue[k] & 255, q = queue[k] >> 8;
+            const int x = x0 + (lane & (TILE_X - 1)), y = y0 + lane / TILE_X;
             int sx, sy, sz;
-            if (!link_source(p.bc[0], x - cx(q), p.g.nx, sx) || !link_source(p.bc[1], y - cy(q), p.g.ny, sy) ||
-                !link_source(p.bc[2], z - cz(q), p.g.nz, sz))
-                continue;
-            const uint32_t src = (uint32_t)sx + (uint32_t)p.g.nx * ((uint32_t)sy + (uint32_t)p.g.ny * (uint32_t)sz);
-            if (mask[src] == 0) continue;
+            (void)source(x, y, q, sx, sy, sz);
             const V3 solid = v3(p.origin[0] + ((float)sx + 0.5f) * p.dx, p.origin[1] + ((float)sy + 0.5f) * p.dx,
                                 p.origin[2] + ((float)sz + 0.5f) * p.dx);
             const V3 fluid = v3(solid.x + (float)cx(q) * p.dx, solid.y + (float)cy(q) * p.dx,
@@ -1395,20 +1474,18 @@ __global__ __launch_bounds__(256) void wing_links(WingShape w, const float4* __r
                 if (wing_violation(w, fr, p.dx, sample) > 0.0f) lower = mid;
                 else upper = mid;
             }
-            out[(size_t)q * TILE_CELLS] = smin(smax(0.5f * (lower + upper), 1.0e-4f), 1.0f);
+            out[(size_t)q * TILE_CELLS + lane] = smin(smax(0.5f * (lower + upper), 1.0e-4f), 1.0f);
         }
+        __syncthreads();
     }
 }
 
 hipError_t launch_wing_geometry(const WingShape& shape, const WingBuffers& b, const BirdParams& p, hipStream_t s) {
     const unsigned tile_blocks = (p.g.tiles + 255) / 256;
-    hipLaunchKernelGGL(wing_prepare, dim3(1), dim3(64), 0, s, shape, p.time, b.frame);
+    const ChainClear counts{nullptr, nullptr, b.list_count, b.general_count, 0u};
+    hipLaunchKernelGGL(wing_prepare, dim3(1), dim3(64), 0, s, shape, p.time, b.frame, counts);
     hipLaunchKernelGGL(wing_mark_tiles, dim3(tile_blocks), dim3(256), 0, s, shape, (const float4*)b.frame, b.dyn_prev,
-                       b.tiles_new, p);
-    hipLaunchKernelGGL(fill_u8, dim3(tile_blocks), dim3(256), 0, s, b.dyn, (uint8_t)0, p.g.tiles);
-    hipLaunchKernelGGL(fill_u32, dim3(1), dim3(64), 0, s, b.list_count, 0u, 1u);
-    hipLaunchKernelGGL(geometry_tile_list, dim3(tile_blocks), dim3(256), 0, s, b.tiles_new, b.tiles_mask_old,
-                       b.tiles_wall_old, p.g.tiles, b.list, b.list_count);
+                       b.tiles_new, b.tiles_mask_old, b.tiles_wall_old, b.dyn, b.list, b.list_count, p);
     hipLaunchKernelGGL(wing_tile_pass, dim3(p.tile_pass_blocks), dim3(256), 0, s, shape, (const float4*)b.frame,
                        b.list, b.list_count, (const uint8_t*)b.tiles_new, b.mask_prev, b.mask, b.wall, b.dyn, p);
     hipLaunchKernelGGL(wing_links, dim3(p.tile_pass_blocks), dim3(256), 0, s, shape, (const float4*)b.frame,
@@ -1422,13 +1499,7 @@ hipError_t launch_mesh_static_keys(const MeshBuffers& b, const MeshParams& m, un
     if (m.g.nx > 65535 || m.g.ny > 65535) return hipErrorInvalidValue;   // raster packs x | y << 16
     if (m.raster_batch < 1 || m.raster_batch > 64 || m.raster_blocks < 1 || m.raster_split < 1 || m.raster_split > 64)
         return hipErrorInvalidValue;
-    if (b.kinematics)
-        hipLaunchKernelGGL(articulated_prepare, dim3((m.vertex_count + 255) / 256), dim3(256), 0, s, b.rest,
-                           b.vertex_joint, b.span_fraction, b.kinematics, b.pos, b.vel, b.body, m);
-    else
-        hipLaunchKernelGGL(mesh_prepare, dim3((m.vertex_count + 255) / 256), dim3(256), 0, s, b.points, b.times,
-                           b.pos, b.vel, b.body, m);
-    hipLaunchKernelGGL(fill_u8, dim3((m.g.tiles + 255) / 256), dim3(256), 0, s, b.tiles_new, (uint8_t)0, m.g.tiles);
+    prepare_vertices(b, m, ChainClear{b.tiles_new, nullptr, nullptr, nullptr, m.g.tiles}, s);
     if (m.raster_count > 0)
         hipLaunchKernelGGL(mesh_raster, dim3(std::min((m.raster_count + m.raster_batch - 1) / m.raster_batch, m.raster_blocks), m.raster_split), dim3(64), 0, s, b.pos,
                            b.tri, b.raster_list, b.keys, b.tiles_new, m);
@@ -1468,8 +1539,9 @@ __device__ __forceinline__ void kin_series(const float (&c)[4][2], uint32_t harm
 __global__ void articulated_prepare(const float* __restrict__ rest, const uint8_t* __restrict__ vertex_joint,
                                     const float* __restrict__ span_fraction, const Kinematics* __restrict__ kin,
                                     float4* __restrict__ pos, float4* __restrict__ vel,
-                                    const double* __restrict__ body, MeshParams m) {
+                                    const double* __restrict__ body, MeshParams m, ChainClear clear) {
     const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+    chain_clear(clear, v);
     if (v >= m.vertex_count) return;
     const Kinematics& k = *kin;
     const float* r = rest + 3 * (size_t)v;
@@ -1527,15 +1599,7 @@ hipError_t launch_mesh_geometry(const MeshBuffers& b, const MeshParams& m, hipSt
     if (m.g.nx > 65535 || m.g.ny > 65535) return hipErrorInvalidValue;   // raster packs x | y << 16
     if (m.raster_batch < 1 || m.raster_batch > 64 || m.raster_blocks < 1 || m.raster_split < 1 || m.raster_split > 64)
         return hipErrorInvalidValue;
-    if (b.kinematics)
-        hipLaunchKernelGGL(articulated_prepare, dim3((m.vertex_count + 255) / 256), dim3(256), 0, s, b.rest,
-                           b.vertex_joint, b.span_fraction, b.kinematics, b.pos, b.vel, b.body, m);
-    else
-        hipLaunchKernelGGL(mesh_prepare, dim3((m.vertex_count + 255) / 256), dim3(256), 0, s, b.points, b.times,
-                           b.pos, b.vel, b.body, m);
-    hipLaunchKernelGGL(fill_u8, dim3((m.g.tiles + 255) / 256), dim3(256), 0, s, b.tiles_new, (uint8_t)0, m.g.tiles);
-    hipLaunchKernelGGL(fill_u8, dim3((m.g.tiles + 255) / 256), dim3(256), 0, s, b.dyn, (uint8_t)0, m.g.tiles);
-    hipLaunchKernelGGL(fill_u32, dim3(1), dim3(64), 0, s, b.list_count, 0u, 1u);
+    prepare_vertices(b, m, ChainClear{b.tiles_new, b.dyn, b.list_count, b.general_count, m.g.tiles}, s);
     if (b.seed_count > 0)
         hipLaunchKernelGGL(seed_keys, dim3((b.seed_count + 255) / 256), dim3(256), 0, s, b.seed_cells, b.seed_keys,
                            b.seed_count, b.keys, b.tiles_new, m.g);
@@ -1551,8 +1615,9 @@ hipError_t launch_mesh_geometry(const MeshBuffers& b, const MeshParams& m, hipSt
 }
 
 hipError_t launch_sphere_geometry(uint8_t* mask, float4* wall, uint8_t* dyn, const Grid& g, float4 cr, float3 gv,
-                                  float4 wv, float t, const int periodic[3], hipStream_t s) {
-    hipLaunchKernelGGL(fill_u8, dim3((g.tiles + 255) / 256), dim3(256), 0, s, dyn, (uint8_t)0, g.tiles);
+                                  float4 wv, float t, const int periodic[3], uint32_t* general_count, hipStream_t s) {
+    hipLaunchKernelGGL(clear_tiles, dim3((g.tiles + 255) / 256), dim3(256), 0, s,
+                       ChainClear{nullptr, dyn, nullptr, general_count, g.tiles});
     hipLaunchKernelGGL(sphere_geometry, dim3((g.n + 255) / 256), dim3(256), 0, s, mask, wall, dyn, g, cr, gv, wv, t,
                        periodic[0], periodic[1], periodic[2]);
     return hipGetLastError();

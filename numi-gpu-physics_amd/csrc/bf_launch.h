@@ -124,6 +124,7 @@ struct BirdBuffers {
     const uint8_t* tiles_wall_old;    // tiles whose `wall` entries an earlier step wrote
     uint32_t* list;                   // scratch: tiles visited by the tile pass
     uint32_t* list_count;
+    uint32_t* general_count;          // length of the step's wall-tile list, cleared here (not built)
     uint8_t* mask;
     float4* wall;
     uint8_t* dyn;
@@ -152,6 +153,7 @@ struct WingBuffers {
     const uint8_t* tiles_wall_old;
     uint32_t* list;
     uint32_t* list_count;
+    uint32_t* general_count;
     uint8_t* mask;
     float4* wall;
     uint8_t* dyn;
@@ -197,6 +199,7 @@ struct MeshBuffers {
     const uint8_t* tiles_wall_old;      // tiles whose `wall` entries an earlier step wrote
     uint32_t* list;                     // scratch: tiles visited by the tile pass
     uint32_t* list_count;
+    uint32_t* general_count;            // optional: length of the step's wall-tile list, cleared here
     uint8_t* mask;
     float4* wall;
     uint8_t* dyn;
@@ -426,7 +429,7 @@ hipError_t launch_bird_geometry(const BirdShape& shape, const BirdBuffers& b, co
                                 const WingDynamics* wing_dynamics = nullptr);
 hipError_t launch_wing_geometry(const WingShape& shape, const WingBuffers& b, const BirdParams& p, hipStream_t s);
 hipError_t launch_sphere_geometry(uint8_t* mask, float4* wall, uint8_t* dyn, const Grid& g, float4 cr, float3 gv,
-                                  float4 wv, float t, const int periodic[3], hipStream_t s);
+                                  float4 wv, float t, const int periodic[3], uint32_t* general_count, hipStream_t s);
 hipError_t launch_mark_tiles(const uint8_t* mask, uint8_t* dyn, const Grid& g, const int periodic[3], bool clear,
                              hipStream_t s);
 hipError_t launch_fill_u8(uint8_t* p, uint8_t v, uint32_t n, hipStream_t s);
