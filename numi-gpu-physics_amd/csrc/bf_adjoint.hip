@@ -126,9 +126,80 @@ __device__ __forceinline__ bool unpulled(const Sources& s, const StepParams& p, 
 // ---------------------------------------------------------------------------
 // Wall-free tiles.
 // ---------------------------------------------------------------------------
-// At least 4 wavefronts per SIMD (128 VGPRs): the RR3 instance spills 22
-// registers to scratch there and still runs 3 % faster than at its natural
-// 140 VGPRs and 3 wavefronts (193 against 200 us at 256 x 128 x 128).
+// A wavefront is one row of the tile: its y, z and source rows are uniform, so
+// the 57 accesses of a cell take their bases from scalar registers and three
+// 32-bit offsets (x and its two neighbours), and the face tests other than x
+// are scalar branches.  With the limiter's share kept in scalars (reverse in
+// bf_adjoint_math.h) the RR3 instance takes 111 VGPRs and 1880 vector
+// instructions, where it took 3090 and spilled 22 of 128.  It is bound by
+// memory all the same: 228 bytes per cell, 195 us per step at 256 x 128 x 128
+// (4.9 TB/s; 197 before).  Plain stores: lambda is the next reverse step's
+// input, and streaming stores take 207 us.
+template <int COLL, int S>
+__device__ __forceinline__ void fast_cell(const AdjointBuffers& b, const StepParams& p, int x, int y, int z) {
+    using T = typename Store<S>::T;
+    const Grid& g = p.g;
+    const uint32_t row = (uint32_t)y + (uint32_t)g.ny * (uint32_t)z;
+    Sources s = sources(p, x, y, z);
+    // a source beyond a far-field face reads an in-domain cell, and is replaced
+    if (s.xm_far) s.xs_p = x;
+    if (s.xp_far) s.xs_m = x;
+    const bool faces = s.ym_far || s.yp_far || s.zm_far || s.zp_far || __any(s.xm_far || s.xp_far) ||
+                       ((p.bc[0][0] == BC_OUTLET || p.bc[0][1] == BC_OUTLET) && __any(x == 0 || x == g.nx - 1));
+    float gq[19], lp[19], mu[19];
+    for_q(AllQ{}, [&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        int xs;
+        uint32_t rows;
+        bool far;
+        source_xr<q>(s, g, x, y, z, xs, rows, far);
+        const bool row_far = (cy(q) > 0 && s.ym_far) || (cy(q) < 0 && s.yp_far) || (cz(q) > 0 && s.zm_far) ||
+                             (cz(q) < 0 && s.zp_far);
+        gq[q] = Store<S>::load(row_ptr<S>((const T*)b.f_prev, g, q, row_far ? row : rows), xs, q);
+        lp[q] = *row_at(row_ptr<STORE_FP32>(b.lam_in, g, q, row), x);
+    });
+    if (faces) {
+        for_q(AllQ{}, [&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            int xs;
+            uint32_t rows;
+            bool far;
+            source_xr<q>(s, g, x, y, z, xs, rows, far);
+            if (far) gq[q] = p.far_eq[q];
+        });
+    }
+    // the sponge blend f_out = post + (f_far - post) s scales the adjoint by 1 - s
+    if (p.sponge_strength > 0.0f) {
+        const float keep = 1.0f - sponge_factor(p, x, y, z);
+        for_q(AllQ{}, [&](auto qc) { lp[decltype(qc)::value] *= keep; });
+    }
+    collision_adjoint<COLL>(gq, p.omega_plus, p.omega_minus, lp, mu);
+    // the store addresses are the load addresses: recomputed, not kept live
+    // across the collision
+    asm volatile("" : "+v"(x), "+v"(s.xs_p), "+v"(s.xs_m), "+s"(y), "+s"(z), "+s"(s.ys_p), "+s"(s.ys_m),
+                 "+s"(s.zs_p), "+s"(s.zs_m));
+    if (faces) {
+        for_q(AllQ{}, [&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            int xs;
+            uint32_t rows;
+            bool far;
+            source_xr<q>(s, g, x, y, z, xs, rows, far);
+            write_pull<q>(b, p, x, y, z, xs, rows, far, mu[q]);
+            if (unpulled<q>(s, p, x)) b.lam_out[lam_at(g, q, x, row)] = 0.0f;
+        });
+        return;
+    }
+    for_q(AllQ{}, [&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        int xs;
+        uint32_t rows;
+        bool far;
+        source_xr<q>(s, g, x, y, z, xs, rows, far);
+        *row_at(row_ptr<STORE_FP32>(b.lam_out, g, q, rows), xs) = mu[q];
+    });
+}
+
 template <int COLL, int S>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void adjoint_fast(AdjointBuffers b,
                                                                                            StepParams p) {
@@ -137,48 +208,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void a
     int x0, y0, z;
     tile_origin(p.g, tile, x0, y0, z);
     const int x = x0 + (int)(threadIdx.x & (TILE_X - 1));
-    const int y = y0 + (int)(threadIdx.x / TILE_X);
-    if (x >= p.g.nx || y >= p.g.ny) return;   // lanes of a partial tile beyond the grid
-    const uint32_t row = (uint32_t)y + (uint32_t)p.g.ny * (uint32_t)z;
-    const Sources s = sources(p, x, y, z);
-    // the sponge blend f_out = post + (f_far - post) s scales the adjoint by 1 - s
-    const float keep = 1.0f - (p.sponge_strength > 0.0f ? sponge_factor(p, x, y, z) : 0.0f);
-    float g[19], lp[19], mu[19];
-    for_q(AllQ{}, [&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        int xs;
-        uint32_t rows;
-        bool far;
-        source_xr<q>(s, p.g, x, y, z, xs, rows, far);
-        // unconditional load (a far-field source reads this cell)
-        const float v = fprev<S>(b, far ? pop_index<S>(p.g, q, x, row) : pop_index<S>(p.g, q, xs, rows), q);
-        g[q] = far ? p.far_eq[q] : v;
-        lp[q] = b.lam_in[lam_at(p.g, q, x, row)] * keep;
-    });
-    collision_adjoint<COLL>(g, p.omega_plus, p.omega_minus, lp, mu);
-    // The sources again, from coordinates the compiler cannot match with the
-    // ones above: otherwise it keeps the 19 load addresses (the store
-    // addresses are the same numbers) live across the collision, 38 VGPRs.
-    int xr = x, yr = y, zr = z;
-    asm volatile("" : "+v"(xr), "+v"(yr), "+v"(zr));
-    const Sources sr = sources(p, xr, yr, zr);
-    const uint32_t rowr = (uint32_t)yr + (uint32_t)p.g.ny * (uint32_t)zr;
-    for_q(AllQ{}, [&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        int xs;
-        uint32_t rows;
-        bool far;
-        source_xr<q>(sr, p.g, xr, yr, zr, xs, rows, far);
-        write_pull<q>(b, p, xr, yr, zr, xs, rows, far, mu[q]);
-        if (unpulled<q>(sr, p, xr)) b.lam_out[lam_at(p.g, q, xr, rowr)] = 0.0f;
-    });
+    const int y = y0 + (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (x < p.g.nx && y < p.g.ny) fast_cell<COLL, S>(b, p, x, y, z);   // not the lanes beyond the grid
 }
 
 // ---------------------------------------------------------------------------
 // Wall tiles, pass 1: collision adjoint and the single-writer pull targets.
 // nu (per listed tile, direction-major, 256 lanes): for a fluid cell the
 // sensitivity of J to each wall-link value (collision part plus the link's
-// own load), for a refilled cell mu.
+// own load), for a refilled cell mu.  Direction 0 has no link: for a fluid
+// cell its entry holds the link directions as bits (0 for a solid cell), which
+// is all that pass 2 reads of a cell without links.
 // ---------------------------------------------------------------------------
 template <int COLL, int S>
 __device__ __forceinline__ void general_p1_cell(const AdjointBuffers& b, const StepParams& p,
@@ -229,62 +269,90 @@ __device__ __forceinline__ void general_p1_cell(const AdjointBuffers& b, const S
         });
         return;
     }
-    const float4 wg4 = b.wall[gid];
-    const float wgv[4] = {wg4.x, wg4.y, wg4.z, wg4.w};
-    const float wx = p.origin[0] + ((float)x + 0.5f) * p.dx;
-    const float wy = p.origin[1] + ((float)y + 0.5f) * p.dx;
-    const float wz = p.origin[2] + ((float)z + 0.5f) * p.dx;
-    bool link[19];
+    // Every source's part and population together (a source beyond a
+    // far-field face reads this cell); then the links, three directions at a
+    // time, each group's loads together: a direction at a time, each behind a
+    // branch, is a round trip to memory for each (256 x 128 x 128, 280 listed
+    // tiles: 41 us; so 34).
+    uint32_t part[19];
     float load_dv[19];
     for_q(AllQ{}, [&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        link[q] = false;
         load_dv[q] = 0.0f;
-        if (far[q]) {
-            gq[q] = p.far_eq[q];
-            return;
-        }
-        const uint8_t part = b.solid_cur[src[q]];
-        if (part == 0) {
-            int xs;
-            uint32_t rows;
-            bool fq;
-            source_xr<q>(s, g, x, y, z, xs, rows, fq);
-            gq[q] = fprev<S>(b, pop_index<S>(g, q, xs, rows), q);
-            return;
-        }
-        link[q] = true;
-        const float4 ws4 = b.wall[src[q]];
-        const float wsv[4] = {ws4.x, ws4.y, ws4.z, ws4.w};
-        const int fx = x + cx(q), fy = y + cy(q), fz = z + cz(q);
-        const bool fin_ok = inside(g, fx, fy, fz);
-        const uint32_t fid = fin_ok ? flat(g, fx, fy, fz) : gid;
-        const bool farther_ok = fin_ok && b.solid_cur[fid] == 0;
-        const float refl = fprev<S>(b, pop_index<S>(g, opp(q), x, row), opp(q));
-        const float farther =
-            farther_ok ? fprev<S>(b, pop_index<S>(g, opp(q), fx, (uint32_t)fy + (uint32_t)g.ny * (uint32_t)fz), opp(q))
-                       : 0.0f;
-        const float pin = fprev<S>(b, pop_index<S>(g, q, x, row), q);
-        float tlf;
-        uint32_t win;
-        const int rule = link_rule(b, p, x, y, z, q, tlf, win);
-        const adj::LinkD<float> d = adj::link_value<float>(cx(q), cy(q), cz(q), weight<float>(q), p.far_rho, rule,
-                                                           farther_ok, refl, farther, pin, wgv, wsv, tlf);
-        gq[q] = d.value;
-        const int sel = p.selected_part;
-        if (p.accumulate_loads && p.load_component != 2 && (sel == 0 || sel == (int)part)) {
-            const float arm[3] = {wx - d.lf * (float)cx(q) * p.dx - bx, wy - d.lf * (float)cy(q) * p.dx - by,
-                                  wz - d.lf * (float)cz(q) * p.dx - bz};
-            // J_link = -fscale (value + reflected) c_q . e(arm)
-            load_dv[q] = -p.force_scale * load_weight<q>(w, arm);
-        }
+        part[q] = b.solid_cur[far[q] ? gid : src[q]];
+        gq[q] = fprev<S>(b, far[q] ? pop_index<S>(g, q, x, row) : pop_index<S>(g, q, sx[q], srow[q]), q);
     });
+    asm volatile("" : BF_ASM19(part), BF_ASM19(gq));
+    uint32_t linkbits = 0;
+    for_q(AllQ{}, [&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        if (far[q]) gq[q] = p.far_eq[q];
+        else linkbits |= (uint32_t)(part[q] != 0) << q;
+    });
+    if (linkbits != 0) {
+        const float4 wg4 = b.wall[gid];
+        const float wgv[4] = {wg4.x, wg4.y, wg4.z, wg4.w};
+        const float wx = p.origin[0] + ((float)x + 0.5f) * p.dx;
+        const float wy = p.origin[1] + ((float)y + 0.5f) * p.dx;
+        const float wz = p.origin[2] + ((float)z + 0.5f) * p.dx;
+        auto link_group = [&](auto seq, auto first_c, uint32_t gmask) {
+            constexpr int q0 = decltype(first_c)::value;
+            if (!(linkbits & gmask)) return;
+            float4 ws[3];
+            float refl[3], fo[3], pin[3];
+            uint32_t fpart[3];
+            for_q(seq, [&](auto qc) {
+                constexpr int q = decltype(qc)::value, j = q - q0;
+                const bool lk = (linkbits >> q) & 1u;
+                const int fx = x + cx(q), fy = y + cy(q), fz = z + cz(q);
+                // (a far side outside the domain reads this cell, then counts as solid)
+                const bool in = lk && inside(g, fx, fy, fz);
+                ws[j] = b.wall[lk ? src[q] : gid];
+                fpart[j] = (uint32_t)b.solid_cur[in ? flat(g, fx, fy, fz) : gid] | (in ? 0u : 256u);
+                refl[j] = fprev<S>(b, pop_index<S>(g, opp(q), x, row), opp(q));
+                pin[j] = fprev<S>(b, pop_index<S>(g, q, x, row), q);
+                fo[j] = fprev<S>(b, in ? pop_index<S>(g, opp(q), fx, (uint32_t)fy + (uint32_t)g.ny * (uint32_t)fz)
+                                       : pop_index<S>(g, opp(q), x, row), opp(q));
+            });
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                asm volatile("" : "+v"(ws[j].x), "+v"(ws[j].y), "+v"(ws[j].z), "+v"(ws[j].w), "+v"(fpart[j]),
+                             "+v"(refl[j]), "+v"(pin[j]), "+v"(fo[j]));
+            for_q(seq, [&](auto qc) {
+                constexpr int q = decltype(qc)::value, j = q - q0;
+                if (!((linkbits >> q) & 1u)) return;
+                const float wsv[4] = {ws[j].x, ws[j].y, ws[j].z, ws[j].w};
+                const bool farther_ok = fpart[j] == 0;
+                float tlf;
+                uint32_t win;
+                const int rule = link_rule(b, p, x, y, z, q, tlf, win);
+                const adj::LinkD<float> d =
+                    adj::link_value<float>(cx(q), cy(q), cz(q), weight<float>(q), p.far_rho, rule, farther_ok, refl[j],
+                                           farther_ok ? fo[j] : 0.0f, pin[j], wgv, wsv, tlf);
+                gq[q] = d.value;
+                const int sel = p.selected_part;
+                if (p.accumulate_loads && p.load_component != 2 && (sel == 0 || sel == (int)part[q])) {
+                    const float arm[3] = {wx - d.lf * (float)cx(q) * p.dx - bx, wy - d.lf * (float)cy(q) * p.dx - by,
+                                          wz - d.lf * (float)cz(q) * p.dx - bz};
+                    // J_link = -fscale (value + reflected) c_q . e(arm)
+                    load_dv[q] = -p.force_scale * load_weight<q>(w, arm);
+                }
+            });
+        };
+        link_group(QSeq<1, 2, 3>{}, std::integral_constant<int, 1>{}, 0xEu);
+        link_group(QSeq<4, 5, 6>{}, std::integral_constant<int, 4>{}, 0x70u);
+        link_group(QSeq<7, 8, 9>{}, std::integral_constant<int, 7>{}, 0x380u);
+        link_group(QSeq<10, 11, 12>{}, std::integral_constant<int, 10>{}, 0x1C00u);
+        link_group(QSeq<13, 14, 15>{}, std::integral_constant<int, 13>{}, 0xE000u);
+        link_group(QSeq<16, 17, 18>{}, std::integral_constant<int, 16>{}, 0x70000u);
+    }
     collision_adjoint<COLL>(gq, p.omega_plus, p.omega_minus, lp, mu);
     for_q(AllQ{}, [&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        write_pull<q>(b, p, x, y, z, sx[q], srow[q], far[q], link[q] ? 0.0f : mu[q]);
-        nu_cell[q * 256] = link[q] ? mu[q] + load_dv[q] : 0.0f;
+        write_pull<q>(b, p, x, y, z, sx[q], srow[q], far[q], (linkbits >> q) & 1u ? 0.0f : mu[q]);
+        if constexpr (q != 0) nu_cell[q * 256] = (linkbits >> q) & 1u ? mu[q] + load_dv[q] : 0.0f;
     });
+    nu_cell[0] = __uint_as_float(linkbits);
 }
 
 template <int COLL, int S>
@@ -295,7 +363,7 @@ __global__ __launch_bounds__(256) void adjoint_general_p1(AdjointBuffers b, Step
         int x0, y0, z;
         tile_origin(p.g, b.general_list[i], x0, y0, z);
         const int x = x0 + (int)(threadIdx.x & (TILE_X - 1));
-        const int y = y0 + (int)(threadIdx.x / TILE_X);
+        const int y = y0 + (int)__builtin_amdgcn_readfirstlane(threadIdx.x / TILE_X);
         if (x < p.g.nx && y < p.g.ny)
             general_p1_cell<COLL, S>(b, p, w, x, y, z, bx, by, bz, b.nu + (size_t)i * 19 * 256 + threadIdx.x);
     }
@@ -349,11 +417,25 @@ __device__ __forceinline__ void block_sum8(double (&v)[8], double* __restrict__ 
     __syncthreads();
 }
 
+// Parameters whose tangents are loaded together in pass 2a: one at a time,
+// each is a round trip to memory.  A step has a few hundred listed tiles, about
+// one workgroup per CU, so the pass takes one wavefront's chain of round trips
+// (256 x 128 x 128, 280 listed tiles, 8 parameters: 61 us one at a time, 58 in
+// twos, 56 in fours).
+constexpr int TANGENT_BATCH = 4;
+
 __device__ __forceinline__ void contract(double (&acc)[8], int K, const float4* __restrict__ dW, size_t n,
                                          uint32_t cell, float gx, float gy, float gz, float gw) {
-    for (int k = 0; k < K; ++k) {
-        const float4 t = dW[(size_t)k * n + cell];
-        acc[k] += (double)gx * t.x + (double)gy * t.y + (double)gz * t.z + (double)gw * t.w;
+#pragma unroll
+    for (int k0 = 0; k0 < 8; k0 += TANGENT_BATCH) {
+        if (k0 >= K) break;
+        float4 t[TANGENT_BATCH];
+#pragma unroll
+        for (int u = 0; u < TANGENT_BATCH; ++u) t[u] = dW[(size_t)min(k0 + u, K - 1) * n + cell];
+#pragma unroll
+        for (int u = 0; u < TANGENT_BATCH; ++u)
+            if (k0 + u < K)
+                acc[k0 + u] += (double)gx * t[u].x + (double)gy * t[u].y + (double)gz * t[u].z + (double)gw * t[u].w;
     }
 }
 
@@ -438,66 +520,44 @@ __device__ __forceinline__ void general_p2a_cell(const AdjointBuffers& b, const 
         contract(acc, w.K, b.dW, n, gid, gx, gy, gz, 0.0f);
         return;
     }
+    const uint32_t linkbits = __float_as_uint(nu_cell[0]);
+    if (linkbits == 0) return;   // a fluid cell without links feeds nothing else
     const Sources s = sources(p, x, y, z);
     const float4 wg4 = b.wall[gid];
     const float wgv[4] = {wg4.x, wg4.y, wg4.z, wg4.w};
     float gxw[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    // Load pass 1, unconditional (a far-field source or a far side outside the
-    // domain reads this cell and is ignored): the part ids of every source
-    // and far side, the cell's previous populations, its adjoint slots (kept
+    // Load pass 1: the cell's previous populations, its adjoint slots (kept
     // in registers and stored once at the end: only this cell writes them
     // in this pass) and nu.
     auto src_of = [&](auto qc) {
         constexpr int q = decltype(qc)::value;
         bool far;
-        const uint32_t src = source_of<q>(s, g, x, y, z, far);
-        return far ? gid : src;
+        return source_of<q>(s, g, x, y, z, far);
     };
-    auto fid_of = [&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        const int fx = x + cx(q), fy = y + cy(q), fz = z + cz(q);
-        return inside(g, fx, fy, fz) ? flat(g, fx, fy, fz) : gid;
-    };
-    uint32_t part[19], fpart[19];
     float fown[19], lam[19], nuv[19];
-    uint32_t farbits = 0, okbits = 0;
     for_q(AllQ{}, [&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        bool far;
-        (void)source_of<q>(s, g, x, y, z, far);
-        farbits |= (uint32_t)far << q;
-        okbits |= (uint32_t)inside(g, x + cx(q), y + cy(q), z + cz(q)) << q;
-        part[q] = b.solid_cur[src_of(qc)];
-        fpart[q] = b.solid_cur[fid_of(qc)];
         fown[q] = fprev<S>(b, pop_index<S>(g, q, x, row), q);
         lam[q] = b.lam_out[lam_at(g, q, x, row)];
         nuv[q] = nu_cell[q * 256];
     });
-    asm volatile("" : BF_ASM19(part), BF_ASM19(fpart), BF_ASM19(fown));
+    asm volatile("" : BF_ASM19(fown));
     asm volatile("" : BF_ASM19(lam), BF_ASM19(nuv));
-    // links, links whose far side is an in-domain fluid cell, links whose
-    // part counts toward the loads
-    uint32_t linkbits = 0, fartherbits = 0, selbits = 0;
     const int sel = p.selected_part;
-    for_q(AllQ{}, [&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        linkbits |= (uint32_t)(part[q] != 0 && !((farbits >> q) & 1u)) << q;
-        fartherbits |= (uint32_t)(((okbits >> q) & 1u) && fpart[q] == 0) << q;
-        selbits |= (uint32_t)(sel == 0 || sel == (int)part[q]) << q;
-    });
     // Load pass 2, three directions at a time: each link's source wall entry
-    // and far-side population loaded together; then the wall-field tangents
-    // of the group's link sources.
+    // and part, and its far side's population and part, loaded together; then
+    // the wall-field tangents of the group's link sources.
     auto link_group = [&](auto seq, auto first_c, uint32_t gmask) {
         constexpr int q0 = decltype(first_c)::value;
         float4 ws[3];
         float fo[3];
-        uint32_t srcs[3];
+        uint32_t srcs[3], part[3], fpart[3];
         float gws[3][4];
         for (int j = 0; j < 3; ++j) {
             ws[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             fo[j] = 0.0f;
             srcs[j] = gid;
+            part[j] = fpart[j] = 0;
             for (int i = 0; i < 4; ++i) gws[j][i] = 0.0f;
         }
         if (!(linkbits & gmask)) return;
@@ -508,10 +568,16 @@ __device__ __forceinline__ void general_p2a_cell(const AdjointBuffers& b, const 
             srcs[q - q0] = src;
             ws[q - q0] = b.wall[src];
             const int fx = x + cx(q), fy = y + cy(q), fz = z + cz(q);
-            fo[q - q0] = fprev<S>(b, lk && inside(g, fx, fy, fz)
+            // (a far side outside the domain reads this cell, then counts as solid)
+            const bool in = inside(g, fx, fy, fz);
+            const uint32_t fid = lk && in ? flat(g, fx, fy, fz) : gid;
+            fo[q - q0] = fprev<S>(b, lk && in
                                       ? pop_index<S>(g, opp(q), fx, (uint32_t)fy + (uint32_t)g.ny * (uint32_t)fz)
                                       : pop_index<S>(g, opp(q), x, row), opp(q));
+            part[q - q0] = b.solid_cur[src];
+            fpart[q - q0] = (uint32_t)b.solid_cur[fid] | (in ? 0u : 256u);
         });
+        asm volatile("" : "+v"(part[0]), "+v"(part[1]), "+v"(part[2]), "+v"(fpart[0]), "+v"(fpart[1]), "+v"(fpart[2]));
         asm volatile("" : "+v"(ws[0].x), "+v"(ws[0].y), "+v"(ws[0].z), "+v"(ws[0].w), "+v"(ws[1].x),
                      "+v"(ws[1].y), "+v"(ws[1].z), "+v"(ws[1].w), "+v"(ws[2].x), "+v"(ws[2].y), "+v"(ws[2].z),
                      "+v"(ws[2].w), "+v"(fo[0]), "+v"(fo[1]), "+v"(fo[2]));
@@ -520,7 +586,7 @@ __device__ __forceinline__ void general_p2a_cell(const AdjointBuffers& b, const 
             if (!((linkbits >> q) & 1u)) return;
             const float4 ws4 = ws[q - q0];
             const float wsv[4] = {ws4.x, ws4.y, ws4.z, ws4.w};
-            const bool farther_ok = (fartherbits >> q) & 1u;
+            const bool farther_ok = fpart[q - q0] == 0;
             const float refl = fown[opp(q)];
             const float farther = farther_ok ? fo[q - q0] : 0.0f;
             const float pin = fown[q];
@@ -544,7 +610,7 @@ __device__ __forceinline__ void general_p2a_cell(const AdjointBuffers& b, const 
                 }
             }
             float refl_load = 0.0f;
-            if (p.accumulate_loads && p.load_component != 2 && ((selbits >> q) & 1u)) {
+            if (p.accumulate_loads && p.load_component != 2 && (sel == 0 || sel == (int)part[q - q0])) {
                 const float larm[3] = {wx - d.lf * (float)cx(q) * p.dx - bx, wy - d.lf * (float)cy(q) * p.dx - by,
                                        wz - d.lf * (float)cz(q) * p.dx - bz};
                 refl_load = -fs * load_weight<q>(w, larm);
@@ -556,13 +622,21 @@ __device__ __forceinline__ void general_p2a_cell(const AdjointBuffers& b, const 
         });
         // contract in ascending q per parameter (a non-link direction adds
         // zero times this cell's tangent)
-        for (int k = 0; k < w.K; ++k) {
-            float4 t[3];
-            for (int j = 0; j < 3; ++j) t[j] = b.dW[(size_t)k * n + srcs[j]];
-            for (int j = 0; j < 3; ++j)
-                if ((linkbits >> (q0 + j)) & 1u)
-                    acc[k] += (double)gws[j][0] * t[j].x + (double)gws[j][1] * t[j].y + (double)gws[j][2] * t[j].z +
-                              (double)gws[j][3] * t[j].w;
+#pragma unroll
+        for (int k0 = 0; k0 < 8; k0 += TANGENT_BATCH) {
+            if (k0 >= w.K) break;
+            float4 t[TANGENT_BATCH][3];
+#pragma unroll
+            for (int u = 0; u < TANGENT_BATCH; ++u)
+                for (int j = 0; j < 3; ++j) t[u][j] = b.dW[(size_t)min(k0 + u, w.K - 1) * n + srcs[j]];
+#pragma unroll
+            for (int u = 0; u < TANGENT_BATCH; ++u) {
+                if (k0 + u >= w.K) break;
+                for (int j = 0; j < 3; ++j)
+                    if ((linkbits >> (q0 + j)) & 1u)
+                        acc[k0 + u] += (double)gws[j][0] * t[u][j].x + (double)gws[j][1] * t[u][j].y +
+                                       (double)gws[j][2] * t[u][j].z + (double)gws[j][3] * t[u][j].w;
+            }
         }
     };
     link_group(QSeq<1, 2, 3>{}, std::integral_constant<int, 1>{}, 0xEu);
@@ -586,7 +660,7 @@ __global__ __launch_bounds__(256) void adjoint_general_p2a(AdjointBuffers b, Ste
         int x0, y0, z;
         tile_origin(p.g, b.general_list[i], x0, y0, z);
         const int x = x0 + (int)(threadIdx.x & (TILE_X - 1));
-        const int y = y0 + (int)(threadIdx.x / TILE_X);
+        const int y = y0 + (int)__builtin_amdgcn_readfirstlane(threadIdx.x / TILE_X);
         double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         if (x < p.g.nx && y < p.g.ny)
             general_p2a_cell<S, RAY>(b, p, w, x, y, z, bx, by, bz, b.nu + (size_t)i * 19 * 256 + threadIdx.x, acc);
@@ -594,19 +668,37 @@ __global__ __launch_bounds__(256) void adjoint_general_p2a(AdjointBuffers b, Ste
     }
 }
 
+// Fixed-order sum of the listed tiles' gradient partials into the running
+// FP64 gradient, by one workgroup.
+__device__ void sum_gradient(const double* __restrict__ partials, uint32_t count, double* __restrict__ total) {
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (uint32_t i = threadIdx.x; i < count; i += blockDim.x) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] += partials[(size_t)i * 8 + k];
+    }
+    __shared__ double out[8];
+    block_sum8(v, out);
+    if (threadIdx.x < 8) total[threadIdx.x] += out[threadIdx.x];
+}
+
 // ---------------------------------------------------------------------------
 // Wall tiles, pass 2b: populations one link beyond the cell.
 // ---------------------------------------------------------------------------
+// (and, by workgroup 0, the sum of pass 2a's gradient partials)
 template <int S>
 __global__ __launch_bounds__(256) void adjoint_general_p2b(AdjointBuffers b, StepParams p, AdjointParams w) {
     const uint32_t count = *b.general_count;
+    if (blockIdx.x == 0) {
+        sum_gradient(b.grad_partials, count, b.grad_total);
+        return;
+    }
     const float bx = (float)b.body[0], by = (float)b.body[1], bz = (float)b.body[2];
     const Grid& g = p.g;
-    for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
+    for (uint32_t i = blockIdx.x - 1; i < count; i += gridDim.x - 1) {
         int x0, y0, z;
         tile_origin(g, b.general_list[i], x0, y0, z);
         const int x = x0 + (int)(threadIdx.x & (TILE_X - 1));
-        const int y = y0 + (int)(threadIdx.x / TILE_X);
+        const int y = y0 + (int)__builtin_amdgcn_readfirstlane(threadIdx.x / TILE_X);
         if (x >= g.nx || y >= g.ny) continue;
         const uint32_t row = (uint32_t)y + (uint32_t)g.ny * (uint32_t)z;
         const uint32_t gid = (uint32_t)x + (uint32_t)g.nx * row;
@@ -631,50 +723,60 @@ __global__ __launch_bounds__(256) void adjoint_general_p2b(AdjointBuffers b, Ste
             });
             continue;
         }
-        if (p.wall_rule == WALL_HALFWAY) continue;
+        const uint32_t linkbits = __float_as_uint(nu_cell[0]);
+        if (p.wall_rule == WALL_HALFWAY || linkbits == 0) continue;
         const Sources s = sources(p, x, y, z);
         const float4 wg4 = b.wall[gid];
         const float wgv[4] = {wg4.x, wg4.y, wg4.z, wg4.w};
-        for_q(AllQ{}, [&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-            bool far;
-            const uint32_t src = source_of<q>(s, g, x, y, z, far);
-            if (far || b.solid_cur[src] == 0) return;
-            const int fx = x + cx(q), fy = y + cy(q), fz = z + cz(q);
-            if (!inside(g, fx, fy, fz)) return;
-            const uint32_t fid = flat(g, fx, fy, fz);
-            if (b.solid_cur[fid] != 0) return;
-            const float4 ws4 = b.wall[src];
-            const float wsv[4] = {ws4.x, ws4.y, ws4.z, ws4.w};
-            float tlf;
-            uint32_t win;
-            const int rule = link_rule(b, p, x, y, z, q, tlf, win);
-            const adj::LinkD<float> d = adj::link_value<float>(
-                cx(q), cy(q), cz(q), weight<float>(q), p.far_rho, rule, true,
-                fprev<S>(b, pop_index<S>(g, opp(q), x, row), opp(q)),
-                fprev<S>(b, pop_index<S>(g, opp(q), fx, (uint32_t)fy + (uint32_t)g.ny * (uint32_t)fz), opp(q)),
-                fprev<S>(b, pop_index<S>(g, q, x, row), q), wgv, wsv, tlf);
-            if (d.uses_farther)
-                b.lam_out[lam_at(g, opp(q), fx, (uint32_t)fy + (uint32_t)g.ny * (uint32_t)fz)] +=
-                    nu_cell[q * 256] * d.d_farther;
-        });
-    }
-}
-
-// Fixed-order sum of the listed tiles' gradient partials into the running
-// FP64 gradient.
-__global__ __launch_bounds__(256) void reduce_gradient(const double* __restrict__ partials,
-                                                       const uint32_t* __restrict__ count,
-                                                       double* __restrict__ total) {
-    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    const uint32_t c = *count;
-    for (uint32_t i = threadIdx.x; i < c; i += blockDim.x) {
+        // six directions at a time, each group's loads together (a direction
+        // without a link, or whose far side lies outside, reads this cell)
+        auto far_group = [&](auto seq, auto first_c, uint32_t gmask) {
+            constexpr int q0 = decltype(first_c)::value;
+            if (!(linkbits & gmask)) return;
+            uint32_t fpart[6];
+            float4 ws[6];
+            float refl[6], farther[6], pin[6], nu[6], lam[6];
+            for_q(seq, [&](auto qc) {
+                constexpr int q = decltype(qc)::value, j = q - q0;
+                const int fx = x + cx(q), fy = y + cy(q), fz = z + cz(q);
+                const bool in = inside(g, fx, fy, fz);
+                const bool lk = ((linkbits >> q) & 1u) && in;
+                bool far;
+                const uint32_t src = source_of<q>(s, g, x, y, z, far);
+                const size_t at = lk ? pop_index<S>(g, opp(q), fx, (uint32_t)fy + (uint32_t)g.ny * (uint32_t)fz)
+                                     : pop_index<S>(g, opp(q), x, row);
+                fpart[j] = (uint32_t)b.solid_cur[lk ? flat(g, fx, fy, fz) : gid] | (lk ? 0u : 256u);
+                ws[j] = b.wall[lk ? src : gid];
+                refl[j] = fprev<S>(b, pop_index<S>(g, opp(q), x, row), opp(q));
+                farther[j] = fprev<S>(b, at, opp(q));
+                pin[j] = fprev<S>(b, pop_index<S>(g, q, x, row), q);
+                nu[j] = nu_cell[q * 256];
+                lam[j] = b.lam_out[at];
+            });
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] += partials[(size_t)i * 8 + k];
+            for (int j = 0; j < 6; ++j)
+                asm volatile("" : "+v"(fpart[j]), "+v"(ws[j].x), "+v"(ws[j].y), "+v"(ws[j].z), "+v"(ws[j].w),
+                             "+v"(refl[j]), "+v"(farther[j]), "+v"(pin[j]), "+v"(nu[j]), "+v"(lam[j]));
+            for_q(seq, [&](auto qc) {
+                constexpr int q = decltype(qc)::value, j = q - q0;
+                if (fpart[j] != 0) return;
+                const float wsv[4] = {ws[j].x, ws[j].y, ws[j].z, ws[j].w};
+                float tlf;
+                uint32_t win;
+                const int rule = link_rule(b, p, x, y, z, q, tlf, win);
+                const adj::LinkD<float> d =
+                    adj::link_value<float>(cx(q), cy(q), cz(q), weight<float>(q), p.far_rho, rule, true, refl[j],
+                                           farther[j], pin[j], wgv, wsv, tlf);
+                if (d.uses_farther)
+                    b.lam_out[lam_at(g, opp(q), x + cx(q),
+                                     (uint32_t)(y + cy(q)) + (uint32_t)g.ny * (uint32_t)(z + cz(q)))] =
+                        lam[j] + nu[j] * d.d_farther;
+            });
+        };
+        far_group(QSeq<1, 2, 3, 4, 5, 6>{}, std::integral_constant<int, 1>{}, 0x7Eu);
+        far_group(QSeq<7, 8, 9, 10, 11, 12>{}, std::integral_constant<int, 7>{}, 0x1F80u);
+        far_group(QSeq<13, 14, 15, 16, 17, 18>{}, std::integral_constant<int, 13>{}, 0x7E000u);
     }
-    __shared__ double out[8];
-    block_sum8(v, out);
-    if (threadIdx.x < 8) total[threadIdx.x] += out[threadIdx.x];
 }
 
 // ---------------------------------------------------------------------------
@@ -1088,8 +1190,7 @@ static hipError_t adjoint_step_t(const AdjointBuffers& b, const StepParams& p, c
         hipLaunchKernelGGL((adjoint_general_p2a<S, true>), dim3(general_blocks), dim3(256), 0, s, b, p, w);
     else
         hipLaunchKernelGGL((adjoint_general_p2a<S, false>), dim3(general_blocks), dim3(256), 0, s, b, p, w);
-    hipLaunchKernelGGL(adjoint_general_p2b<S>, dim3(general_blocks), dim3(256), 0, s, b, p, w);
-    hipLaunchKernelGGL(reduce_gradient, dim3(1), dim3(256), 0, s, b.grad_partials, b.general_count, b.grad_total);
+    hipLaunchKernelGGL(adjoint_general_p2b<S>, dim3(general_blocks + 1), dim3(256), 0, s, b, p, w);
     return hipGetLastError();
 }
 

@@ -394,58 +394,66 @@ __host__ __device__ __forceinline__ void reverse(const R (&f)[19], R op, R om, c
         const R c2 = R(1) / R(3);
         const R h_one = R(1) - c2;
         const R om1 = R(1) - op;
-        // limiter: post = feq + s (cand - feq)
-        R lcand[19], lfeq[19];
-        each(AllQ{}, [&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-            lcand[q] = lp[q];
-            lfeq[q] = R(0);
-        });
-        if (t.limited) {
-            R cand[19], feq[19];
-            cand[0] = t.post0;
-            feq[0] = t.feq0;
+        // limiter: post = feq + s (cand - feq), so lcand = s lp and
+        // lfeq = (1 - s) lp, and the binding direction's two get its share of
+        // s's own adjoint.  Formed below from these scalars where they are
+        // used: held as arrays they are 38 registers in every cell.
+        R star_cand = R(0), star_feq = R(0);
+        if (t.limited && t.qstar >= 0) {
+            R ls = (t.post0 - t.feq0) * lp[0];
+            R fe = t.feq0, ca = t.post0;
             each(Pairs{}, [&](auto kc) {
                 constexpr int k = decltype(kc)::value, q = 2 * k + 1;
-                cand[q] = t.P[k] + t.Q[k];
-                cand[q + 1] = t.P[k] - t.Q[k];
-                feq[q] = t.A[k] + t.B[k];
-                feq[q + 1] = t.A[k] - t.B[k];
+                const R cp = t.P[k] + t.Q[k], cm = t.P[k] - t.Q[k];
+                const R fp = t.A[k] + t.B[k], fm = t.A[k] - t.B[k];
+                ls = ls + (cp - fp) * lp[q];
+                ls = ls + (cm - fm) * lp[q + 1];
+                if (t.qstar == q) {
+                    fe = fp;
+                    ca = cp;
+                } else if (t.qstar == q + 1) {
+                    fe = fm;
+                    ca = cm;
+                }
             });
-            R ls = R(0);
-            each(AllQ{}, [&](auto qc) {
-                constexpr int q = decltype(qc)::value;
-                ls = ls + (cand[q] - feq[q]) * lp[q];
-                lcand[q] = t.scale * lp[q];
-                lfeq[q] = (R(1) - t.scale) * lp[q];
-            });
-            if (t.qstar >= 0) {
-                each(AllQ{}, [&](auto qc) {
-                    constexpr int q = decltype(qc)::value;
-                    if (q == t.qstar) {
-                        const R fe = feq[q], ca = cand[q];
-                        const bool lin = R(1.0e-6) * fe > R(1.0e-12);
-                        const R fl = lin ? R(1.0e-6) * fe : R(1.0e-12);
-                        const R d = fe - ca, n = fe - fl;
-                        lfeq[q] = lfeq[q] + ls * ((R(1) - (lin ? R(1.0e-6) : R(0))) * d - n) / (d * d);
-                        lcand[q] = lcand[q] + ls * n / (d * d);
-                    }
-                });
+            const bool lin = R(1.0e-6) * fe > R(1.0e-12);
+            const R fl = lin ? R(1.0e-6) * fe : R(1.0e-12);
+            const R d = fe - ca, n = fe - fl;
+            star_feq = ls * ((R(1) - (lin ? R(1.0e-6) : R(0))) * d - n) / (d * d);
+            star_cand = ls * n / (d * d);
+        }
+        auto limited_pair = [&](int q, R& cq, R& eq) {
+            cq = t.scale * lp[q];
+            eq = (R(1) - t.scale) * lp[q];
+            if (q == t.qstar) {
+                cq = cq + star_cand;
+                eq = eq + star_feq;
             }
+        };
+        R lcand0 = lp[0];
+        if (t.limited) {
+            R e0;
+            limited_pair(0, lcand0, e0);
+            lfeq0 = e0;
         }
         // cand0 = feq0 - 4.5 w0 om1 c2T ; cand_q, cand_{q+1} = P +- Q
-        R lc2T = R(-4.5) * wq<R>(0) * om1 * lcand[0];
-        lfeq0 = lcand[0] + lfeq[0];
+        R lc2T = R(-4.5) * wq<R>(0) * om1 * lcand0;
+        lfeq0 = lcand0 + lfeq0;
         R ldg0 = R(0), ldg1 = R(0), ldg2 = R(0), lod0 = R(0), lod1 = R(0), lod2 = R(0);
         R laXxy = R(0), laXxz = R(0), laXyy = R(0), laXzz = R(0), laYyz = R(0), laYzz = R(0);
         each(Pairs{}, [&](auto kc) {
             constexpr int k = decltype(kc)::value, q = 2 * k + 1;
             constexpr int X = cx(q), Y = cy(q), Z = cz(q);
             const R w = wq<R>(q);
-            const R lP = lcand[q] + lcand[q + 1];
-            const R lQ = lcand[q] - lcand[q + 1];
-            lA[k] = lP + (lfeq[q] + lfeq[q + 1]);
-            lB[k] = lQ + (lfeq[q] - lfeq[q + 1]);
+            R c0 = lp[q], c1 = lp[q + 1], e0 = R(0), e1 = R(0);
+            if (t.limited) {
+                limited_pair(q, c0, e0);
+                limited_pair(q + 1, c1, e1);
+            }
+            const R lP = c0 + c1;
+            const R lQ = c0 - c1;
+            lA[k] = lP + (e0 + e1);
+            lB[k] = lQ + (e0 - e1);
             const R lcontr = (R(4.5) * w) * om1 * lP;
             lc2T = lc2T - lcontr;
             if constexpr (X != 0) ldg0 = ldg0 + lcontr;

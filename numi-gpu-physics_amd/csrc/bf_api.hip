@@ -2457,8 +2457,8 @@ bf_status adjoint_alloc(bf_context* c, uint32_t interval, uint32_t segments) {
     a.gpos = (float4*)A.take(e, 16 * verts);
     a.gvel = (float4*)A.take(e, 16 * verts);
     for (int i = 0; i < 2 && e == hipSuccess; ++i) {
-        if (!a.ev_geo[i]) e = hipEventCreateWithFlags(&a.ev_geo[i], hipEventDisableTiming);
-        if (e == hipSuccess && !a.ev_done[i]) e = hipEventCreateWithFlags(&a.ev_done[i], hipEventDisableTiming);
+        if (!a.ev_geo[i]) e = hipEventCreateWithFlags(&a.ev_geo[i], STREAM_EVENT);
+        if (e == hipSuccess && !a.ev_done[i]) e = hipEventCreateWithFlags(&a.ev_done[i], STREAM_EVENT);
     }
     a.lam[0] = (float*)A.take(e, pop);
     a.lam[1] = (float*)A.take(e, pop);
@@ -2467,8 +2467,8 @@ bf_status adjoint_alloc(bf_context* c, uint32_t interval, uint32_t segments) {
     a.dW[1] = (float4*)A.take(e, 8 * 16 * n);
     if (e == hipSuccess && !a.sc) e = hipStreamCreateWithFlags(&a.sc, hipStreamNonBlocking);
     for (int i = 0; i < 2 && e == hipSuccess; ++i) {
-        if (!a.ev_tan[i]) e = hipEventCreateWithFlags(&a.ev_tan[i], hipEventDisableTiming);
-        if (e == hipSuccess && !a.ev_used[i]) e = hipEventCreateWithFlags(&a.ev_used[i], hipEventDisableTiming);
+        if (!a.ev_tan[i]) e = hipEventCreateWithFlags(&a.ev_tan[i], STREAM_EVENT);
+        if (e == hipSuccess && !a.ev_used[i]) e = hipEventCreateWithFlags(&a.ev_used[i], STREAM_EVENT);
     }
     for (int i = 0; i < 2; ++i) {
         a.vpos[i] = (float4*)A.take(e, 16 * verts);
