@@ -778,9 +778,9 @@ class BirdFlowSimulation:
         return out[:19].copy(), int(out[19]), int(out[20])
 
     def set_profiling(self, enabled=True, level=None):
-        """Per-step HIP events: level 1 around the fast-fluid kernel only, 2
-        also around the general kernel and the geometry (default 2 when
-        enabled)."""
+        """Per-step HIP events: level 1 around the step's fluid launch, 2 around
+        its wall-free tiles and its wall tiles (then launched apart) and the
+        geometry (default 2 when enabled)."""
         lvl = 0 if not enabled else (2 if level is None else int(level))
         self._check(self._lib.bf_set_profiling(self._ctx, lvl))
 
