@@ -627,9 +627,11 @@ bf_status ensure_ray_static(bf_context* c) {
     return BF_OK;
 }
 
-// (Also clears the length of the step's wall-tile list.)
+// exact: the geometry of a step that is over, with the full key band; else
+// that of a step to come, which also clears the length of its wall-tile list.
 bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
     hipError_t e = hipSuccess;
+    uint32_t* general_count = exact ? nullptr : &c->counters[par2(s)];
     if (c->source == BF_GEOMETRY_MESH) {
         MeshBuffers b = mesh_buffers(c);
         b.keys = c->keys;
@@ -638,7 +640,7 @@ bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
         b.tiles_wall_old = fresh ? c->no_tiles : c->tflags[mod4(s - 2)];   // wall[s&1] last written at s-2
         b.list = c->geo_list;
         b.list_count = &c->counters[2];
-        b.general_count = &c->counters[par2(s)];
+        b.general_count = general_count;
         b.mask = c->mask[mod3(s)];
         b.wall = c->wall[par2(s)];
         b.dyn = c->dyn[mod3(s)];
@@ -684,7 +686,7 @@ bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
         b.tiles_wall_old = fresh ? c->no_tiles : c->tflags[mod4(s - 2)];
         b.list = c->geo_list;
         b.list_count = &c->counters[2];
-        b.general_count = &c->counters[par2(s)];
+        b.general_count = general_count;
         b.mask = c->mask[mod3(s)];
         b.wall = c->wall[par2(s)];
         b.dyn = c->dyn[mod3(s)];
@@ -716,7 +718,7 @@ bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
         b.tiles_wall_old = fresh ? c->no_tiles : c->tflags[mod4(s - 2)];
         b.list = c->geo_list;
         b.list_count = &c->counters[2];
-        b.general_count = &c->counters[par2(s)];
+        b.general_count = general_count;
         b.mask = c->mask[mod3(s)];
         b.wall = c->wall[par2(s)];
         b.dyn = c->dyn[mod3(s)];
@@ -738,8 +740,7 @@ bf_status enqueue_geometry(bf_context* c, int64_t s, bool exact, bool fresh) {
         int periodic[3];
         for (int a = 0; a < 3; ++a) periodic[a] = periodic_axis(c->cfg, a) ? 1 : 0;
         e = launch_sphere_geometry(c->mask[mod3(s)], c->wall[par2(s)], c->dyn[mod3(s)], c->g, c->sphere_cr,
-                                   c->sphere_gv, c->sphere_wv, time_of(c, s), periodic, &c->counters[par2(s)],
-                                   c->sb);
+                                   c->sphere_gv, c->sphere_wv, time_of(c, s), periodic, general_count, c->sb);
     }
     if (e != hipSuccess) return hip_fail(c, e, "geometry launch");
     return BF_OK;
@@ -1614,8 +1615,10 @@ bf_status bf_mesh_build(bf_context* c, float t) {
     if (c->source != BF_GEOMETRY_MESH) return fail(c, BF_ERROR_INVALID_ARGUMENT, "no mesh uploaded");
     // Rebuild the current step's geometry at time t with the full key band
     // (geometry audit).  A prefetched next-step geometry stays valid: it
-    // neither reads nor writes the current step's buffers.
+    // neither reads nor writes the current step's buffers.  Its wall-tile list
+    // does not: that step's previous mask is the one built here.
     const int64_t st = c->step;
+    c->list_step = -1;
     hipError_t e0 = launch_fill_u8(c->mask[mod3(st)], 0, c->g.n, c->sb);
     if (e0 == hipSuccess) e0 = launch_fill_wall(c->wall[par2(st)], c->g.n, c->sb);
     if (e0 != hipSuccess) return hip_fail(c, e0, "mesh build");
