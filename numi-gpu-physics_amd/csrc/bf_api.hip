@@ -112,7 +112,7 @@ struct bf_context {
     // static geometry: the wall-tile list in slot 1 holds the current mask's
     // tiles (slot 0 the first step's, when its previous mask differs)
     bool static_list_ready = false;
-    uint32_t static_tiles = 0;            // and how many they are
+    uint32_t static_tiles = 0;            // at most so many
     int last_list = 0;                    // list slot of the last step
     double* partials = nullptr;
     double* block_out = nullptr;
@@ -374,6 +374,13 @@ StepParams make_step_params(const bf_context* c) {
     p.force_scale = c->cfg.force_to_physical;
     for (int q = 0; q < 19; ++q) p.far_eq[q] = equilibrium<float>(q, p.far_rho, p.far_u[0], p.far_u[1], p.far_u[2]);
     return p;
+}
+
+// Where the geometry of the steps to come is from; the static wall-tile list
+// is another geometry's from here on.
+void set_source(bf_context* c, int source) {
+    c->source = source;
+    c->static_list_ready = false;
 }
 
 // Geometry views of step s.
@@ -1288,7 +1295,7 @@ bf_status bf_set_geometry(bf_context* c, const uint8_t* mask_prev, const uint8_t
     if (check_host_array(c, mask_cur, "mask_cur") || check_host_array(c, wall4, "wall"))
         return BF_ERROR_INVALID_ARGUMENT;
     const size_t n = c->g.n;
-    c->source = BF_GEOMETRY_STATIC;
+    set_source(c, BF_GEOMETRY_STATIC);
     c->static_prev_differs = mask_prev && std::memcmp(mask_prev, mask_cur, n) != 0;
     hipStream_t s = c->sb;
     hipError_t e = copy_to_device(c->pipe, c->device, c->mask[0], mask_cur, n, s);
@@ -1453,7 +1460,7 @@ static bf_status install_mesh(bf_context* c, const MeshSource& src, uint32_t ver
     c->m_static_list = (uint32_t*)A.take(e, 4ull * std::max<size_t>(static_list.size(), 1));
     if (e != hipSuccess) {
         A.release();
-        c->source = BF_GEOMETRY_STATIC;
+        set_source(c, BF_GEOMETRY_STATIC);
         return fail(c, BF_ERROR_ALLOCATION_FAILED, std::string("mesh buffers: ") + hipGetErrorString(e));
     }
     hipStream_t s = c->sb;
@@ -1488,7 +1495,7 @@ static bf_status install_mesh(bf_context* c, const MeshSource& src, uint32_t ver
     c->m_triangles = triangle_count;
     c->m_half = half_thickness;
     for (int i = 0; i < 3; ++i) c->m_translation[i] = translation ? translation[i] : 0.0f;
-    c->source = BF_GEOMETRY_MESH;
+    set_source(c, BF_GEOMETRY_MESH);
     c->static_prev_differs = false;
     c->time_start = time_start - (float)((double)c->step * c->cfg.time_step);
     return rebuild_mesh_geometry(c);
@@ -1652,7 +1659,7 @@ bf_status bf_set_translating_sphere(bf_context* c, const float cr[4], const floa
     c->sphere_cr = make_float4(cr[0], cr[1], cr[2], cr[3]);
     c->sphere_gv = make_float3(gv[0], gv[1], gv[2]);
     c->sphere_wv = make_float4(wv[0], wv[1], wv[2], wv[3]);
-    c->source = BF_GEOMETRY_SPHERE;
+    set_source(c, BF_GEOMETRY_SPHERE);
     c->static_prev_differs = false;
     c->time_start = 0.0f;
     return rebuild_sphere_geometry(c);
@@ -1699,7 +1706,7 @@ bf_status bf_set_bird(bf_context* c, const bf_bird_geometry* bird) {
     if (c->bird_keyframe_count > 0 && !(b.frequency > 0.0f))
         return fail(c, BF_ERROR_INVALID_ARGUMENT, "measured keyframes need a positive flapping frequency");
     std::memcpy(&c->bird, bird, sizeof(BirdShape));
-    c->source = BF_GEOMETRY_BIRD;
+    set_source(c, BF_GEOMETRY_BIRD);
     c->static_prev_differs = false;
     c->time_start = 0.0f;
     return rebuild_bird_geometry(c);
@@ -1759,7 +1766,7 @@ bf_status bf_set_flapping_wing(bf_context* c, const bf_flapping_wing* wing) {
         }
     }
     std::memcpy(&c->wing, wing, sizeof(WingShape));
-    c->source = BF_GEOMETRY_WING;
+    set_source(c, BF_GEOMETRY_WING);
     c->static_prev_differs = false;
     c->time_start = 0.0f;
     return rebuild_wing_geometry(c);
@@ -2048,7 +2055,10 @@ static bf_status step_static(bf_context* c, uint32_t steps) {
         const int slot = differs ? 0 : 1;
         if (differs || !c->static_list_ready) {
             if (bf_status r = enqueue_tile_list(c, s, slot, false, c->sa)) return r;
-            if (!differs) c->static_list_ready = true;
+            if (!differs) {
+                c->static_list_ready = true;
+                c->static_tiles = c->g.tiles;    // its length is known on the device alone
+            }
         }
         hipEvent_t* pe = nullptr;
         if (bf_status r = profile_events(c, pe)) return r;
