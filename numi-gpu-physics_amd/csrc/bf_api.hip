@@ -256,7 +256,7 @@ struct bf_context {
         float* lam[2] = {nullptr, nullptr};
         int lam_cur = 0;
         bool have_sensitivity = false;
-        float* nu = nullptr;              // [tiles][19][256]
+        float* nu = nullptr;              // [tiles][19][256]; also the recompute's link table
         float4* dW[2] = {nullptr, nullptr};           // [8][N], by step parity
         hipStream_t sc = nullptr;                     // wall tangents (third stream, default priority)
         hipEvent_t ev_tan[2] = {nullptr, nullptr};    // dW[j] written (stream C)
@@ -2777,15 +2777,18 @@ bf_status bf_adjoint_gradient(bf_context* c, uint32_t steps, const double* load_
             fb.body = c->body;
             StepParams ps = pf;
             if (ray) {
-                // the exact-root table of step s, as the forward step built it
+                // the exact-root table of step s, as the forward step built it,
+                // in the room of nu: the reverse steps write that before they
+                // read it and run on this stream too.  The stepping's tables
+                // hold the last step's and the next one's and stay as they are.
                 MeshBuffers mb = mesh_buffers(c);
                 mb.pos = a.rpos;
                 mb.vel = a.rvel;
                 e = launch_mesh_prepare(mb, mesh_params(c, time_of(c, s), false), c->sb);
                 if (e == hipSuccess) e = launch_ray_links(ray_buffers(c, gc, a.rpos, c->ray_list, c->ray_count,
-                                                                      c->ray_dirs, c->ray_links[s & 1], nullptr),
+                                                                      c->ray_dirs, a.nu, nullptr),
                                                           ray_params(c), c->sb);
-                ps.links = c->ray_links[s & 1];
+                ps.links = a.nu;
             }
             if (e == hipSuccess)
                 e = launch_fluid_step(arith, storage, coll, fb, ps, STEP_ALL, wall_blocks_for(c, c->g.tiles), c->sb);
