@@ -2049,6 +2049,12 @@ static bf_status step_static(bf_context* c, uint32_t steps) {
     if (e == hipSuccess) e = hipStreamWaitEvent(c->sa, c->ev_ready[0], 0);
     if (e != hipSuccess) return hip_fail(c, e, "event wait");
     uint32_t waiting = 0;                // steps whose loads wait for their reduction
+    auto reduce_loads = [&](int64_t last, const FluidBuffers& fb) {
+        const hipError_t r = launch_load_reduction(load_buffers(c, fb), make_step_params(c),
+                                                   (uint64_t)last - waiting + 1, waiting, c->sa);
+        waiting = 0;
+        return r;
+    };
     for (uint32_t i = 0; i < steps; ++i) {
         const int64_t s = c->step + 1;
         const bool differs = c->static_prev_differs;   // the first step after bf_set_geometry with another mask
@@ -2061,7 +2067,11 @@ static bf_status step_static(bf_context* c, uint32_t steps) {
             }
         }
         hipEvent_t* pe = nullptr;
-        if (bf_status r = profile_events(c, pe)) return r;
+        if (bf_status r = profile_events(c, pe)) {
+            // the steps that ran keep their loads
+            e = reduce_loads(c->step, fluid_buffers(c, c->step, 1));
+            return e == hipSuccess ? r : hip_fail(c, e, "load reduction");
+        }
         const bool split = pe && c->profiling_level >= 2;
         const FluidBuffers fb = fluid_buffers(c, s, slot);
         const StepParams p = step_params(c, s);
@@ -2079,10 +2089,8 @@ static bf_status step_static(bf_context* c, uint32_t steps) {
             e = launch_fluid_step(arith, storage, coll, fb, p, split ? STEP_FAST_TILES : STEP_ALL, wall_blocks, c->sa);
         if (pe && e == hipSuccess) e = hipEventRecord(pe[1], c->sa);
         ++waiting;
-        if (e == hipSuccess && (waiting == LOAD_SLOTS || i + 1 == steps || differs)) {
-            e = launch_load_reduction(load_buffers(c, fb), p, (uint64_t)s - waiting + 1, waiting, c->sa);
-            waiting = 0;
-        }
+        if (e == hipSuccess && (waiting == LOAD_SLOTS || i + 1 == steps || differs))
+            e = reduce_loads(s, fb);
         if (e != hipSuccess) return hip_fail(c, e, "fluid step launch");
         c->step = s;
         c->cur = 1 - c->cur;

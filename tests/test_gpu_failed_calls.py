@@ -1,12 +1,14 @@
 """Calls that fail for want of memory leave a simulation that steps on
-correctly.  Each case runs in a child process whose HIP allocations pass
-through a small library that refuses them on request (hipMalloc beyond a
-size), as the runtime does when memory is short:
+correctly.  Each case runs in a child process whose HIP allocations and events
+pass through a small library that refuses them on request (hipMalloc beyond a
+size, hipEventCreate beyond a count), as the runtime does when memory is short:
 
 * a mesh upload that cannot allocate falls back to static geometry with the
   masks and walls in place: the steps after it equal the FP32 oracle's with
   those, bit for bit, whether the geometry before it was a moving sphere alone
-  or one set over a static obstacle."""
+  or one set over a static obstacle;
+* a profiled batch that cannot create its events stops with the loads of the
+  steps that ran in the history, and the steps after it carry on from there."""
 import ctypes
 import os
 import subprocess
@@ -21,13 +23,19 @@ SHIM = r"""
 #include <dlfcn.h>
 #include <stddef.h>
 static size_t largest = (size_t)-1;
-void refuse(size_t bytes_above) { largest = bytes_above; }
+static long events = -1;               /* events left; negative: no limit */
+void refuse(size_t bytes_above, long events_after) { largest = bytes_above; events = events_after; }
 static void* real(const char* name) {
     return dlsym(dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_NOLOAD), name);
 }
 int hipMalloc(void** p, size_t n) {
     if (n > largest) { *p = NULL; return 2; }      /* hipErrorOutOfMemory */
     return ((int (*)(void**, size_t))real("hipMalloc"))(p, n);
+}
+int hipEventCreate(void** e) {
+    if (events == 0) return 2;
+    if (events > 0) --events;
+    return ((int (*)(void**))real("hipEventCreate"))(e);
 }
 """
 
@@ -48,14 +56,14 @@ def failed_mesh(bh, bfref, cases, refuse, over_static):
             sim.init_equilibrium()
             sim.advance(6)
         points = np.tile(np.float32([[5, 5, 5], [9, 5, 5], [5, 9, 5]]), (2, 1, 1))
-        refuse(0)
+        refuse(0, -1)
         try:
             sim.upload_mesh(points, np.float32([0.0, 1.0]), np.uint32([[0, 1, 2]]), np.uint8([1]), 0.5)
             raise AssertionError("the upload was not refused")
         except bh.BirdFlowError as err:
             print("upload refused:", err, flush=True)
         finally:
-            refuse(2 ** 64 - 1)
+            refuse(2 ** 64 - 1, -1)
         mask, wall = sim.read_geometry()
         assert mask.any()
         f = sim.read_populations()
@@ -67,7 +75,43 @@ def failed_mesh(bh, bfref, cases, refuse, over_static):
     assert np.array_equal(got, f)
 
 
-CHILDREN = {"mesh after a sphere": (failed_mesh, False), "mesh after a sphere over an obstacle": (failed_mesh, True)}
+def failed_events(bh, bfref, cases, refuse, created):
+    shape, steps = (70, 18, 12), 9
+    n = shape[0] * shape[1] * shape[2]
+    rng = np.random.default_rng(2)
+    p = bfref.make_params(shape, omega_plus=1.9, omega_minus=1.1, collision=bfref.COLLISION_RR3, force_mode=6,
+                          accumulate_loads=True, body_position=(35.0, 9.0, 6.0))
+    mask = np.zeros(shape[::-1], np.uint8)
+    mask[4:7, 6:10, 60:67] = 1
+    wall = np.zeros((n, 4), np.float32)
+    # rough enough for the positivity limiter, whose counts the history carries
+    f0 = (bfref.init_equilibrium(p, mask.ravel(), wall) * rng.uniform(0.1, 1.9, 19 * n)).astype(np.float32)
+    out = []
+    for refused in (False, True):
+        with bh.BirdFlowSimulation(cases.solver_config(p)) as sim:
+            sim.set_geometry(mask.ravel(), wall)
+            sim.write_populations(f0)
+            if refused:
+                sim.set_profiling(True, level=1)
+                refuse(2 ** 64 - 1, created)
+                try:
+                    sim.advance(steps)
+                    raise AssertionError("the batch was not refused")
+                except bh.BirdFlowError as err:
+                    print("batch refused:", err, "after step", sim.step_index, flush=True)
+                finally:
+                    refuse(2 ** 64 - 1, -1)
+                sim.set_profiling(False)
+            sim.advance(steps - sim.step_index)
+            out.append((sim.load_history(steps), sim.read_populations(), sim.read_loads()))
+    assert out[0][0][0, 6] > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+CHILDREN = {"mesh after a sphere": (failed_mesh, False), "mesh after a sphere over an obstacle": (failed_mesh, True),
+            "events, 1 step run": (failed_events, 8), "events, 3 steps run": (failed_events, 20),
+            "events, 5 steps run": (failed_events, 30)}
 
 
 @pytest.mark.gpu
@@ -85,7 +129,7 @@ def test_steps_after_a_refused_call(case, tmp_path):
 
 if __name__ == "__main__":
     shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)    # before the HIP library: its names win
-    shim.refuse.argtypes = [ctypes.c_size_t]
+    shim.refuse.argtypes = [ctypes.c_size_t, ctypes.c_long]
     for sub in ("oracle", "numi-gpu-physics_amd", "tests"):
         sys.path.insert(0, os.path.join(os.path.dirname(HERE), sub))
     import bfref
