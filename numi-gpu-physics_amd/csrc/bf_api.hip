@@ -111,7 +111,7 @@ struct bf_context {
     uint32_t* counters = nullptr;
     // static geometry: the wall-tile list in slot 1 holds the current mask's
     // tiles (slot 0 the first step's, when its previous mask differs)
-    bool static_list_ready = false;
+    bool static_list_ready = true;        // (no geometry yet: no tiles)
     uint32_t static_tiles = 0;            // at most so many
     int last_list = 0;                    // list slot of the last step
     double* partials = nullptr;
