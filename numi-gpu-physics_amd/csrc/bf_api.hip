@@ -303,7 +303,8 @@ struct bf_context {
     // fluid kernel of step s most of the machine
     uint32_t raster_blocks = 1u << 30;
     uint32_t raster_batch = 0;            // triangles per raster wave; 0: from the mesh size
-    int fast_priority = 0, general_priority = 0;   // s_setprio of the fluid kernels' wavefronts
+    int fast_priority = -1, general_priority = 0;  // s_setprio of the fluid kernels' wavefronts (-1: by the step)
+    int apart = -1;                                // a flight's wall-free tiles in a kernel of their own (-1: by the size)
     bool pair_cells = true;                        // 2-byte storage: fast tiles two cells per lane
     uint32_t raster_batch_cap = 32;                // largest automatic raster batch
     uint32_t compute_units = 1;
@@ -350,7 +351,7 @@ hipError_t drain(bf_context* c) {
 StepParams make_step_params(const bf_context* c) {
     StepParams p{};
     p.g = c->g;
-    p.fast_priority = c->fast_priority;
+    p.fast_priority = std::max(0, c->fast_priority);
     p.general_priority = c->general_priority;
     p.pair_cells = c->pair_cells ? 1 : 0;
     for (int a = 0; a < 3; ++a)
@@ -772,6 +773,29 @@ uint32_t wall_blocks_for(const bf_context* c, uint32_t tiles) {
     return tiles == 0 ? 0u : std::min(c->wall_blocks, (tiles + 7u) & ~7u);
 }
 
+// Sizes of grids for the rules below, in cells.
+constexpr uint32_t LARGE_GRID = 8000000u, VERY_LARGE_GRID = 16000000u;
+// STEP_APART or 0 for the wall-free tiles of a coupled flight, launched after
+// the wall tiles in any case: from the size at which they last longer than the chain of
+// reduction, body and geometry beside them (FP32 bird in flight, in fluid_step /
+// apart, ms per step: 224x140x112 0.197 / 0.206, 320x200x168 0.424 / 0.395,
+// 512x256x256 1.059 / 1.030; FP16: 256x160x136 0.130 / 0.131, 320x200x168
+// 0.236 / 0.215).
+int flight_apart(const bf_context* c) {
+    if (c->apart >= 0) return c->apart ? STEP_APART : 0;
+    return c->g.n >= LARGE_GRID ? STEP_APART : 0;
+}
+// Their issue priority over that chain, where it has the time: FP32 0 / 2, ms
+// per step: 352x220x176 0.453 / 0.457, 384x240x192 0.555 / 0.540, 512x256x256
+// 1.030 / 1.013.  No other step takes it: raised over the next step's geometry
+// it starves that where it is the longer of the two (160x160x128 wing 137 ->
+// 176 us per step, 384x192x192 bird with exact roots 561 -> 608) and gains
+// 0.5 % where it is not (512x256x256 bird).
+int flight_priority(const bf_context* c) {
+    if (c->fast_priority >= 0) return c->fast_priority;
+    return c->cfg.storage == BF_STORAGE_FP32 && c->g.n >= VERY_LARGE_GRID ? 2 : 0;
+}
+
 LoadBuffers load_buffers(const bf_context* c, const FluidBuffers& fb) {
     LoadBuffers b{};
     b.partials = c->partials;
@@ -956,16 +980,11 @@ bf_status bf_create(const bf_config* cfg, bf_context** out) {
     c->tile_pass_blocks = (uint32_t)std::max(1, prop.multiProcessorCount);
     // tuning overrides (workgroup counts)
     if (const char* v = std::getenv("BIRDFLOW_RASTER_BLOCKS")) c->raster_blocks = (uint32_t)std::max(1, std::atoi(v));
-    // Issue priority of the wall-free tiles' wavefronts: none.  Raised over the
-    // next step's geometry it gained 0.5 % on the 512x256x256 bird (FP32,
-    // 984 -> 982 us) and starved that geometry where it is the longer of the
-    // two (160x160x128 wing 137 -> 176 us per step, 384x192x192 bird with exact
-    // roots 561 -> 608).
     const bool fp32 = cfg->storage == BF_STORAGE_FP32;
-    c->fast_priority = 0;
     c->general_priority = 3;
     c->raster_batch_cap = fp32 ? 32u : 16u;
     if (const char* v = std::getenv("BIRDFLOW_FAST_PRIORITY")) c->fast_priority = std::min(3, std::max(0, std::atoi(v)));
+    if (const char* v = std::getenv("BIRDFLOW_APART")) c->apart = std::atoi(v) != 0;
     // FP16 / BF16: fast tiles two cells per lane (0 selects one cell per lane)
     if (const char* v = std::getenv("BIRDFLOW_PAIR_CELLS")) c->pair_cells = std::atoi(v) != 0;
     // meshes: cached keys of static triangles (0 rasters every triangle every step)
@@ -2169,7 +2188,10 @@ bf_status bf_step(bf_context* c, uint32_t steps) {
             if (split && e == hipSuccess) e = hipEventRecord(pe[5], c->sa);
             if (early_loads && e == hipSuccess) e = hipEventRecord(c->ev_general[par2(s)], c->sa);
             if (pe && e == hipSuccess) e = hipEventRecord(pe[0], c->sa);
-            if (e == hipSuccess) e = launch_fluid_step(arith, storage, coll, fb, p, STEP_FAST_TILES, 0, c->sa);
+            StepParams pf = p;
+            if (early_loads) pf.fast_priority = flight_priority(c);
+            const int apart = early_loads ? flight_apart(c) : 0;
+            if (e == hipSuccess) e = launch_fluid_step(arith, storage, coll, fb, pf, STEP_FAST_TILES | apart, 0, c->sa);
         } else {
             if (pe && e == hipSuccess) e = hipEventRecord(pe[0], c->sa);
             if (e == hipSuccess) e = launch_fluid_step(arith, storage, coll, fb, p, STEP_ALL, wall_blocks, c->sa);

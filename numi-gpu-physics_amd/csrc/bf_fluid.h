@@ -3,7 +3,8 @@
 //
 // Replaces the fluid part of stepFluidTRT (Sources/BirdFlowMetal/Metal/
 // BirdFlow.metal:2507-3236).  The lattice is split into 64x4 tiles, one
-// 256-lane workgroup each; one launch (fluid_step) covers both kinds:
+// 256-lane workgroup each; one launch (fluid_step) covers both kinds, or the
+// wall-free tiles follow in one of their own (fluid_stream):
 //   * fluid_fast    — tiles with no solid cell (current or previous step) in
 //                     their 1-cell halo: pure pull stream with per-face
 //                     boundary sources, collision, sponge blend, store.
@@ -22,6 +23,8 @@
 // Both kernels share the collision code; a fluid cell gets bit-identical
 // results from either.
 #pragma once
+
+#include <utility>
 
 #include "bf_launch.h"
 
@@ -1379,31 +1382,55 @@ void fluid_step(const typename Store<S>::T* __restrict__ fin, typename Store<S>:
         fluid_fast<ARITH, COLL, S>(block, blocks, fin, fout, dyn_prev, dyn_cur, activation, p);
 }
 
+// The wall-free tiles in a launch and kernel of their own (STEP_APART), at the
+// streaming code's natural occupancy (7 wavefronts per SIMD) and without the
+// wall path's LDS and its scalar registers: for the streaming beside a geometry
+// chain that needs room on the card (flight_apart in bf_api.hip).
+template <int ARITH, int COLL, int S, bool PAIR>
+__global__ __launch_bounds__(256)
+void fluid_stream(const typename Store<S>::T* __restrict__ fin, typename Store<S>::T* __restrict__ fout,
+                  const uint8_t* __restrict__ dyn_prev, const uint8_t* __restrict__ dyn_cur,
+                  uint32_t* __restrict__ activation, StepParams p) {
+    if constexpr (PAIR)
+        fluid_fast_pair<ARITH, COLL, S>(blockIdx.x, gridDim.x, fin, fout, dyn_prev, dyn_cur, activation, p);
+    else
+        fluid_fast<ARITH, COLL, S>(blockIdx.x, gridDim.x, fin, fout, dyn_prev, dyn_cur, activation, p);
+}
+
 // ---------------------------------------------------------------------------
 // Host-side launchers (called from bf_api.hip).
 // ---------------------------------------------------------------------------
 
 template <int ARITH, int COLL, int S, bool PAIR>
-static hipError_t launch_step_p(const FluidBuffers& b, const StepParams& p, uint32_t wall_blocks, uint32_t fast_blocks,
+static hipError_t launch_step_p(const FluidBuffers& b, const StepParams& p, int parts, uint32_t wall_blocks,
                                 hipStream_t s) {
     using T = typename Store<S>::T;
-    if (wall_blocks + fast_blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL((fluid_step<ARITH, COLL, S, PAIR>), dim3(wall_blocks + fast_blocks), dim3(256), 0, s,
-                       (const T*)b.fin, (T*)b.fout, b.solid_prev, b.solid_cur, b.wall, b.dyn_prev, b.dyn_cur,
-                       b.general_list, b.general_count, b.partials, b.body, b.activation, p, wall_blocks);
+    if (!(parts & STEP_WALL_TILES)) wall_blocks = 0;
+    uint32_t fast_blocks = parts & STEP_FAST_TILES ? (PAIR ? p.g.tiles / 2 : p.g.tiles) : 0u, stream_blocks = 0;
+    // coupled flights launch apart with TRT alone
+    constexpr bool STREAM = COLL == COLL_TRT;
+    if (STREAM && (parts & STEP_APART)) std::swap(fast_blocks, stream_blocks);
+    if (wall_blocks + fast_blocks > 0)
+        hipLaunchKernelGGL((fluid_step<ARITH, COLL, S, PAIR>), dim3(wall_blocks + fast_blocks), dim3(256), 0, s,
+                           (const T*)b.fin, (T*)b.fout, b.solid_prev, b.solid_cur, b.wall, b.dyn_prev, b.dyn_cur,
+                           b.general_list, b.general_count, b.partials, b.body, b.activation, p, wall_blocks);
+    if constexpr (STREAM) {
+        if (stream_blocks > 0)
+            hipLaunchKernelGGL((fluid_stream<ARITH, COLL, S, PAIR>), dim3(stream_blocks), dim3(256), 0, s,
+                               (const T*)b.fin, (T*)b.fout, b.dyn_prev, b.dyn_cur, b.activation, p);
+    }
     return hipGetLastError();
 }
 
 template <int ARITH, int COLL, int S>
 static hipError_t launch_step_t(const FluidBuffers& b, const StepParams& p, int parts, uint32_t wall_blocks,
                                 hipStream_t s) {
-    const uint32_t wb = parts & STEP_WALL_TILES ? wall_blocks : 0u;
     if constexpr (S != STORE_FP32) {
         // two cells per lane over tile pairs (whole pairs along x)
         if (p.g.nx % (2 * TILE_X) == 0 && p.pair_cells)
-            return launch_step_p<ARITH, COLL, S, true>(b, p, wb, parts & STEP_FAST_TILES ? p.g.tiles / 2 : 0u, s);
+            return launch_step_p<ARITH, COLL, S, true>(b, p, parts, wall_blocks, s);
     }
-    return launch_step_p<ARITH, COLL, S, false>(b, p, wb, parts & STEP_FAST_TILES ? p.g.tiles : 0u, s);
+    return launch_step_p<ARITH, COLL, S, false>(b, p, parts, wall_blocks, s);
 }
 
 }  // namespace bf

@@ -340,8 +340,10 @@ hipError_t launch_body_step(double* state, const double* load, double* history, 
                             const float* wing_reaction = nullptr);
 
 // The fluid step in one launch, or one of its parts alone: the wall tiles of
-// b.general_list over wall_blocks workgroups, the wall-free tiles.
-enum : int { STEP_WALL_TILES = 1, STEP_FAST_TILES = 2, STEP_ALL = 3 };
+// b.general_list over wall_blocks workgroups, the wall-free tiles.  With
+// STEP_APART the wall-free tiles go in a launch and kernel of their own, after
+// the wall tiles.
+enum : int { STEP_WALL_TILES = 1, STEP_FAST_TILES = 2, STEP_ALL = 3, STEP_APART = 4 };
 hipError_t launch_fluid_step(int arith, int storage, int coll, const FluidBuffers& b, const StepParams& p, int parts,
                              uint32_t wall_blocks, hipStream_t s);
 // Per translation unit: fused arithmetic by storage (FP32, FP16, BF16), strict
