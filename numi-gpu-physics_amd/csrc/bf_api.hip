@@ -304,7 +304,7 @@ struct bf_context {
     uint32_t raster_blocks = 1u << 30;
     uint32_t raster_batch = 0;            // triangles per raster wave; 0: from the mesh size
     int fast_priority = -1, general_priority = 0;  // s_setprio of the fluid kernels' wavefronts (-1: by the step)
-    int apart = -1;                                // a flight's wall-free tiles in a kernel of their own (-1: by the size)
+    int apart = -1;                                // wall-free tiles in a launch of their own (-1: by the step)
     bool pair_cells = true;                        // 2-byte storage: fast tiles two cells per lane
     uint32_t raster_batch_cap = 32;                // largest automatic raster batch
     uint32_t compute_units = 1;
@@ -775,8 +775,32 @@ uint32_t wall_blocks_for(const bf_context* c, uint32_t tiles) {
 
 // Sizes of grids for the rules below, in cells.
 constexpr uint32_t LARGE_GRID = 8000000u, VERY_LARGE_GRID = 16000000u;
-// STEP_APART or 0 for the wall-free tiles of a coupled flight, launched after
-// the wall tiles in any case: from the size at which they last longer than the chain of
+// Triangles from which a mesh's geometry is a long chain beside the step
+// (12 are none, 40,000 are; nothing between was measured).
+constexpr uint32_t MANY_TRIANGLES = 4096u;
+
+// STEP_APART or 0 for a step that could go in one launch.  FP32: one launch at
+// every size.  16-bit storage, one launch against two, us per step:
+//   * one cell per lane (rows that are not whole tile pairs): apart from the
+//     size at which streaming is the step (FP16 203x117x91 obstacle 72 / 84,
+//     320x160x160 plate 168 / 162, 320x200x160 obstacle 214 / 201, 576x288x288
+//     bird 948 / 756; BF16, with fewer spills, 320x200x160 185 / 193,
+//     448x224x224 plate 359 / 341, 320x320x240 FP16 wing 428 / 394);
+//   * a mesh of many triangles: its raster finds no room beside the one launch
+//     of four wavefronts per SIMD (40,000 triangles, FP16: 192x96x96 152 / 125,
+//     256x128x128 154 / 131), until two-cell streaming is the step (384x192x192
+//     266 / 282, 512x256x256 534 / 552).
+int step_apart(const bf_context* c) {
+    if (c->apart >= 0) return c->apart ? STEP_APART : 0;
+    if (c->cfg.storage == BF_STORAGE_FP32) return 0;
+    const bool pair = c->pair_cells && c->g.nx % (2 * TILE_X) == 0;
+    const bool many = c->source == BF_GEOMETRY_MESH && c->m_triangles >= MANY_TRIANGLES;
+    if (pair) return many && c->g.n < LARGE_GRID ? STEP_APART : 0;
+    return many || c->g.n >= (c->cfg.storage == BF_STORAGE_FP16_OFFSET ? LARGE_GRID : VERY_LARGE_GRID) ? STEP_APART : 0;
+}
+
+// The same for the wall-free tiles of a coupled flight, launched after the wall
+// tiles in any case: from the size at which they last longer than the chain of
 // reduction, body and geometry beside them (FP32 bird in flight, in fluid_step /
 // apart, ms per step: 224x140x112 0.197 / 0.206, 320x200x168 0.424 / 0.395,
 // 512x256x256 1.059 / 1.030; FP16: 256x160x136 0.130 / 0.131, 320x200x168
@@ -2067,6 +2091,7 @@ static bf_status step_static(bf_context* c, uint32_t steps) {
     hipError_t e = hipEventRecord(c->ev_ready[0], c->sb);
     if (e == hipSuccess) e = hipStreamWaitEvent(c->sa, c->ev_ready[0], 0);
     if (e != hipSuccess) return hip_fail(c, e, "event wait");
+    const int apart = step_apart(c);
     uint32_t waiting = 0;                // steps whose loads wait for their reduction
     auto reduce_loads = [&](int64_t last, const FluidBuffers& fb) {
         const hipError_t r = launch_load_reduction(load_buffers(c, fb), make_step_params(c),
@@ -2105,7 +2130,8 @@ static bf_status step_static(bf_context* c, uint32_t steps) {
         }
         if (pe && e == hipSuccess) e = hipEventRecord(pe[0], c->sa);
         if (e == hipSuccess)
-            e = launch_fluid_step(arith, storage, coll, fb, p, split ? STEP_FAST_TILES : STEP_ALL, wall_blocks, c->sa);
+            e = launch_fluid_step(arith, storage, coll, fb, p, (split ? STEP_FAST_TILES : STEP_ALL) | apart, wall_blocks,
+                                  c->sa);
         if (pe && e == hipSuccess) e = hipEventRecord(pe[1], c->sa);
         ++waiting;
         if (e == hipSuccess && (waiting == LOAD_SLOTS || i + 1 == steps || differs))
@@ -2190,11 +2216,12 @@ bf_status bf_step(bf_context* c, uint32_t steps) {
             if (pe && e == hipSuccess) e = hipEventRecord(pe[0], c->sa);
             StepParams pf = p;
             if (early_loads) pf.fast_priority = flight_priority(c);
-            const int apart = early_loads ? flight_apart(c) : 0;
+            const int apart = early_loads ? flight_apart(c) : step_apart(c);
             if (e == hipSuccess) e = launch_fluid_step(arith, storage, coll, fb, pf, STEP_FAST_TILES | apart, 0, c->sa);
         } else {
             if (pe && e == hipSuccess) e = hipEventRecord(pe[0], c->sa);
-            if (e == hipSuccess) e = launch_fluid_step(arith, storage, coll, fb, p, STEP_ALL, wall_blocks, c->sa);
+            if (e == hipSuccess)
+                e = launch_fluid_step(arith, storage, coll, fb, p, STEP_ALL | step_apart(c), wall_blocks, c->sa);
         }
         if (pe && e == hipSuccess) e = hipEventRecord(pe[1], c->sa);
         if (e == hipSuccess) e = hipEventRecord(c->ev_fast[par2(s)], c->sa);
@@ -2821,7 +2848,8 @@ bf_status bf_adjoint_gradient(bf_context* c, uint32_t steps, const double* load_
                 ps.links = a.nu;
             }
             if (e == hipSuccess)
-                e = launch_fluid_step(arith, storage, coll, fb, ps, STEP_ALL, wall_blocks_for(c, c->g.tiles), c->sb);
+                e = launch_fluid_step(arith, storage, coll, fb, ps, STEP_ALL | step_apart(c),
+                                      wall_blocks_for(c, c->g.tiles), c->sb);
         }
         if (e != hipSuccess) return hip_fail(c, e, "adjoint recompute");
         for (int64_t s = sb_; s > sa_; --s) {

@@ -1383,9 +1383,17 @@ void fluid_step(const typename Store<S>::T* __restrict__ fin, typename Store<S>:
 }
 
 // The wall-free tiles in a launch and kernel of their own (STEP_APART), at the
-// streaming code's natural occupancy (7 wavefronts per SIMD) and without the
-// wall path's LDS and its scalar registers: for the streaming beside a geometry
-// chain that needs room on the card (flight_apart in bf_api.hip).
+// streaming code's natural occupancy (7 wavefronts per SIMD; TRT with the
+// limiter 4) and without the wall path's LDS and its scalar registers.  Where
+// fluid_step loses to that:
+//   * 16-bit storage one cell per lane: half the bytes in flight per wavefront,
+//     and 200 spilled scalars (576x288x288 box FP16 RR3 842 -> 668 us per step,
+//     bird 948 -> 756; BF16 TRT 706 -> 624 and 804 -> 729);
+//   * the limiter of TRT (512x256x256 box FP32 940 -> 912 us);
+//   * beside a geometry chain that needs room on the card (step_apart and
+//     early_loads in bf_api.hip).
+// Elsewhere it is the slower form (512x256x256 bird FP16, two cells per lane:
+// 534 against 552 us; 203x117x91 obstacle FP16: 72 against 84).
 template <int ARITH, int COLL, int S, bool PAIR>
 __global__ __launch_bounds__(256)
 void fluid_stream(const typename Store<S>::T* __restrict__ fin, typename Store<S>::T* __restrict__ fout,
@@ -1401,15 +1409,25 @@ void fluid_stream(const typename Store<S>::T* __restrict__ fin, typename Store<S
 // Host-side launchers (called from bf_api.hip).
 // ---------------------------------------------------------------------------
 
+// Cells of a grid without wall tiles from which one-cell 16-bit streaming goes
+// apart (129x65x63 FP16 TRT 15.6 us in fluid_step, 16.7 apart; 192x96x96 BF16
+// TRT 32.4 and 29.2).
+constexpr uint32_t STREAM_FREE_CELLS = 1000000u;
+
 template <int ARITH, int COLL, int S, bool PAIR>
 static hipError_t launch_step_p(const FluidBuffers& b, const StepParams& p, int parts, uint32_t wall_blocks,
                                 hipStream_t s) {
     using T = typename Store<S>::T;
+    constexpr bool LIMITED = COLL == COLL_TRT_SYMMETRIC_LIMITER, ONE_CELL_16 = S != STORE_FP32 && !PAIR;
     if (!(parts & STEP_WALL_TILES)) wall_blocks = 0;
     uint32_t fast_blocks = parts & STEP_FAST_TILES ? (PAIR ? p.g.tiles / 2 : p.g.tiles) : 0u, stream_blocks = 0;
-    // coupled flights launch apart with TRT alone
-    constexpr bool STREAM = COLL == COLL_TRT;
-    if (STREAM && (parts & STEP_APART)) std::swap(fast_blocks, stream_blocks);
+    // FP32 RR3 and regularized streaming gains nothing apart (512x256x256 box
+    // RR3 907 us in fluid_step, 925 apart): they have no instance of it
+    constexpr bool STREAM = S != STORE_FP32 || COLL == COLL_TRT || LIMITED;
+    // a step without any wall tile is apart at no further launch
+    const bool free_step = parts == STEP_ALL && wall_blocks == 0 &&
+                           (LIMITED || (ONE_CELL_16 && p.g.n >= STREAM_FREE_CELLS));
+    if (STREAM && ((parts & STEP_APART) || free_step)) std::swap(fast_blocks, stream_blocks);
     if (wall_blocks + fast_blocks > 0)
         hipLaunchKernelGGL((fluid_step<ARITH, COLL, S, PAIR>), dim3(wall_blocks + fast_blocks), dim3(256), 0, s,
                            (const T*)b.fin, (T*)b.fout, b.solid_prev, b.solid_cur, b.wall, b.dyn_prev, b.dyn_cur,
