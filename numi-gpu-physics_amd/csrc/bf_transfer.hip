@@ -20,7 +20,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 #include "bf_launch.h"
@@ -85,7 +85,7 @@ static void run_workers(int n, F&& worker) {
         try {
             threads[t] = std::thread(worker, t);
             started = t;
-        } catch (const std::system_error&) {
+        } catch (const std::exception&) {     // no thread, or no memory for one
             break;
         }
     }
