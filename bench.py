@@ -11,10 +11,10 @@ mesh whose 3-harmonic Fourier wing kinematics the device evaluates every
 step (--mesh frames uploads one recorded frame per step instead).
 
 A step is one full pass of the path: vertex prepare, raster, resolve, fluid
-(fast + general tiles), load reduction.  value = cells x steps / wall time of
+(wall tiles + wall-free tiles), load reduction.  value = cells x steps / wall time of
 K steps bracketed by stream synchronizations, in MLUPS; the roofline entry is
-the fast fluid kernel (populations only: 152 B per cell update) timed with HIP
-events recorded on the library's stream inside the timed region.
+the step's fluid launch, fluid_step (populations only: 152 B per cell update),
+timed with HIP events recorded on the library's stream inside the timed region.
 """
 from __future__ import annotations
 
@@ -33,7 +33,7 @@ HBM_PEAK_GBS = 8000.0
 METRIC = "MLUPS + %HBM roofline, moving-bird 512×256×256 FP32 vs FP16-store; adjoint/fwd"
 STORAGES = {"fp32": 0, "fp16": 1, "bf16": 2}
 ARITHMETIC = {"default": 0, "strict": 1, "fused": 2}
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "fluid_fast_traffic.json")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "fluid_step_traffic.json")
 POP_BYTES = {"fp32": 152, "fp16": 76, "bf16": 76}
 BREAKDOWN_STEPS = 10
 
@@ -86,7 +86,7 @@ def run_gpu(shape, steps, warmup, storage, arithmetic="default", form="articulat
         sim.init_equilibrium()
         sim.advance(warmup)
         sim.synchronize()
-        # timed steps: HIP events around the fast kernel only (on its stream)
+        # timed steps: HIP events around the fluid launch only (on its stream)
         sim.set_profiling(True, level=1)
         t0 = time.perf_counter()
         sim.advance(steps, synchronize=False)
@@ -95,7 +95,7 @@ def run_gpu(shape, steps, warmup, storage, arithmetic="default", form="articulat
         prof = sim.read_profile()
         loads = sim.load_history(steps)
         census, cov, unc = sim.link_census()
-        # untimed: general kernel and geometry durations (more events per step)
+        # untimed: both kinds of tile in launches of their own, and the geometry (more events per step)
         sim.set_profiling(True, level=2)
         sim.advance(BREAKDOWN_STEPS)
         brk = sim.read_profile()
@@ -104,18 +104,18 @@ def run_gpu(shape, steps, warmup, storage, arithmetic="default", form="articulat
         sim.close()
     n = cfg.cells
     elapsed = t1 - t0
-    fast_tiles = prof["tiles"] - prof["general_tiles"]
-    fast_cells = fast_tiles * 256
-    fast_ms = prof["fast_ms"] / max(prof["steps"], 1)
-    achieved = POP_BYTES[storage] * fast_cells / (fast_ms * 1e-3) / 1e9
+    launch_ms = prof["fast_ms"] / max(prof["steps"], 1)
+    achieved = POP_BYTES[storage] * n / (launch_ms * 1e-3) / 1e9
+    k = max(brk["steps"], 1)
     step_bytes = (POP_BYTES[storage] + 2) * n
     return {
         "mlups": n * steps / elapsed / 1e6,
         "ms_per_step": elapsed * 1e3 / steps,
-        "fast_kernel_ms": fast_ms,
-        "general_ms": brk["general_ms"] / max(brk["steps"], 1),
-        "geometry_ms": brk["geometry_ms"] / max(brk["steps"], 1),
-        "fast_cells": fast_cells,
+        "fluid_step_ms": launch_ms,
+        "wall_free_ms": brk["fast_ms"] / k,
+        "wall_ms": brk["general_ms"] / k,
+        "geometry_ms": brk["geometry_ms"] / k,
+        "cells": n,
         "general_tiles": prof["general_tiles"],
         "achieved_gbs": achieved,
         "step_gbs": step_bytes * steps / elapsed / 1e9,
@@ -169,8 +169,8 @@ def run_sdf_bird(shape, steps, warmup):
     k = max(brk["steps"], 1)
     return {"value": n * steps / (t1 - t0) / 1e6, "unit": "MLUPS", "ms_per_step": (t1 - t0) * 1e3 / steps,
             "steps": steps, "solid_cells": solid, "general_tiles": int(brk["general_tiles"]), "tiles": int(brk["tiles"]),
-            "step_breakdown_ms": {"geometry": brk["geometry_ms"] / k, "fluid_fast": brk["fast_ms"] / k,
-                                  "fluid_general": brk["general_ms"] / k},
+            "step_breakdown_ms": {"geometry": brk["geometry_ms"] / k, "wall_free_tiles": brk["fast_ms"] / k,
+                                  "wall_tiles": brk["general_ms"] / k},
             "finite": bool(np.isfinite(loads).all() and np.isfinite(body).all() and np.isfinite(last).all()),
             "body_velocity_end": body[7:10].tolist(),
             "workload": f"analytic demonstration bird {shape[0]}x{shape[1]}x{shape[2]}, free flight, TRT, "
@@ -217,8 +217,8 @@ def run_wing(shape, steps, warmup):
     return {"value": n * steps / (t1 - t0) / 1e6, "unit": "MLUPS", "ms_per_step": (t1 - t0) * 1e3 / steps,
             "steps": steps, "solid_cells": int((mask != 0).sum()), "general_tiles": int(brk["general_tiles"]),
             "tiles": int(brk["tiles"]),
-            "step_breakdown_ms": {"geometry": brk["geometry_ms"] / k, "fluid_fast": brk["fast_ms"] / k,
-                                  "fluid_general": brk["general_ms"] / k},
+            "step_breakdown_ms": {"geometry": brk["geometry_ms"] / k, "wall_free_tiles": brk["fast_ms"] / k,
+                                  "wall_tiles": brk["general_ms"] / k},
             "finite": bool(np.isfinite(loads).all()),
             "workload": f"Li & Nabawy beta-planform wing {shape[0]}x{shape[1]}x{shape[2]}, chord 32 cells, "
                         "link-table walls, TRT, FP32"}
@@ -321,12 +321,11 @@ def run_adjoint(shape, steps, interval):
 
 
 def measured_traffic(storage, arithmetic, cells):
-    """HBM bytes of one fast-kernel launch over `cells` cells, from the
-    committed rocprofv3 PMC passes (FETCH_SIZE and WRITE_SIZE per dispatch,
-    calibrated on a copy kernel) for this storage and arithmetic: the
-    measured bytes per cell times the cells of this launch (the number of
-    wall-free tiles moves by a few per step as the bird flaps).  None when no
-    such measurement exists."""
+    """HBM bytes of one fluid launch over `cells` cells, from the committed
+    rocprofv3 PMC passes (FETCH_SIZE and WRITE_SIZE per dispatch, calibrated on
+    a copy kernel) for this storage and arithmetic on the bird: the measured
+    bytes per cell times the cells of this launch.  None when no such
+    measurement exists."""
     try:
         rec = json.load(open(TRAFFIC_FILE))[f"{storage}/{arithmetic}"]
         per_cell = rec["bytes_per_launch"] / rec["cells_per_launch"]
@@ -406,13 +405,13 @@ def main():
         r16 = run_gpu(shape, args.steps, args.warmup, "fp16", args.arithmetic, args.mesh)
         print(f"# gpu fp16: {r16}", file=sys.stderr, flush=True)
         extra["fp16_store"] = {"value": r16["mlups"], "unit": "MLUPS", "ratio_vs_fp32": r16["mlups"] / r["mlups"],
-                               "fast_kernel_ms": r16["fast_kernel_ms"], "achieved_gbs": r16["achieved_gbs"]}
+                               "fluid_step_ms": r16["fluid_step_ms"], "achieved_gbs": r16["achieved_gbs"]}
     if args.ray_steps > 0:
         rr = run_gpu(shape, args.ray_steps, args.warmup, args.storage, args.arithmetic, args.mesh,
                      wall_rule=bh.WALL_INTERPOLATED_RAY)
         print(f"# gpu, exact ray roots: {rr}", file=sys.stderr, flush=True)
         extra["exact_ray_roots"] = {"value": rr["mlups"], "unit": "MLUPS", "ms_per_step": rr["ms_per_step"],
-                                    "geometry_ms": rr["geometry_ms"], "fast_kernel_ms": rr["fast_kernel_ms"],
+                                    "geometry_ms": rr["geometry_ms"], "fluid_step_ms": rr["fluid_step_ms"],
                                     "steps": args.ray_steps,
                                     "workload": "the same bird with BF_WALL_INTERPOLATED_RAY link fractions"}
     if args.sdf_bird_steps > 0:
@@ -464,11 +463,12 @@ def main():
                    else "one uploaded frame per step"},
         "roofline": {"bound": "hbm", "achieved": r["achieved_gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": r["achieved_gbs"] / HBM_PEAK_GBS,
-                     "traffic": measured_traffic(args.storage, args.arithmetic, r["fast_cells"]),
-                     "kernel": "fluid_fast", "bytes_per_cell": POP_BYTES[args.storage],
-                     "cells_per_launch": r["fast_cells"], "avg_ms": r["fast_kernel_ms"]},
-        "step_breakdown_ms": {"geometry": r["geometry_ms"], "fluid_fast": r["fast_kernel_ms"],
-                              "fluid_general": r["general_ms"]},
+                     "traffic": measured_traffic(args.storage, args.arithmetic, r["cells"]),
+                     "kernel": "fluid_step", "bytes_per_cell": POP_BYTES[args.storage],
+                     "cells_per_launch": r["cells"], "avg_ms": r["fluid_step_ms"]},
+        # the step's fluid launch; its two kinds of tile launched apart, and the next step's geometry beside it
+        "step_breakdown_ms": {"fluid_step": r["fluid_step_ms"], "wall_free_tiles": r["wall_free_ms"],
+                              "wall_tiles": r["wall_ms"], "geometry": r["geometry_ms"]},
         "step_roofline_frac": r["step_gbs"] / HBM_PEAK_GBS,
         "cpu_baseline": cpu,
     }
