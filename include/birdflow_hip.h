@@ -413,9 +413,9 @@ bf_status bf_link_census(bf_context* ctx, uint64_t counts[21]);
  * pair and launch adds latency to the step); 0: off. */
 bf_status bf_set_profiling(bf_context* ctx, int enabled);
 /* {geometry ms, fluid ms (level 2: its wall-free tiles), wall-tile ms (0
- * unless level 2), steps profiled, tiles on the general path in the last step, total tiles (64 x 4
- * cells)} summed over the steps profiled since the last reset; resets the
- * counters. */
+ * unless level 2), steps profiled, tiles on the general path in the last
+ * step, total tiles (64 x 4 cells)} summed over the steps profiled since the
+ * last reset; resets the counters. */
 bf_status bf_read_profile(bf_context* ctx, double out[6]);
 
 /* Device copy bandwidth on the current device: a plain 16-byte-per-lane copy

@@ -7,7 +7,8 @@
 // masks, load reduction, swap.
 //
 // With moving geometry two HIP streams form a software pipeline, per step s:
-//   stream A  fluid_step(s): wall tiles and wall-free tiles in one launch
+//   stream A  fluid_step(s): wall tiles and wall-free tiles, in one launch
+//             or (step_apart, flight_apart) in two
 //   stream B  geometry(s+1) + tile list(s+1)  [overlaps fluid_step(s)],
 //             then the load reduction of step s    [overlaps fluid_step(s+1)]
 // fluid_step(s) waits for L[s] (its tile list, stream B); the reduction of
@@ -50,7 +51,7 @@ constexpr uint32_t PROFILE_CAPACITY = 4096;
 // and no system-scope fence (the host waits for streams, never for these;
 // 4 - 6 us less between the fluid launches of consecutive steps).
 constexpr unsigned STREAM_EVENT = hipEventDisableTiming | hipEventDisableSystemFence;
-constexpr int PROFILE_EVENTS = 6;   // A: fast start/end; B: geometry start/end, general start/end
+constexpr int PROFILE_EVENTS = 6;   // fluid launch (or wall-free tiles), geometry, wall tiles: start / end each
 
 struct DeviceAlloc {
     std::vector<void*> ptrs;
@@ -289,7 +290,7 @@ struct bf_context {
     std::string error;
     // profiling
     bool profiling = false;
-    int profiling_level = 0;              // 1: fast kernel only; 2: also general and geometry
+    int profiling_level = 0;              // 1: the fluid launch; 2: its kinds of tile apart, and the geometry
     std::vector<hipEvent_t> events;
     uint32_t profiled = 0;
     uint32_t wall_blocks = 512;           // workgroups of a step that walk the wall-tile list
@@ -3031,10 +3032,10 @@ bf_status bf_read_profile(bf_context* c, double out[6]) {
     for (uint32_t i = 0; i < c->profiled; ++i) {
         float a = 0, b = 0, d = 0;
         const hipEvent_t* ev = &c->events[(size_t)i * PROFILE_EVENTS];
-        (void)hipEventElapsedTime(&a, ev[0], ev[1]);   // fast kernel (stream A)
+        (void)hipEventElapsedTime(&a, ev[0], ev[1]);   // fluid launch, or its wall-free tiles (stream A)
         if (c->profiling_level >= 2) {
             (void)hipEventElapsedTime(&d, ev[2], ev[3]);   // next step's geometry + tile list (stream B)
-            (void)hipEventElapsedTime(&b, ev[4], ev[5]);   // general kernel (stream A, before fast)
+            (void)hipEventElapsedTime(&b, ev[4], ev[5]);   // wall tiles (stream A, before them)
         }
         fast += a;
         general += b;

@@ -80,9 +80,9 @@ struct StepParams {
     int load_component;
     int selected_part;
     int accumulate_loads;
-    int fast_priority;         // s_setprio level of the fast kernel's wavefronts (0..3)
+    int fast_priority;         // s_setprio level of the wall-free tiles' wavefronts (0..3)
     int pair_cells;            // 2-byte storage: fast tiles two cells per lane (fluid_fast_pair)
-    int general_priority;      // and of the general kernel's
+    int general_priority;      // and of the wall tiles'
     float omega_plus, omega_minus;
     float sponge_strength, sponge_width;
     float far_u[3], far_rho;

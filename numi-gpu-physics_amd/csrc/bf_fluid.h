@@ -592,9 +592,9 @@ __device__ __forceinline__ void fluid_fast(uint32_t block, uint32_t blocks,
     const int nx = p.g.nx, ny = p.g.ny, nz = p.g.nz;
     // Lanes of a partial tile beyond the grid load from the last column / row,
     // so no load leaves the lattice, and store nothing; in whole tiles the
-    // clamp changes nothing.  Partial tiles used to take the general path:
-    // a grid of odd sides then spent most of its step there (203x117x91 BF16,
-    // 3,407 of 10,920 tiles: 99 of 163 us per step).
+    // clamp changes nothing.  (On the general path the partial tiles of a grid
+    // of odd sides are most of its step: 203x117x91 BF16, 3,407 of 10,920
+    // tiles, 99 us.)
     //
     // A wavefront is one row of the tile: y, the nine source rows and
     // everything derived from them are wave-uniform, so the row addresses and
@@ -1354,12 +1354,14 @@ __device__ __forceinline__ void fluid_general(uint32_t block, uint32_t blocks,
 // launches their 208-register wavefronts found no room beside the others'.
 // In one launch they start first and the streaming fills the rest.  Held to 4
 // wavefronts per SIMD (128 registers): the wall path spills 7 - 72 of them
-// and still ends long before the streaming does; the streaming alone loses 1 %
-// to its natural 7 wavefronts at 512x256x256.  5 wavefronts gain that back on
-// the largest grids (969 against 982 us per step) and lose where the wall
-// tiles are the step (80x80x48 half-way plate: 34.6 against 27.2); 6 lose
-// everywhere.  256x128x128 plate 168 -> 139 us per step, 64^3 box 46 -> 10
-// (with the launches that static geometry no longer needs).
+// and still ends long before the streaming does.  FP32 streaming loses 1 % to
+// its natural 7 wavefronts at 512x256x256; 5 gain that back on the largest
+// grids (969 against 982 us per step) and lose where the wall tiles are the
+// step (80x80x48 half-way plate: 34.6 against 27.2); 6 lose everywhere.
+// 16-bit streaming two cells per lane loses 5 - 7 % (FP16 RR3 491 -> 524 us),
+// less than the launch saves from 8M cells on; one cell per lane it loses up
+// to a third: see fluid_stream.  256x128x128 plate 168 -> 139 us per step, 64^3
+// box 46 -> 10 (with the launches that static geometry does not need).
 // ---------------------------------------------------------------------------
 template <int ARITH, int COLL, int S, bool PAIR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))

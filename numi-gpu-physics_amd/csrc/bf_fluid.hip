@@ -1,8 +1,8 @@
 // Non-templated fluid kernels and their launchers: the general-tile work
 // list, the fixed-order load reduction, initialisation, field extraction and
 // storage conversion; plus the dispatch of the fluid step over arithmetic,
-// storage and collision (instantiations live in bf_fluid_fused.hip and
-// bf_fluid_strict.hip).
+// storage and collision (instantiations live in bf_fluid_strict.hip,
+// bf_fluid_fused.hip, bf_fluid_fp16.hip and bf_fluid_bf16.hip).
 #include "bf_fluid.h"
 
 namespace bf {
